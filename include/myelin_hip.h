@@ -421,6 +421,43 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
                         int64_t cols, int transpose, myelin_stream_t stream);
 
 /*
+ * Exact fp32 synapse currents of small-integer inputs (spikes) on the int8
+ * MFMA.  myelin_spike_limit(F) is the largest input magnitude the digit
+ * products of an F-wide layer hold in 32 bits (0: F too wide).
+ *
+ * myelin_cast_spikes: x [rows, F] fp32 -> xi [rows, Kp] int8, zeros past F
+ * (Kp a multiple of 128, 16-byte aligned), and, unless xb is NULL, xb [rows,
+ * F] bf16.  Sets flags[0] if some element is not bf16-exact (as
+ * myelin_cast_bf16_checked) and flags[1] if some element is no integer of
+ * magnitude <= myelin_spike_limit(F); never clears them.
+ *
+ * myelin_weight_digits: w [F, N] fp32 -> per column n a power of two
+ * scale[n] and w = scale[n] * (d3 2^24 + d2 2^16 + d1 2^8 + d0), balanced
+ * base-256 digits, exact for weights down to 2^-6 of the column's largest
+ * and within 2^-30 of that below; digits [ceil(N/32), 4 planes, 32, Kp]
+ * int8, zeros past F and N.  Sets flags[1] if a column is not finite or its
+ * largest magnitude is below 2^-96.
+ *
+ * myelin_gemm_spikes: C [M, N] = xi w (+ bias), every output the exact sum
+ * of the digit products rounded once to fp32 (twice past 2^10 column
+ * maxima), then scaled and biased: independent of order, tiles and rows.
+ * Meaningful only where the two calls above left flags[1] clear.
+ * Replaces: as myelin_gemm_f32 (the fp32 synapse GEMMs when the layer input
+ *   is spikes).
+ */
+int64_t myelin_spike_limit(int64_t F);
+int myelin_cast_spikes(const float *x, int8_t *xi, uint16_t *xb, int64_t rows,
+                       int64_t F, int64_t Kp, int *flags,
+                       myelin_stream_t stream);
+int myelin_weight_digits(const float *w, int8_t *digits, float *scale,
+                         int64_t F, int64_t N, int64_t Kp, int *flags,
+                         myelin_stream_t stream);
+int myelin_gemm_spikes(const int8_t *xi, const int8_t *digits,
+                       const float *scale, const float *bias, float *C,
+                       int64_t M, int64_t N, int64_t Kp, int64_t ldc,
+                       myelin_stream_t stream);
+
+/*
  * Reverse recurrence over C steps of a saved pre-reset trace [C, BN]:
  *   d = slope*sigma'(slope*(pre - thr)); gp = gm*((1-s) + (reset-pre)*d)
  *   + g_spike*d; G[j] = gp; gm = gp*decay   (grad_m is in/out)

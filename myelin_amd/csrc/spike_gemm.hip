@@ -1,0 +1,479 @@
+// Exact fp32 synapse currents of integer-valued inputs (spikes) on the int8
+// MFMA.
+//
+// An fp32 weight column is written as a 31-bit fixed-point number against
+// its own largest magnitude: w = scale * q, |q| <= 2^30, scale a power of
+// two, and q as four balanced base-256 digits q = d3 2^24 + d2 2^16 + d1 2^8
+// + d0.  Weights down to 2^-6 of their column's largest keep every bit of
+// their fp32 value, and smaller ones are off by at most 2^-30 of it.  With
+// inputs that are small integers, each digit plane's product is an integer
+// sum without rounding; the planes are joined and rounded once per output.
+// So an output does not depend on the order, the tiles or the rows it is
+// computed with, and lies within about half an ulp of the exact sum
+// (measured on 8192 x 4096 currents of 1024 inputs at 5 % activity: 3.0e-8
+// of the largest from float64; the three-plane bf16 split 6.8e-8, an fp32
+// GEMM 5e-7).
+//
+// Cost: four int8 planes at twice the bf16 rate against three bf16 planes:
+// 2/3 of the matrix time, half the input bytes.
+
+#include "common.h"
+
+namespace {
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+constexpr int kPlanes = 4;   // base-256 digits per weight
+constexpr int kStage = 128;  // k per LDS stage (bytes of a row)
+
+inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// ---------------------------------------------------------------------------
+// Operands.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
+
+// v survives its bf16 rounding and is zero or normal
+__device__ __forceinline__ bool bf16_exact(float v) {
+  const float a = __builtin_fabsf(v);
+  return static_cast<float>(static_cast<__bf16>(v)) == v && (a == 0.0f || a >= 1.17549435e-38f);
+}
+
+struct CastArgs {
+  const float *x;
+  int8_t *xi;
+  uint16_t *xb;
+  int *flags;
+  int64_t rows;
+  int F, Kp, lim;
+};
+
+// x [rows, F] fp32 -> xi [rows, Kp] int8 (zeros past F) and, if xb is given,
+// xb [rows, F] bf16.  flags[0] is set where a value is not bf16-exact,
+// flags[1] where one is no integer of magnitude <= lim; neither is cleared.
+// Bound by memory: each lane takes groups of four elements of a row, lane
+// after lane, so every load and store instruction of a wave is contiguous.
+template <bool VEC>
+__global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
+  constexpr int U = 4;  // groups per lane
+  const uint32_t per = static_cast<uint32_t>(p.Kp) / 4;
+  const int64_t total = p.rows * per;
+  const int64_t g0 = static_cast<int64_t>(blockIdx.x) * (256 * U) + threadIdx.x;
+  float v[U][4];
+  int64_t row[U];
+  int col[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t g = g0 + u * 256;
+    row[u] = g / per;
+    col[u] = static_cast<int>(g - row[u] * per) * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[u][e] = 0.0f;
+    if (g < total && col[u] < p.F) {
+      const float *src = p.x + row[u] * p.F + col[u];
+      if constexpr (VEC) {  // F % 4 == 0 and 16-byte aligned rows
+        const f4 t = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(src));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = t[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col[u] + e < p.F) v[u][e] = src[e];
+      }
+    }
+  }
+  bool inexact = false, wide = false;
+  const float lim = static_cast<float>(p.lim);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (g0 + u * 256 >= total) continue;
+    uint32_t q = 0;
+    uint16_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float f = v[u][e], r = __builtin_rintf(f);
+      inexact = inexact || !bf16_exact(f);
+      const bool ok = r == f && __builtin_fabsf(f) <= lim;  // false for NaN
+      wide = wide || !ok;
+      q |= static_cast<uint32_t>(static_cast<uint8_t>(ok ? static_cast<int>(r) : 0)) << (8 * e);
+      h[e] = to_bf16(f);
+    }
+    *reinterpret_cast<uint32_t *>(p.xi + row[u] * p.Kp + col[u]) = q;
+    if (p.xb != nullptr && col[u] < p.F) {
+      uint16_t *dst = p.xb + row[u] * p.F + col[u];
+      if constexpr (VEC) {
+        typedef uint16_t h4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<h4 *>(dst) = h4{h[0], h[1], h[2], h[3]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col[u] + e < p.F) dst[e] = h[e];
+      }
+    }
+  }
+  const bool any0 = __ballot(inexact) != 0, any1 = __ballot(wide) != 0;
+  if ((threadIdx.x & 63) == 0) {
+    if (any0) p.flags[0] = 1;
+    if (any1) p.flags[1] = 1;
+  }
+}
+
+// w [F, N] -> digits [ceil(N / 32)][4 planes][32 neurons][Kp] int8 (zeros
+// past F and N) and scale [N].  flags[1] is set where a column holds a
+// non-finite value or its largest magnitude is outside [2^-96, 2^128).
+// A workgroup writes `chunk` k of 32 neurons: it first finds the columns'
+// maxima over all F (re-read from L2 by each of a column's workgroups: one
+// launch instead of a reduction and a second pass), then turns tiles of 128
+// k around through LDS so that rows are written 16 bytes at a time.
+__global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ w, int8_t *__restrict__ q,
+                                                      float *__restrict__ scale, int *__restrict__ flags, int F, int N,
+                                                      int Kp, int chunk) {
+  __shared__ uint32_t red[32][33];
+  __shared__ int tile[32][kStage + 1];
+  const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const int64_t n = static_cast<int64_t>(blockIdx.x) * 32 + c;
+  const bool in = n < N;
+  uint32_t mx = 0;
+  if (in) {
+    // four rows in flight
+    int f = r;
+    for (; f + 96 < F; f += 128) {
+      uint32_t b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[u] = __builtin_bit_cast(uint32_t, w[static_cast<int64_t>(f + 32 * u) * N + n]) & 0x7fffffffu;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) mx = mx > b[u] ? mx : b[u];
+    }
+    for (; f < F; f += 32) {
+      const uint32_t b = __builtin_bit_cast(uint32_t, w[static_cast<int64_t>(f) * N + n]) & 0x7fffffffu;
+      mx = mx > b ? mx : b;
+    }
+  }
+  red[r][c] = mx;
+  __syncthreads();
+  mx = 0;
+#pragma unroll 8
+  for (int i = 0; i < 32; ++i) mx = mx > red[i][c] ? mx : red[i][c];
+  // every value is below 2^e; a zero column has digits 0 and scale 0
+  const int e = static_cast<int>(mx >> 23) - 126;
+  const bool bad = mx >= 0x7f800000u || (mx != 0 && e < -96);
+  const float up = (mx == 0 || bad) ? 0.0f : __builtin_bit_cast(float, static_cast<uint32_t>(30 - e + 127) << 23);
+  if (blockIdx.y == 0 && r == 0 && in) {
+    scale[n] = (mx == 0 || bad) ? 0.0f : __builtin_bit_cast(float, static_cast<uint32_t>(e - 30 + 127) << 23);
+    if (bad) flags[1] = 1;
+  }
+  const int k_begin = blockIdx.y * chunk, k_end = k_begin + chunk < Kp ? k_begin + chunk : Kp;
+  for (int k0 = k_begin; k0 < k_end; k0 += kStage) {
+#pragma unroll
+    for (int u = 0; u < kStage / 32; ++u) {
+      const int f = k0 + r + 32 * u;
+      // exact: |w| up is at most 2^30 and a power of two times w
+      tile[c][r + 32 * u] = (in && f < F) ? static_cast<int>(__builtin_rintf(w[static_cast<int64_t>(f) * N + n] * up)) : 0;
+    }
+    __syncthreads();
+    // thread -> plane, neuron, 16 k
+    const int pl = threadIdx.x >> 8, nn = (threadIdx.x >> 3) & 31, kc = (threadIdx.x & 7) * 16;
+    uint32_t out[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t word = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        int v = tile[nn][kc + 4 * i + b], d = 0;
+        for (int s = 0; s <= pl; ++s) {  // balanced digit pl
+          d = static_cast<int8_t>(v & 0xff);
+          v = (v - d) >> 8;
+        }
+        word |= static_cast<uint32_t>(static_cast<uint8_t>(d)) << (8 * b);
+      }
+      out[i] = word;
+    }
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<u4 *>(q + ((static_cast<int64_t>(blockIdx.x) * kPlanes + pl) * 32 + nn) * Kp + k0 + kc) =
+        u4{out[0], out[1], out[2], out[3]};
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// C[M, N] = (x digits) joined, scaled (+ bias).
+//
+// The four digit planes of 32 neurons are 128 "virtual" columns that one
+// wave owns: its tile is 32 WM rows x 128 virtual columns, WM x 4 blocks of
+// 32 x 32 (v_mfma_i32_32x32x32_i8: a lane's fragment is 16 bytes of k, as in
+// the bf16 kernels), so an input fragment read from LDS feeds four MFMAs and
+// the planes of an output element end in the same lane and register index:
+// they are joined without a second accumulator set.  WGM x WGN waves share a
+// stage of 128 k of their rows and virtual columns, staged by direct global
+// -> LDS loads of 16 bytes (rows unpadded, 16-byte pieces swizzled as
+// position c ^ swz(row), two stages).
+//
+// Persistent: each workgroup walks tiles (one workgroup per CU on the large
+// tile), and the first stage of its next tile is loaded during the last
+// stage and the epilogue of this one; K is short here (1024 inputs are eight
+// stages), so a tile started cold would spend a third of its life filling
+// the pipe.
+// ---------------------------------------------------------------------------
+struct SpikeArgs {
+  const int8_t *x;  // [M, Kp]
+  const int8_t *q;  // digits
+  const float *scale, *bias;
+  float *C;
+  int64_t M, N, ldc;
+  int Kp;
+};
+
+// position of 16-byte piece c of row r of a stage: c ^ swz(r).  A function of
+// r & 31, so the 32-row blocks of a wave share it, distinct over any 8
+// aligned rows and, with the row's bank half, over any 16: fragment reads
+// (32 rows of one piece per half-wave) meet no bank conflict
+__device__ __forceinline__ int swz(int r) { return (r ^ ((r >> 3) & 3)) & 7; }
+
+__device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+template <int WM, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(2))) void spike_gemm(SpikeArgs g) {
+  constexpr int NT = 64 * WGM * WGN;
+  constexpr int BM = 32 * WM * WGM, BV = 128 * WGN;
+  constexpr int TILE = (BM + BV) * kStage;
+  constexpr int NPA = BM * 8 / NT, NPB = BV * 8 / NT;
+  __shared__ __attribute__((aligned(1024))) char lds[2 * TILE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w / WGN, wn = w % WGN;
+  const uint32_t tiles_m = static_cast<uint32_t>((g.M + BM - 1) / BM);
+  const uint32_t tiles_n = static_cast<uint32_t>((g.N + 32 * WGN - 1) / (32 * WGN));
+  const uint32_t tiles = tiles_m * tiles_n;
+  // Workgroup ids go round-robin to the 8 XCDs (each with its own L2): XCD d
+  // walks a contiguous run of logical tiles, its workgroups side by side.
+  const uint32_t xcds = gridDim.x % 8 == 0 ? 8 : 1;
+  const uint32_t xcd = blockIdx.x % xcds, slot = blockIdx.x / xcds, slots = gridDim.x / xcds;
+  const uint32_t first = static_cast<uint32_t>(static_cast<uint64_t>(tiles) * xcd / xcds);
+  const uint32_t last = static_cast<uint32_t>(static_cast<uint64_t>(tiles) * (xcd + 1) / xcds);
+  const int64_t vrows = (g.N + 31) / 32 * 128;  // virtual columns stored
+  const int nst = g.Kp / kStage;
+
+  // logical tile -> (row tile, column tile): groups of 8 row tiles walked
+  // column by column, so a run shares input rows and digit rows
+  auto place = [&](uint32_t t, int64_t &m0, int64_t &n0) {
+    const uint32_t per_group = 8 * tiles_n, group = t / per_group, fst = group * 8;
+    const uint32_t gs = tiles_m - fst < 8 ? tiles_m - fst : 8, in = t - group * per_group;
+    m0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(fst + in % gs)) * BM;
+    n0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(in / gs)) * (32 * WGN);
+  };
+
+  // load side: pieces of the tile being loaded, as 32-bit offsets from a
+  // uniform base; rows past the edge read the last row
+  uint32_t oa[NPA], ob[NPB];
+  const int8_t *ba = nullptr, *bb = nullptr;
+  uint32_t lt = first + slot;
+  int ls = 0, lbuf = 0;
+  auto point = [&]() {
+    int64_t m0, n0;
+    place(lt, m0, n0);
+    ba = g.x + m0 * g.Kp;
+    bb = g.q + n0 * kPlanes * g.Kp;
+    const int64_t lim_a = g.M - m0, lim_b = vrows - n0 * kPlanes;
+#pragma unroll
+    for (int e = 0; e < NPA; ++e) {
+      const int idx = e * NT + tid, row = idx >> 3;
+      const uint32_t rc = static_cast<uint32_t>(row < lim_a ? row : lim_a - 1);
+      oa[e] = rc * static_cast<uint32_t>(g.Kp) + 16 * ((idx & 7) ^ swz(row));
+    }
+#pragma unroll
+    for (int e = 0; e < NPB; ++e) {
+      const int idx = e * NT + tid, row = idx >> 3;
+      const uint32_t rc = static_cast<uint32_t>(row < lim_b ? row : lim_b - 1);
+      ob[e] = rc * static_cast<uint32_t>(g.Kp) + 16 * ((idx & 7) ^ swz(row));
+    }
+  };
+  auto issue = [&]() {
+    if (lt >= last) return;  // uniform
+    if (ls == 0) point();
+    char *tile = lds + lbuf * TILE;
+    const int8_t *pa = ba + ls * kStage, *pb = bb + ls * kStage;
+#pragma unroll
+    for (int e = 0; e < NPA + NPB; ++e) {
+      const int eo = e < NPA ? e : e - NPA;
+      const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+          (lds_void *)(tile + (e < NPA ? 0 : BM * kStage) + (eo * NT + w * 64) * 16)));
+      const uint32_t o = e < NPA ? oa[e] : ob[eo];
+      const int8_t *base = e < NPA ? pa : pb;
+      uint32_t m0_saved;  // M0 (the LDS base of the load) is the compiler's
+      asm volatile(
+          "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+          : "=&s"(m0_saved)
+          : "v"(o), "s"(base), "s"(dst)
+          : "memory");
+    }
+    lbuf ^= 1;
+    if (++ls == nst) {
+      ls = 0;
+      lt += slots;
+    }
+  };
+
+  // fragment byte offsets in a stage; the 32-row blocks of a wave lie 32
+  // rows apart
+  int fa[4], fb[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    const int c = 2 * ks + (lane >> 5), r = lane & 31;
+    fa[ks] = (32 * WM * wm + r) * kStage + ((c ^ swz(r)) << 4);
+    fb[ks] = (BM + 128 * wn + r) * kStage + ((c ^ swz(r)) << 4);
+  }
+
+  issue();
+  int buf = 0;
+  for (uint32_t t = first + slot; t < last; t += slots) {
+    i32x16 acc[WM][kPlanes];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < kPlanes; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    for (int s = 0; s < nst; ++s) {
+      // this stage's loads (and, of the first stage of a later tile, none:
+      // the epilogue before it has waited); the barrier makes every wave's
+      // pieces visible, and retires its LDS reads of the other buffer, which
+      // the loads issued after it overwrite
+      if (s > 0 || t == first + slot) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const char *cur = lds + buf * TILE;
+      i32x4 a[2][WM], b[2][kPlanes];
+      auto rd = [&](int ks, int set) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i) a[set][i] = *reinterpret_cast<const i32x4 *>(cur + fa[ks] + 32 * kStage * i);
+#pragma unroll
+        for (int j = 0; j < kPlanes; ++j) b[set][j] = *reinterpret_cast<const i32x4 *>(cur + fb[ks] + 32 * kStage * j);
+      };
+      rd(0, 0);
+      issue();
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if (ks + 1 < 4) rd(ks + 1, (ks + 1) & 1);
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int j = 0; j < kPlanes; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[ks & 1][i], b[ks & 1][j], acc[i][j], 0, 0, 0);
+        if (ks + 1 < 4) {
+          // the next k step's fragment reads one after each MFMA: left to
+          // itself the scheduler issues them after the last
+          constexpr int NR = WM + kPlanes, NM = WM * kPlanes;
+#pragma unroll
+          for (int z = 0; z < (NR < NM ? NR : NM); ++z) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, NR > NM ? 2 : 1, 0);
+          }
+          if constexpr (NM > NR) __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
+        }
+      }
+      buf ^= 1;
+    }
+    // the next tile's first stage has landed before this tile's stores are
+    // issued, so its first stage needs no wait behind them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int64_t m0, n0;
+    place(t, m0, n0);
+    const int64_t n = n0 + 32 * wn + (lane & 31);
+    if (n < g.N) {
+      const float sc = g.scale[n], bi = g.bias != nullptr ? g.bias[n] : 0.0f;
+      const int64_t mw = m0 + 32 * WM * wm;
+      const bool whole = mw + 32 * WM <= g.M;  // uniform
+      // the lane's column and row half, from each row's scalar base
+      const uint32_t off = static_cast<uint32_t>((4 * (lane >> 5) * g.ldc + 32 * wn + (lane & 31)) * 4);
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          // hi 2^16 + lo, both exact in 32 bits (the host bounds K |x|);
+          // hi is exact in fp32 while the sum is under 2^10 column maxima
+          const int lo = (acc[i][1][r] << 8) + acc[i][0][r];
+          const int hi = (acc[i][3][r] << 8) + acc[i][2][r];
+          float v = __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo)) * sc;
+          if (g.bias != nullptr) v = v + bi;
+          const float *base = g.C + (mw + 32 * i + acc_row(r, 0)) * g.ldc + n0;
+          if (whole || mw + 32 * i + acc_row(r, lane) < g.M)
+            asm volatile("global_store_dword %0, %1, %2" ::"v"(off), "v"(v), "s"(base) : "memory");
+        }
+    }
+  }
+}
+
+template <int WM, int WGM, int WGN>
+int launch_spike(const SpikeArgs &g, int per_cu, hipStream_t s) {
+  const int64_t tiles = cdiv(g.M, 32 * WM * WGM) * cdiv(g.N, 32 * WGN);
+  const int64_t wgs = tiles < 256 * per_cu ? tiles : 256 * per_cu;
+  spike_gemm<WM, WGM, WGN><<<dim3(static_cast<unsigned>(wgs)), dim3(64 * WGM * WGN), 0, s>>>(g);
+  return myelin::launched("gemm_spikes");
+}
+
+}  // namespace
+
+// the largest input magnitude whose joined digit sums stay in 32 bits:
+// K |x| 128 257 < 2^31
+extern "C" int64_t myelin_spike_limit(int64_t F) {
+  const int64_t kp = cdiv(F < 1 ? 1 : F, kStage) * kStage, lim = 65000 / kp;
+  return lim > 127 ? 127 : lim;
+}
+
+extern "C" int myelin_cast_spikes(const float *x, int8_t *xi, uint16_t *xb, int64_t rows, int64_t F, int64_t Kp,
+                                  int *flags, myelin_stream_t stream) {
+  if (rows < 0 || F < 1) return myelin::invalid("cast_spikes: rows must be >= 0 and F >= 1");
+  if (Kp % kStage != 0 || Kp < F || Kp > 65000) return myelin::invalid("cast_spikes: bad row pitch");
+  if (rows == 0) return MYELIN_OK;
+  if (x == nullptr || xi == nullptr || flags == nullptr) return myelin::invalid("cast_spikes: null pointer");
+  if (!myelin::aligned(xi, 16)) return myelin::invalid("cast_spikes: xi must be 16-byte aligned");
+  const int64_t blocks = cdiv(rows * (Kp / 4), 1024);
+  if (blocks > 0x7fffffff) return myelin::invalid("cast_spikes: too many elements");
+  const CastArgs a{x, xi, xb, flags, rows, static_cast<int>(F), static_cast<int>(Kp), static_cast<int>(myelin_spike_limit(F))};
+  const dim3 grid(static_cast<unsigned>(blocks));
+  if (F % 4 == 0 && myelin::aligned(x, 16) && (xb == nullptr || myelin::aligned(xb, 8)))
+    cast_spikes<true><<<grid, dim3(256), 0, myelin::as_hip(stream)>>>(a);
+  else
+    cast_spikes<false><<<grid, dim3(256), 0, myelin::as_hip(stream)>>>(a);
+  return myelin::launched("cast_spikes");
+}
+
+extern "C" int myelin_weight_digits(const float *w, int8_t *digits, float *scale, int64_t F, int64_t N, int64_t Kp,
+                                    int *flags, myelin_stream_t stream) {
+  if (F < 1 || N < 1) return myelin::invalid("weight_digits: F and N must be positive");
+  if (Kp % kStage != 0 || Kp < F || Kp > 65000) return myelin::invalid("weight_digits: bad row pitch");
+  if (w == nullptr || digits == nullptr || scale == nullptr || flags == nullptr)
+    return myelin::invalid("weight_digits: null pointer");
+  if (!myelin::aligned(digits, 16)) return myelin::invalid("weight_digits: digits must be 16-byte aligned");
+  const int64_t groups = cdiv(N, 32), stages = Kp / kStage;
+  if (N > 0x7fffffff || groups > 0x7fffffff) return myelin::invalid("weight_digits: N too large");
+  // about 512 workgroups: each of a column's re-reads it once
+  int64_t parts = cdiv(512, groups);
+  if (parts > stages) parts = stages;
+  const int64_t chunk = cdiv(stages, parts) * kStage;
+  weight_digits<<<dim3(static_cast<unsigned>(groups), static_cast<unsigned>(cdiv(Kp, chunk))), dim3(1024), 0,
+                  myelin::as_hip(stream)>>>(w, digits, scale, flags, static_cast<int>(F), static_cast<int>(N),
+                                            static_cast<int>(Kp), static_cast<int>(chunk));
+  return myelin::launched("weight_digits");
+}
+
+extern "C" int myelin_gemm_spikes(const int8_t *xi, const int8_t *digits, const float *scale, const float *bias,
+                                  float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc, myelin_stream_t stream) {
+  if (M < 0 || N < 0) return myelin::invalid("gemm_spikes: negative size");
+  if (Kp < kStage || Kp % kStage != 0 || Kp > 65000) return myelin::invalid("gemm_spikes: bad row pitch");
+  if (ldc < N) return myelin::invalid("gemm_spikes: ldc < N");
+  if (M == 0 || N == 0) return MYELIN_OK;
+  if (xi == nullptr || digits == nullptr || scale == nullptr || C == nullptr)
+    return myelin::invalid("gemm_spikes: null pointer");
+  if (!myelin::aligned(xi, 16) || !myelin::aligned(digits, 16))
+    return myelin::invalid("gemm_spikes: operands must be 16-byte aligned");
+  if (ldc >= (int64_t{1} << 27)) return myelin::invalid("gemm_spikes: rows too long");
+  if (cdiv(M, 128) * cdiv(N, 32) > 0x7fffffff) return myelin::invalid("gemm_spikes: output too large");
+  const SpikeArgs g{xi, digits, scale, bias, C, M, N, ldc, static_cast<int>(Kp)};
+  hipStream_t s = myelin::as_hip(stream);
+  // 256 rows x 64 neurons (eight waves, 128 KB of LDS, one workgroup per CU)
+  // where that fills the chip, else 128 x 32 (four waves, two per CU)
+  if (cdiv(M, 256) * cdiv(N, 64) >= 256) return launch_spike<2, 4, 2>(g, 1, s);
+  return launch_spike<1, 4, 1>(g, 2, s);
+}

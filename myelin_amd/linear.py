@@ -120,8 +120,8 @@ def _gemm_parts(A, B, parts, b_part, C, M, N, K, lda, ldb, ldc, trans_a, trans_b
                   dst.numel(), stream)
 
 
-# exact bf16 split of an fp32 synapse: tried for products of at least this
-# many multiply-adds (the input check costs one host synchronisation)
+# exact split of an fp32 synapse: tried for products of at least this many
+# multiply-adds (the input check costs one host synchronisation)
 _SPLIT_MIN_MACS = 1 << 32
 
 
@@ -150,67 +150,156 @@ class _LazyBf16:
         return self._last[1]
 
 
+def _cast_spikes(x, pitch, flags, stream, bf16=True):
+    """(int8 copy of x ``[..., F]`` in rows of ``pitch`` bytes, its bf16 copy
+    or None); flags as myelin_cast_spikes."""
+
+    F = x.shape[-1]
+    xi = torch.empty((*x.shape[:-1], pitch), dtype=torch.int8, device=x.device)
+    xb = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if bf16 else None
+    _lib.call("myelin_cast_spikes", _lib.ptr(x), _lib.ptr(xi), _lib.ptr(xb), x.numel() // F, F, pitch,
+              _lib.ptr(flags), stream)
+    return xi, xb
+
+
+class _Digits:
+    """An fp32 weight ``[F, N]`` as the four int8 digit planes and the column
+    scales myelin_gemm_spikes reads (the ``wt`` of an int8 input)."""
+
+    def __init__(self, q: torch.Tensor, scale: torch.Tensor):
+        self.q = q
+        self.scale = scale
+
+
 class _Split:
-    """The fp32 synapse on the bf16 MFMA, exactly: when every input value is
-    a bf16 value (spikes, small integers), ``x @ W = x @ W_hi + x @ W_mid +
-    x @ W_lo`` with the three bf16 planes of W summing exactly to W, so every
-    product is exact and only the fp32 summation rounds -- at the bf16
-    engine's rate (about 5x the fp32 one per pass).
+    """The fp32 synapse on the int8 or the bf16 MFMA, exactly.
 
-    Construction launches the checked bf16 copy of x (``xb``; with ``lean``
-    only the check, ``xb`` then a _LazyBf16 view), the split of W into
-    transposed planes ``w3 [3, N, F]`` and an asynchronous copy of the
-    check's flag to pinned host memory, without waiting.  ``exact()``
-    waits for the flag alone (not for later work on the stream) and caches
-    the answer; when it is False the fp32 GEMMs must run instead."""
+    An input of small integers (spikes) times W runs as four int8 products
+    with the base-256 digits of W, summed without rounding and rounded once
+    (``myelin_gemm_spikes``).  An input whose every value is a bf16 value
+    runs as three bf16 products, ``x @ W = x @ W_hi + x @ W_mid + x @ W_lo``
+    with the three bf16 planes of W summing exactly to W, so every product
+    is exact and only the fp32 summation rounds.  Per multiply-add the first
+    costs 2/3 of the second, and that a fifth of the fp32 engine.
 
-    def __init__(self, x, w, stream, lean=False):
-        flag = torch.zeros(1, dtype=torch.int32, device=x.device)
+    Construction launches the checked copies of x (``xi`` int8 and ``xb``
+    bf16; without ``bf16`` only ``xi``), both forms of W and an asynchronous
+    copy of the check's flags to pinned host memory; ``exact()`` and
+    ``operands()`` wait for those flags, the bf16 planes of W being formed
+    meanwhile.
+
+    ``ints=False`` takes the bf16 products alone, and ``lean`` (the memory
+    policy) implies it: no whole copy of x is kept then (``xb`` is a
+    _LazyBf16), and a second copy and the digits of W beside the bf16 slices
+    that its weight gradient reads anyway would be its largest buffers."""
+
+    def __init__(self, x, w, stream, lean=False, bf16=True, ints=True):
+        F, N = w.shape
+        dev = x.device
+        flags = torch.zeros(2, dtype=torch.int32, device=dev)
+        self.x = x
+        self.xi = self.xb = self.digits = None
         if lean:
             # no whole bf16 copy: check x slice by slice into one scratch
             # buffer (the flag is only ever set), and cast per chunk later
             self.xb = _LazyBf16(x)
             step = max(1, (1 << 22) // max(1, x[0].numel()))
-            scratch = torch.empty((min(step, x.shape[0]), *x.shape[1:]), dtype=torch.bfloat16, device=x.device)
+            scratch = torch.empty((min(step, x.shape[0]), *x.shape[1:]), dtype=torch.bfloat16, device=dev)
             for t0 in range(0, x.shape[0], step):
                 part = x[t0:t0 + step]
-                _lib.call("myelin_cast_bf16_checked", _lib.ptr(part), _lib.ptr(scratch), part.numel(), _lib.ptr(flag),
+                _lib.call("myelin_cast_bf16_checked", _lib.ptr(part), _lib.ptr(scratch), part.numel(), _lib.ptr(flags),
                           stream)
+        elif ints and _lib.load().myelin_spike_limit(F) > 0:
+            pitch = -(-F // 128) * 128
+            self.xi, self.xb = _cast_spikes(x, pitch, flags, stream, bf16=bf16)
+            # a weight the digits cannot hold raises the int8 flag as well
+            q = torch.empty((-(-N // 32), 4, 32, pitch), dtype=torch.int8, device=dev)
+            self.digits = _Digits(q, torch.empty(N, dtype=torch.float32, device=dev))
+            _lib.call("myelin_weight_digits", _lib.ptr(w), _lib.ptr(q), _lib.ptr(self.digits.scale), F, N, pitch,
+                      _lib.ptr(flags), stream)
         else:
-            self.xb = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
-            _lib.call("myelin_cast_bf16_checked", _lib.ptr(x), _lib.ptr(self.xb), x.numel(), _lib.ptr(flag), stream)
-        self._host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-        self._host.copy_(flag, non_blocking=True)
+            self.xb = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
+            _lib.call("myelin_cast_bf16_checked", _lib.ptr(x), _lib.ptr(self.xb), x.numel(), _lib.ptr(flags), stream)
+        self._host = torch.empty(2, dtype=torch.int32, pin_memory=True)
+        self._host.copy_(flags, non_blocking=True)
         self._ready = torch.cuda.Event()
-        self._ready.record(torch.cuda.current_stream(x.device))
-        F, N = w.shape
-        self.w3 = torch.empty((3, N, F), dtype=torch.bfloat16, device=w.device)
+        self._ready.record(torch.cuda.current_stream(dev))
+        self.w3 = torch.empty((3, N, F), dtype=torch.bfloat16, device=dev)
         _lib.call("myelin_split_bf16x3", _lib.ptr(w), _lib.ptr(self.w3), F, N, 1, stream)
-        self._exact = None
+        self._flags = None
+
+    def _answer(self):
+        if self._flags is None:
+            self._ready.synchronize()
+            self._flags = tuple(self._host.tolist())
+        return self._flags
 
     def exact(self) -> bool:
-        if self._exact is None:
-            self._ready.synchronize()
-            self._exact = int(self._host[0]) == 0
-        return self._exact
+        """Every value of x is a bf16 value."""
+
+        return self._answer()[0] == 0
+
+    def operands(self):
+        """(xs, wt, xg): the currents' operands on the engine that takes this
+        input -- int8 and digits, bf16 and planes, or the fp32 input and None
+        -- and what the weight gradient's GEMM reads (the bf16 copy if the
+        input is exact in it, else x; None on digits without ``bf16``)."""
+
+        inexact, wide = self._answer()
+        if inexact:
+            return self.x, None, self.x
+        if self.digits is not None and not wide:
+            return self.xi, self.digits, self.xb
+        if self.xb is None:
+            flags = torch.empty(2, dtype=torch.int32, device=self.x.device)  # known to hold: not read
+            self.xb = _cast_spikes(self.x, self.xi.shape[-1], flags, _lib.stream(self.x.device))[1]
+        return self.xb, self.w3, self.xb
 
 
-def _split_synapse(x, w, stream, lean=False):
+def _exact_split(wt) -> bool:
+    """``wt`` belongs to an exact split of the fp32 synapse (see _lif_fwd)."""
+
+    return isinstance(wt, _Digits) or (wt is not None and wt.ndim == 3)
+
+
+def _pack_operands(x, xs, wt, xg):
+    """(tensors to save, how to read them back) of a layer's operands (xs,
+    wt, xg); a _LazyBf16 is saved as its fp32 input."""
+
+    lazy = isinstance(xs, _LazyBf16)
+    digits = isinstance(wt, _Digits)
+    tensors = [x, x] if lazy else [xs, xg]
+    return tensors + ([wt.q, wt.scale] if digits else [wt]), (lazy, digits)
+
+
+def _unpack_operands(how, tensors):
+    lazy, digits = how
+    xs, xg = tensors[:2]
+    if lazy:
+        xs = xg = _LazyBf16(xs)
+    return xs, _Digits(tensors[2], tensors[3]) if digits else tensors[2], xg
+
+
+def _split_synapse(x, w, stream, lean=False, bf16=True, ints=True):
     """Start the exact split of ``x @ W`` (see _Split)."""
 
-    return _Split(x, w, stream, lean)
+    return _Split(x, w, stream, lean, bf16, ints)
 
 
-def _split_eligible(prec: int, T: int, B: int, F: int, N: int) -> bool:
-    """fp32 synapse on the chunked route with rows the bf16 loaders take and
-    enough work to amortise the input check -- and no graph being captured
-    on the current stream: the split's choice needs the input check's flag
-    on the host (``_Split.exact``), a wait that capture does not allow and
-    whose answer a replay could not revisit, so captured layers keep the
-    fp32 engine."""
+def _split_eligible(prec: int, T: int, B: int, F: int, N: int, ints: bool = True) -> bool:
+    """fp32 synapse wide enough for tiles (narrower outputs stream the input
+    once through the narrow kernels) with enough work to amortise the input
+    check -- and no graph being captured on the current stream: the split's
+    choice needs the input check's flags on the host (``_Split.operands``),
+    a wait that capture does not allow and whose answer a replay could not
+    revisit, so captured layers keep the fp32 engine."""
 
-    return (prec == _lib.PREC["fp32"] and not _fused(B, N) and F % 8 == 0 and N % 8 == 0
-            and T * B * F * N >= _SPLIT_MIN_MACS and not torch.cuda.is_current_stream_capturing())
+    if prec != _lib.PREC["fp32"] or N <= 32 or F % 8 != 0 or N % 8 != 0 or T * B * F * N < _SPLIT_MIN_MACS:
+        return False
+    # the bf16 products alone: the shapes the fused kernel does not take
+    if _fused(B, N) and not (ints and _lib.load().myelin_spike_limit(F) > 0):
+        return False
+    return not torch.cuda.is_current_stream_capturing()
 
 
 class HipLinearFunction(torch.autograd.Function):
@@ -322,12 +411,14 @@ def _budgets(lean: bool, checkpoint, B: int, N: int) -> tuple[int, int]:
 
 def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, stream, *, m_final=None,
              spikes=None, pre=None, packed=None, rates=None, ckpt=None, ckpt_every=1, wt=None, exact=False,
-             pre_from=None, split=None, x32=None, x_bits=None, budget=_CURRENT_CHUNK_ELEMS, cur=None):
+             pre_from=None, x_bits=None, budget=_CURRENT_CHUNK_ELEMS, cur=None):
     """Synaptic currents + LIF recurrence over steps [t0, t1).
 
     ``x`` is fp32 with ``w [F, N]`` fp32, or bf16 (bf16 synapse) with ``wt``,
-    the bf16 transposed weight ``[N, F]``.  Fused (one launch, currents stay
-    in LDS) when N >= 64 and the fused grid has >= 1024 workgroups.
+    the bf16 transposed weight ``[N, F]``; or an exact split's operands: bf16
+    with ``wt`` its planes ``[3, N, F]``, or int8 with ``wt`` a _Digits.
+    Fused (one launch, currents stay in LDS) when N >= 64 and the fused grid
+    has >= 1024 workgroups, except on the exact split.
     Otherwise each workgroup would walk many chunks serially, so the steps
     are processed in chunks of up to ``budget`` currents: an MFMA GEMM (split-K
     when narrow) writes ``x_t @ W + b`` for the chunk, then the recurrence
@@ -339,12 +430,6 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     ``exact``: the GEMM never splits K, so a checkpointed forward and the
     backward's recompute of any chunk of it produce the same currents bit
     for bit (the fused kernel always sums that way).
-    ``split`` (a _Split whose ``xb`` / ``w3`` are passed as x / wt, with
-    ``x32`` the same steps of the fp32 input): the first chunk's GEMM is
-    launched on the split before ``split.exact()`` is asked, so the GPU
-    works while the host waits for the check; if the input is not
-    bf16-exact that GEMM is redone on the fp32 engine into the same buffer
-    and every later chunk takes the fp32 engine.
     ``x_bits``: the input as packed spike words ``[T, B, ceil(F / 32)]``,
     which the chunked route's GEMM reads in place of ``x`` (fp32 synapse
     weights ``w``; the same sums bit for bit).
@@ -358,14 +443,15 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
         F = w.shape[0]
     else:
         T, B, F = x.shape
-    half = x_bits is None and x.dtype == torch.bfloat16
+    digits = wt if isinstance(wt, _Digits) else None
+    half = x_bits is None and digits is None and x.dtype == torch.bfloat16
     parts = half and wt.ndim == 3  # exact split: wt holds the planes [3, N, F]
+    if digits is not None:
+        F = w.shape[0]
     N = wt.shape[-2] if half else w.shape[1]
-    if _fused(B, N):
+    if digits is None and not parts and _fused(B, N):
         if pre_from not in (None, t0):
             raise ValueError("pre_from is a chunked-route option")
-        if parts or split is not None:
-            raise ValueError("the split synapse is a chunked-route option")
         outs = (_lib.ptr(b), _lib.ptr(m0), _lib.ptr(m_final), _lib.ptr(spikes), _lib.ptr(pre), _lib.ptr(packed),
                 _lib.ptr(rates), _lib.ptr(ckpt), T, B, F, N, t0, t1, ckpt_every, decay, threshold, reset, slope, rule)
         if half:
@@ -396,7 +482,7 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     # T=2000, B=32: 7.92-8.01 ms overlapped, 7.53 serial), so they run in
     # turn on the one stream.
     overlap = False
-    if n > 1 and not half:
+    if n > 1 and not half and digits is None:
         main = torch.cuda.current_stream(dev)
         side = _side_stream(dev)
         overlap = main.cuda_stream == stream and side.cuda_stream != stream
@@ -422,6 +508,9 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
         if x_bits is not None:
             _gemm(x_bits[c0:c1], w, cur, rows, N, F, x_bits.shape[2], N, N, False, False, False, prec, s, bias=b,
                   a_bits=True, split=not exact)
+        elif digits is not None:
+            _lib.call("myelin_gemm_spikes", _lib.ptr(x[c0:c1]), _lib.ptr(digits.q), _lib.ptr(digits.scale),
+                      _lib.ptr(b), _lib.ptr(cur), rows, N, x.shape[2], N, s)
         elif parts:
             _gemm_parts(x[c0:c1], wt, 3, N * F, cur, rows, N, F, F, F, N, False, True, False, s, bias=b,
                         split=not exact)
@@ -429,11 +518,6 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
             _gemm(x[c0:c1], wt, cur, rows, N, F, F, F, N, False, True, False, prec, s, bias=b, split=not exact)
         else:
             _gemm(x[c0:c1], w, cur, rows, N, F, F, N, N, False, False, False, prec, s, bias=b, split=not exact)
-
-    def fallback():
-        # the input was not bf16-exact: the fp32 engine from here on
-        nonlocal x, wt, half, parts
-        x, wt, half, parts = x32, None, False, False
 
     for c in range(n):
         c0, c1 = bounds[c], bounds[c + 1]
@@ -444,9 +528,6 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
             if overlap and c >= 2:
                 side.wait_event(used[i])
             gemm(c0, c1, cur, s_)
-            if c == 0 and split is not None and not split.exact():
-                fallback()
-                gemm(c0, c1, cur, s_)
             if overlap:
                 done[i].record(side)
         if overlap:
@@ -465,7 +546,7 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     if overlap:
         # the main stream waited on every side GEMM; the inputs' and buffers'
         # last users include the side stream
-        for t_ in (*curs, x, w, b, wt, x32, *(() if split is None else (split.xb, split.w3))):
+        for t_ in (*curs, x, w, b, wt):
             if t_ is not None:
                 t_.record_stream(side)
 
@@ -542,10 +623,10 @@ class HipLinearLIFFunction(torch.autograd.Function):
         xs, wt = _cast_transpose_bf16(x, w, stream) if half else (x, None)
         bits = _spike_bits(x) if _bits_consumer(B, F, N, prec) else None
         fwd_budget, budget = _budgets(lean, checkpoint, B, N)
+        xg = xs
         split = None
-        if not half and bits is None and _split_eligible(prec, T, B, F, N):
-            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None)
-            xs, wt = split.xb, split.w3
+        if not half and bits is None and _split_eligible(prec, T, B, F, N, ints=not lean or checkpoint is None):
+            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None, bf16=need)
         m_final = torch.empty((B, N), dtype=x.dtype, device=dev)
         out = torch.empty((B, N) if rate else (T, B, N), dtype=x.dtype, device=dev)
         # spikes: their packed twin too (N / 8 bytes per row more), for a
@@ -553,6 +634,9 @@ class HipLinearLIFFunction(torch.autograd.Function):
         words = torch.empty((T, B, -(-N // 32)), dtype=torch.int32, device=dev) if not rate else None
         if checkpoint is not None and _keep_trace(F, N):
             checkpoint = None
+        if split is not None:
+            xs, wt, xg = split.operands()
+        chunked = not _fused(B, N) or _exact_split(wt)
         pre = ckpt = None
         tail = 0
         if need:
@@ -560,7 +644,7 @@ class HipLinearLIFFunction(torch.autograd.Function):
                 pre = torch.empty((T, B, N), dtype=x.dtype, device=dev)
             else:
                 ckpt = torch.empty((math.ceil(T / checkpoint), B, N), dtype=x.dtype, device=dev)
-                if not _fused(B, N):
+                if chunked:
                     # the backward starts with the last span, whose trace
                     # this forward computes anyway: keep it (the buffer the
                     # backward would fill) instead of recomputing it there
@@ -569,22 +653,22 @@ class HipLinearLIFFunction(torch.autograd.Function):
                     pre = torch.empty((T - tail, B, N), dtype=x.dtype, device=dev)
         _lif_fwd(xs, w, b, None, 0, T, decay, threshold, reset, slope, rule, prec, stream, m_final=m_final,
                  spikes=None if rate else out, pre=pre, packed=words, rates=out if rate else None, ckpt=ckpt,
-                 ckpt_every=checkpoint or 1, wt=wt, exact=ckpt is not None, pre_from=tail, split=split, x32=x,
-                 x_bits=bits, budget=fwd_budget)
-        if split is not None and not split.exact():
-            xs, wt = x, None
+                 ckpt_every=checkpoint or 1, wt=wt, exact=ckpt is not None, pre_from=tail, x_bits=bits,
+                 budget=fwd_budget)
         if words is not None:
             _attach_bits(out, words)
         if bits is not None:
-            xs = bits  # what the backward's weight GEMM reads
-        lazy = isinstance(xs, _LazyBf16)
+            xs = xg = bits  # what the backward's weight GEMM reads
         ctx.set_materialize_grads(False)
+        # the bf16 synapse keeps the bf16 copies of x and W^T (what its
+        # GEMMs read), the exact split its copies of x and form of W
+        if checkpoint is None:
+            xs, wt = (xg, wt) if not isinstance(wt, _Digits) else (xg, None)  # nothing to recompute
+        saved, how = _pack_operands(x, xs, wt, xg) if need else ((), None)
         ctx.meta = (decay, threshold, reset, sid, slope, checkpoint, rate, prec, rule, b is not None,
-                    F if bits is not None else None, budget, lazy)
+                    F if bits is not None else None, budget, how)
         if need:
-            # the bf16 synapse keeps the bf16 copies of x and W^T (what its
-            # GEMMs read); the lean split keeps x and casts per span
-            ctx.save_for_backward(x if lazy else xs, w, b, pre, ckpt, wt)
+            ctx.save_for_backward(w, b, pre, ckpt, *saved)
         return m_final, out
 
     @staticmethod
@@ -592,19 +676,18 @@ class HipLinearLIFFunction(torch.autograd.Function):
         none = (None,) * 13
         if (g_m is None and g_out is None) or not any(ctx.needs_input_grad[:3]):
             return none
-        decay, threshold, reset, sid, slope, checkpoint, rate, prec, rule, has_b, bits_f, budget, lazy = ctx.meta
-        xs, w, b, pre, ckpt, wt = ctx.saved_tensors
-        if lazy:
-            xs = _LazyBf16(xs)
+        decay, threshold, reset, sid, slope, checkpoint, rate, prec, rule, has_b, bits_f, budget, how = ctx.meta
+        w, b, pre, ckpt, *saved = ctx.saved_tensors
+        xs, wt, xg = _unpack_operands(how, saved)
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
         gx, gw, gb = linear_backward(xs, w, b if has_b else None, pre, ckpt, wt, g_m, g_out, decay, threshold,
                                      reset, sid, slope, checkpoint, rate, prec, rule, need_x, need_w,
-                                     need_b and has_b, bits_f=bits_f, budget=budget)
+                                     need_b and has_b, bits_f=bits_f, budget=budget, xg=xg)
         return gx, gw, gb, None, None, None, None, None, None, None, None, None, None
 
 
 def linear_backward(xs, w, b, pre, ckpt, wt, g_m, g_out, decay, threshold, reset, sid, slope, checkpoint, rate,
-                    prec, rule, need_x=True, need_w=True, need_b=True, bits_f=None, budget=_CURRENT_CHUNK_ELEMS):
+                    prec, rule, need_x=True, need_w=True, need_b=True, bits_f=None, budget=_CURRENT_CHUNK_ELEMS, xg=None):
     """Gradients (dX, dW, db) of the streamed-synapse LIF, span by span in
     reverse time: recompute the span's pre-reset trace from its first
     checkpoint (``checkpoint=None``: the saved trace ``pre`` covers all T;
@@ -613,18 +696,19 @@ def linear_backward(xs, w, b, pre, ckpt, wt, g_m, g_out, decay, threshold, reset
     ``dW += X^T G`` on the MFMA GEMM and ``db`` as a fixed-order column
     sum.  ``xs`` is fp32, or
     bf16 with ``wt = W^T`` bf16 for the bf16 synapse, or (``bits_f`` = F)
-    the input spikes' packed words ``[T, B, ceil(F / 32)]``; ``g_out`` is
-    dL/dspikes ``[T, B, N]`` or, with ``rate``, dL/drates ``[B, N]``."""
+    the input spikes' packed words ``[T, B, ceil(F / 32)]``, or an exact
+    split's operand with its ``wt`` (see _lif_fwd); ``xg`` is what dW's GEMM
+    reads where that is not ``xs``; ``g_out`` is dL/dspikes ``[T, B, N]`` or, with ``rate``, dL/drates ``[B, N]``."""
 
-    T, B, F = xs.shape
+    T, B = xs.shape[:2]
     x_bits = xs if bits_f is not None else None
-    if x_bits is not None:
-        F = bits_f
-    N = w.shape[1]
+    F, N = w.shape
     BN = B * N
-    dev = xs.device
-    parts = wt is not None and wt.ndim == 3  # exact split: xs bf16-exact, wt the planes of W
-    half = xs.dtype == torch.bfloat16 and not parts
+    dev = w.device
+    xg = xs if xg is None else xg
+    split = _exact_split(wt) or (xg.dtype == torch.bfloat16 and prec == _lib.PREC["fp32"])
+    half = xs.dtype == torch.bfloat16 and not split
+    parts = split and xg.dtype == torch.bfloat16  # dW: x exact in bf16, G as three planes
     with torch.cuda.device(dev):
         stream = _lib.stream(dev)
         wg = _cast_bf16(w, stream) if (half and need_x) else w
@@ -670,7 +754,7 @@ def linear_backward(xs, w, b, pre, ckpt, wt, g_m, g_out, decay, threshold, reset
         # overlaps span k's reverse pass and weight GEMMs (the bf16 engines
         # and the split run in turn, as in the forward).  ready[i]: buffer i
         # holds its span's trace; free[i]: the reverse pass has read buffer i.
-        overlap = checkpoint is not None and n_spans > 1 and not (half or parts)
+        overlap = checkpoint is not None and n_spans > 1 and not (half or split)
         # in turn, the trace buffer is spent once the reverse pass has read
         # it and is refilled only by the next span's recompute: it doubles
         # as the split-K workspace of the span's dX and dW GEMMs
@@ -751,14 +835,14 @@ def linear_backward(xs, w, b, pre, ckpt, wt, g_m, g_out, decay, threshold, reset
             if gw is not None and parts:
                 if G is not G3:
                     _lib.call("myelin_split_bf16x3", _lib.ptr(G), _lib.ptr(G3), rows, N, 0, stream)
-                _gemm_parts(xs[t0:t1], G3, 3, rows * N, gw, F, N, rows, F, N, N, True, False, k != n_spans - 1,
+                _gemm_parts(xg[t0:t1], G3, 3, rows * N, gw, F, N, rows, F, N, N, True, False, k != n_spans - 1,
                             stream, ws=ws, col_sum=cs)
             elif gw is not None and x_bits is not None:
                 _gemm(x_bits[t0:t1], G, gw, F, N, rows, x_bits.shape[2], N, N, True, False, k != n_spans - 1, prec,
                       stream, a_bits=True, ws=ws, col_sum=cs)
             elif gw is not None:
                 # dW (+)= X[t0:t1]^T @ G : [F, rows] x [rows, N]
-                _gemm(xs[t0:t1], G, gw, F, N, rows, F, N, N, True, False, k != n_spans - 1, prec, stream, ws=ws,
+                _gemm(xg[t0:t1], G, gw, F, N, rows, F, N, N, True, False, k != n_spans - 1, prec, stream, ws=ws,
                       col_sum=cs)
         if overlap:
             # every side-stream kernel is behind a ready[] the main stream
@@ -824,7 +908,10 @@ def linear_packed_forward(x, w, b, params, checkpoint: int, precision: str):
     m_final = torch.empty((B, N), device=x.device)
     words = torch.empty((T, B, packed_last_dim_size(N)), dtype=torch.int32, device=x.device)
     with torch.cuda.device(x.device):
-        _lif_fwd(x, w, b, None, 0, T, float(params.decay), float(params.threshold), float(params.reset), 10.0,
-                 _lib.RULE_THRESHOLD, _lib.PREC[precision], _lib.stream(x.device), m_final=m_final, packed=words,
-                 ckpt_every=checkpoint)
+        prec, stream = _lib.PREC[precision], _lib.stream(x.device)
+        xs, wt = x, None
+        if _split_eligible(prec, T, B, F, N):
+            xs, wt, _ = _split_synapse(x, w, stream, bf16=False).operands()
+        _lif_fwd(xs, w, b, None, 0, T, float(params.decay), float(params.threshold), float(params.reset), 10.0,
+                 _lib.RULE_THRESHOLD, prec, stream, m_final=m_final, packed=words, ckpt_every=checkpoint, wt=wt)
     return m_final, PackedSpikes(data=words, original_shape=(T, B, N))

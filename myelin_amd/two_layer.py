@@ -44,8 +44,8 @@ import torch
 
 from myelin_amd import _lib
 from myelin_amd.linear import (_CURRENT_CHUNK_ELEMS, _LEAN_FWD_ELEMS, _cast_bf16, _cast_transpose_bf16, _gemm,
-                               _gemm_parts, _half, _keep_trace, _LazyBf16, _lif_fwd, _side_stream, _split_eligible,
-                               _split_synapse)
+                               _gemm_parts, _half, _keep_trace, _lif_fwd, _exact_split, _pack_operands,
+                               _side_stream, _split_eligible, _split_synapse, _unpack_operands)
 
 # trace budget of a backward span (floats per buffer): the backward walks
 # whole checkpoint chunks, as many at a time as keep each per-span buffer
@@ -119,6 +119,21 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         O = wo.shape[1]
         dev = x.device
         stream = _lib.stream(dev)
+        # bf16 synapse: the hidden GEMMs read bf16 copies of x and W_h^T
+        half = _half(prec, F, H)
+        xs, wt = _cast_transpose_bf16(x, wh, stream) if half else (x, None)
+        # spike inputs: the hidden synapse on the exact bf16 products, its
+        # operands asked for below, when the input check has had the time of
+        # the allocations.  (The int8 products take a step at T=2000, B=32,
+        # 1024 -> 4096 -> 20 from 6.20 to 5.93 ms.  Both are exact but for
+        # the last rounding; a superspike adjoint amplifies a last bit over
+        # thousands of steps, and where the hidden layer is nearly silent
+        # the two routes' gradients, each 1.5e-5 from the true one, lie
+        # 2.8e-5 apart: this network keeps the sums its results were
+        # established with.)
+        split = None
+        if not half and _split_eligible(prec, T, B, F, H, ints=False):
+            split = _split_synapse(x, wh, stream, lean=lean, ints=False)
         need = any(ctx.needs_input_grad[:5])
         K = math.ceil(T / C)
         L0 = min(C, T)
@@ -146,15 +161,9 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         cur = torch.empty((T if packed_hidden else LG, B, O), device=dev)
         pre_o = torch.empty((T, B, O), device=dev) if keep else None
         words = torch.empty((T, B, (H + 31) // 32), dtype=torch.int32, device=dev) if packed_hidden else None
-        # bf16 synapse: the hidden GEMMs read bf16 copies of x and W_h^T
-        half = _half(prec, F, H)
-        xs, wt = _cast_transpose_bf16(x, wh, stream) if half else (x, None)
-        # spike inputs: the hidden synapse on the exact bf16 split (the first
-        # group's forward learns whether the input qualifies)
-        split = None
-        if not half and _split_eligible(prec, T, B, F, H):
-            split = _split_synapse(x, wh, stream, lean=lean)
-            xs, wt = split.xb, split.w3
+        xg = xs
+        if split is not None:
+            xs, wt, xg = split.operands()
         for k in range(0, K, G):
             t0 = k * C
             t1 = min(t0 + G * C, T)
@@ -162,10 +171,7 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
             _lif_fwd(xs[t0:t1], wh, bh, m_h, 0, L, decay, threshold, reset, slope, _lib.RULE_THRESHOLD, prec, stream,
                      m_final=m_h, spikes=None if hs is None else hs[:L],
                      packed=None if words is None else words[t0:t1], ckpt=None if ck_h is None else ck_h[k:],
-                     ckpt_every=C, wt=wt, exact=need, split=split if k == 0 else None,
-                     x32=x[t0:t1] if k == 0 else None, budget=LG * B * H)
-            if k == 0 and split is not None and not split.exact():
-                xs, wt = x, None
+                     ckpt_every=C, wt=wt, exact=need, budget=LG * B * H)
             if hs is not None:
                 _readout_chunk(cur[:L], hs[:L], wo, bo, m_o, m_o, None if pre_o is None else pre_o[t0:t1], counts,
                                rates if t1 == T else None, ck_o, T, t0, t1, C, decay, threshold, reset, slope, prec,
@@ -173,12 +179,12 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         if hs is None:
             _readout_chunk(cur, words, wo, bo, m_o, m_o, pre_o, counts, rates, ck_o, T, 0, T, C, decay, threshold,
                            reset, slope, prec, stream, exact=need and not keep)
-        lazy = isinstance(xs, _LazyBf16)
+        saved, how = _pack_operands(x, xs, wt, xg) if need else ((), None)
         ctx.set_materialize_grads(False)
-        ctx.meta = (decay, threshold, reset, sid, slope, C, prec, bh is not None, bo is not None, lean, lazy)
+        ctx.meta = (decay, threshold, reset, sid, slope, C, prec, bh is not None, bo is not None, lean, how)
         if need:
-            # the lean split keeps x and casts each span's steps to bf16
-            ctx.save_for_backward(x if lazy else xs, wh, bh, wo, bo, ck_h, ck_o, words, wt, pre_o)
+            # (the lean split keeps x and casts each span's steps)
+            ctx.save_for_backward(wh, bh, wo, bo, ck_h, ck_o, words, pre_o, *saved)
         return rates
 
     @staticmethod
@@ -186,18 +192,18 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         none = (None,) * 14
         if g_rates is None or not any(ctx.needs_input_grad[:5]):
             return none
-        decay, threshold, reset, sid, slope, C, prec, has_bh, has_bo, lean, lazy = ctx.meta
-        xs, wh, bh, wo, bo, ck_h, ck_o, words, wt, pre_all = ctx.saved_tensors
-        if lazy:
-            xs = _LazyBf16(xs)
-        parts = wt is not None and wt.ndim == 3  # exact split of the hidden synapse
-        half = xs.dtype == torch.bfloat16 and not parts
+        decay, threshold, reset, sid, slope, C, prec, has_bh, has_bo, lean, how = ctx.meta
+        wh, bh, wo, bo, ck_h, ck_o, words, pre_all, *saved = ctx.saved_tensors
+        xs, wt, xg = _unpack_operands(how, saved)
+        split = _exact_split(wt)  # of the hidden synapse
+        half = xs.dtype == torch.bfloat16 and not split
+        parts = split and xg.dtype == torch.bfloat16  # dW_h: x exact in bf16, G_h as three planes
         need_x, need_wh, need_bh, need_wo, need_bo = ctx.needs_input_grad[:5]
         need_hidden = need_x or need_wh or (need_bh and has_bh)
-        T, B, F = xs.shape
-        H = wh.shape[1]
+        T, B = xs.shape[:2]
+        F, H = wh.shape
         O = wo.shape[1]
-        dev = xs.device
+        dev = wh.device
         K = math.ceil(T / C)
         # spans of `per` whole chunks (recomputed from the span's first
         # checkpoints, which the recurrences carry through the later ones
@@ -410,15 +416,15 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
                     if parts:
                         if G_h is not G3:
                             _lib.call("myelin_split_bf16x3", _lib.ptr(G_h), _lib.ptr(G3), rows, H, 0, stream)
-                        _gemm_parts(xs[t0:t1], G3, 3, rows * H, gwh, F, H, rows, F, H, H, True, False, k != NS - 1,
+                        _gemm_parts(xg[t0:t1], G3, 3, rows * H, gwh, F, H, rows, F, H, H, True, False, k != NS - 1,
                                     stream, ws=pool, col_sum=cs)
                     else:
-                        _gemm(xs[t0:t1], G_h, gwh, F, H, rows, F, H, H, True, False, k != NS - 1, prec, stream,
+                        _gemm(xg[t0:t1], G_h, gwh, F, H, rows, F, H, H, True, False, k != NS - 1, prec, stream,
                               ws=pool, col_sum=cs)
             if nset == 2:
                 # every side-stream kernel is behind a ready[] the main stream
                 # waited on; these tensors' last users include the side stream
-                for t_ in (*hs_b, *pre_b, xs.x if lazy else xs, wh, ck_h, bh, wt):
+                for t_ in (*hs_b, *pre_b, *saved, wh, ck_h, bh):
                     if t_ is not None:
                         t_.record_stream(side)
             if o_side:
