@@ -190,6 +190,16 @@ int myelin_packed_counts(const int32_t *words, int ndim_lead,
                          int64_t n, int64_t *out, myelin_stream_t stream);
 
 /*
+ * As myelin_packed_counts, but out = count / denominator (dtype F32 or F64,
+ * the count converted first).  counts: as many int64 as outputs, scratch.
+ * Replaces: packing.packed_spike_rate's division (src/myelin/packing.py:145-162).
+ */
+int myelin_packed_rates(const int32_t *words, int ndim_lead,
+                        const int64_t *lead_shape, uint32_t reduce_mask,
+                        int64_t n, int64_t denominator, int64_t *counts,
+                        void *out, int dtype, myelin_stream_t stream);
+
+/*
  * Per-neuron counts over a block of leading rows that are NOT packed:
  * words viewed as [R, K, ceil(n/32)]; out[k, j] = sum_r bit j of row (r, k),
  * int64 [K, n].

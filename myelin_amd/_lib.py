@@ -55,6 +55,7 @@ SIGNATURES: dict[str, list] = {
     "myelin_pack": [_P, _INT, _P, _I64, _I64, _P],
     "myelin_unpack": [_P, _P, _INT, _I64, _I64, _P],
     "myelin_packed_counts": [_P, _INT, _P, ctypes.c_uint32, _I64, _P, _P],
+    "myelin_packed_rates": [_P, _INT, _P, ctypes.c_uint32, _I64, _I64, _P, _P, _INT, _P],
     "myelin_packed_counts_keep_last": [_P, _I64, _I64, _I64, _P, _P],
     "myelin_counts_to_rate": [_P, _P, _INT, _I64, _I64, _P],
     "myelin_gemm_f32": [_P, _P, _P, _P] + [_I64] * 6 + [_INT] * 4 + [_P, _I64, _P],

@@ -1,11 +1,13 @@
 // Spike bitpacking for gfx950: 32 spikes per int32 word along the last
 // dimension, bit i of word w = element 32*w + i (LSB first), padding bits 0.
 //
-// pack:   one lane per element; a wave ballot turns 64 consecutive elements
-//         into two words.  Each wave handles 64 words (32 ballots) per pass
-//         and lane j stores word j, so the word store is one coalesced
-//         256-byte write and every element load is a coalesced wave load.
-// unpack: one lane per 4 elements (same word), vector store of 4 outputs.
+// pack:   elements of 4 and 8 bytes: one lane per element; a wave ballot
+//         turns 64 consecutive elements into two words.  Each wave handles
+//         64 words (32 ballots) per pass and lane j stores word j, so the
+//         word store is one coalesced 256-byte write and every element load
+//         is a coalesced wave load.  Elements of 1 and 2 bytes: one lane per
+//         word, which reads its 32 elements as whole dwords.
+// unpack: one lane per 16 bytes of output.
 // counts: popcount with the padding bits of the last word masked.
 
 #include "common.h"
@@ -23,13 +25,11 @@ struct F64 {
   using T = double;
   __device__ static bool nz(double v) { return v != 0.0; }
 };
-struct H16 {  // fp16 and bf16: zero iff all bits but the sign are zero
+struct H16 {  // fp16 and bf16: zero iff all bits but the sign are zero (nonzero_bits)
   using T = uint16_t;
-  __device__ static bool nz(uint16_t v) { return (v & 0x7fffu) != 0; }
 };
 struct U8 {
   using T = uint8_t;
-  __device__ static bool nz(uint8_t v) { return v != 0; }
 };
 struct I32 {
   using T = int32_t;
@@ -41,7 +41,9 @@ struct I64 {
 };
 
 // words: [rows, W]; total = rows * W.  ALIGNED: n % 32 == 0 so the element
-// of (word g, bit i) is simply 32*g + i.
+// of (word g, bit i) is simply 32*g + i; else a lane's row and column are
+// found by one division and then advanced two words at a time (a 64-bit
+// division per word: 15000 rows of 2312 floats 44.6 -> 22.3 us).
 template <class E, bool ALIGNED>
 __global__ __launch_bounds__(256) void pack_kernel(const typename E::T *__restrict__ src, int32_t *__restrict__ words,
                                                    int64_t total, int64_t W, int64_t n) {
@@ -52,17 +54,39 @@ __global__ __launch_bounds__(256) void pack_kernel(const typename E::T *__restri
   const int half = lane >> 5, bit = lane & 31;
 
   typename E::T v[32];
+  if constexpr (ALIGNED) {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    const int64_t g = g0 + 2 * i + half;
-    v[i] = typename E::T(0);
-    if (g < total) {
-      if constexpr (ALIGNED) {
-        v[i] = __builtin_nontemporal_load(src + g * 32 + bit);
-      } else {
-        const int64_t r = g / W;
-        const int64_t col = (g - r * W) * 32 + bit;
-        if (col < n) v[i] = src[r * n + col];
+    for (int i = 0; i < 32; ++i) {
+      const int64_t g = g0 + 2 * i + half;
+      v[i] = typename E::T(0);
+      if (g < total) v[i] = __builtin_nontemporal_load(src + g * 32 + bit);
+    }
+  } else {
+    int64_t r = (g0 + half) / W;
+    int64_t col = (g0 + half - r * W) * 32 + bit;
+    const typename E::T *p = src + r * n + col;
+    const int64_t wide = W * 32, pad = wide - n;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      v[i] = typename E::T(0);
+      if (g0 + 2 * i + half < total && col < n) {
+        // (streamed 8-byte loads of unaligned rows measured slower: 30000 x
+        // 1000 doubles 56 -> 65 us)
+        if constexpr (sizeof(typename E::T) == 8)
+          v[i] = *p;
+        else
+          v[i] = __builtin_nontemporal_load(p);
+      }
+      // two words on: past the row's last word, `pad` elements fewer per row
+      col += 64;
+      p += 64;
+      if (col >= wide) {
+        col -= wide;
+        p -= pad;
+        if (col >= wide) {  // rows of one word
+          col -= wide;
+          p -= pad;
+        }
       }
     }
   }
@@ -77,32 +101,140 @@ __global__ __launch_bounds__(256) void pack_kernel(const typename E::T *__restri
   if (g0 + lane < total) words[g0 + lane] = static_cast<int32_t>(mine);
 }
 
-// ALIGNED (n % 32 == 0): lane handles 4 consecutive elements of one word.
-template <typename S>
-__global__ __launch_bounds__(256) void unpack_aligned(const int32_t *__restrict__ words, S *__restrict__ dst,
-                                                      int64_t quads, S one) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= quads) return;
-  const int64_t e = q * 4;
-  const uint32_t w = static_cast<uint32_t>(words[e >> 5]);
-  const uint32_t nib = (w >> (e & 31)) & 0xfu;
-  S out[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) out[i] = ((nib >> i) & 1u) ? one : S(0);
-  if constexpr (sizeof(S) == 4) {
-    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    u4 t = {out[0], out[1], out[2], out[3]};
-    __builtin_nontemporal_store(t, reinterpret_cast<u4 *>(dst + e));
-  } else if constexpr (sizeof(S) == 2) {
-    typedef uint16_t h4 __attribute__((ext_vector_type(4)));
-    h4 t = {out[0], out[1], out[2], out[3]};
-    __builtin_nontemporal_store(t, reinterpret_cast<h4 *>(dst + e));
+// The bits of the nonzero elements in a dword of four bytes or of two
+// halves (zero but for the sign), the first element in bit 0.
+template <int SIZE>
+__device__ __forceinline__ uint32_t nonzero_bits(uint32_t d) {
+  if constexpr (SIZE == 1) {
+    // bit 7 of each byte: some bit of it is set; then the four gathered into
+    // the top nibble by one multiplication (no two products share a bit)
+    const uint32_t t = ((d & 0x7f7f7f7fu) + 0x7f7f7f7fu) | d;
+    return (((t >> 7) & 0x01010101u) * 0x10204080u) >> 28;
   } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[e + i] = out[i];
+    const uint32_t t = (d & 0x7fff7fffu) + 0x7fff7fffu;  // bit 15 / 31: magnitude not zero
+    return ((t >> 15) & 1u) | ((t >> 30) & 2u);
   }
 }
 
+// One lane per word, elements of SIZE (1 or 2) bytes: the lane's 32 elements
+// are 8 SIZE dwords.  Rows that start on multiples of G = 16 or 8 bytes are
+// read G bytes at a time; others (G = 4) as the whole dwords that hold the
+// elements (one more where the row is not dword-aligned), shifted into
+// place.  A piece past the last element's is never read.  (Byte elements
+// used to take one load instruction per 64 bytes of a wave and a 64-bit
+// division per word: 15000 rows of 2312 bytes, G = 8, 44.8 -> 6.4 us (6.1
+// TB/s); of 2311, G = 4, 44.6 -> 18.3 us; 8192 bf16, G = 16, 289 -> 111 us
+// for 32768 rows.)
+template <int SIZE, int G>
+__global__ __launch_bounds__(256) void pack_words(const uint8_t *__restrict__ src, int32_t *__restrict__ words,
+                                                  int64_t total, int64_t W, int64_t n) {
+  typedef uint32_t vec __attribute__((ext_vector_type(G / 4)));
+  constexpr int ND = 8 * SIZE, NV = 4 * ND / G + (G == 4 ? 1 : 0);  // dwords of a word, pieces read
+  const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (g >= total) return;
+  int64_t r;
+  if (total <= 0x7fffffff)  // 32-bit division
+    r = static_cast<uint32_t>(g) / static_cast<uint32_t>(W);
+  else
+    r = g / W;
+  const int64_t col = (g - r * W) * 32;
+  const int64_t left = n - col;  // elements of this word, if under 32
+  const uintptr_t first = reinterpret_cast<uintptr_t>(src) + static_cast<uintptr_t>((r * n + col) * SIZE);
+  const uintptr_t last = first + static_cast<uintptr_t>((left < 32 ? left : 32) * SIZE - 1);
+  const vec *p = reinterpret_cast<const vec *>(first & ~uintptr_t{G - 1});
+  const int lim = static_cast<int>(last / G - first / G);  // pieces past the first that hold elements
+  vec v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) v[i] = p[i < lim ? i : lim];
+  uint32_t word = 0;
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    uint32_t d;
+    if constexpr (G == 4) {
+      const uint32_t sh = static_cast<uint32_t>(first & 3) * 8;
+      d = static_cast<uint32_t>(((static_cast<uint64_t>(v[i + 1][0]) << 32) | v[i][0]) >> sh);
+    } else {
+      d = v[i / (G / 4)][i % (G / 4)];
+    }
+    word |= nonzero_bits<SIZE>(d) << (4 / SIZE * i);
+  }
+  if (left < 32) word &= (1u << left) - 1u;
+  words[g] = static_cast<int32_t>(word);
+}
+
+// The `count` (<= 16) bits from column `col` of a row of words on, reading
+// only words that hold some of them.
+__device__ __forceinline__ uint32_t row_bits(const int32_t *__restrict__ row, int64_t col, int count) {
+  const uint32_t s = static_cast<uint32_t>(col & 31);
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(row) + (col >> 5);
+  uint32_t b = w[0] >> s;
+  if (s + count > 32) b |= w[1] << (32 - s);
+  return b & ((1u << count) - 1u);
+}
+
+// One lane per 16 bytes (PER elements) of the flat output, one vector store.
+// ALIGNED (n % 32 == 0): the elements share a word.  Otherwise a lane finds
+// its row by one division, and where its elements run past the row's end
+// continues with the next row's; the last elements of an output that is no
+// multiple of 16 bytes are stored one by one.  (A division and a store per
+// byte took 51.8 us on 15000 rows of 2312 bytes, this 6.7; on aligned rows a
+// byte's own stores 106 -> 41 us for 32768 x 8192.)
+template <typename S, bool ALIGNED>
+__global__ __launch_bounds__(256) void unpack_kernel(const int32_t *__restrict__ words, S *__restrict__ dst,
+                                                     int64_t total, int64_t n, int64_t W, S one) {
+  constexpr int PER = 16 / sizeof(S);
+  const int64_t e = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * PER;
+  if (e >= total) return;
+  const int m = total - e < PER ? static_cast<int>(total - e) : PER;  // elements of this lane
+  uint32_t bits;
+  if constexpr (ALIGNED) {
+    bits = static_cast<uint32_t>(words[e >> 5]) >> (e & 31);
+  } else {
+    int64_t r;
+    if (total <= 0x7fffffff && n <= 0x7fffffff)
+      r = static_cast<uint32_t>(e) / static_cast<uint32_t>(n);
+    else
+      r = e / n;
+    int64_t col = e - r * n;
+    const int32_t *row = words + r * W;
+    int got = n - col < m ? static_cast<int>(n - col) : m;
+    bits = row_bits(row, col, got);
+    while (got < m) {  // the next row, or rows narrower than the lane
+      row += W;
+      const int take = n < m - got ? static_cast<int>(n) : m - got;
+      bits |= row_bits(row, 0, take) << got;
+      got += take;
+    }
+  }
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  u4 out;
+  if constexpr (sizeof(S) == 1) {
+    // bit i of a nibble to byte i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = ((((bits >> (4 * i)) & 0xfu) * 0x00204081u) & 0x01010101u) * one;
+  } else if constexpr (sizeof(S) == 2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      out[i] = ((bits >> (2 * i)) & 1u) * one + (((bits >> (2 * i + 1)) & 1u) * (static_cast<uint32_t>(one) << 16));
+  } else if constexpr (sizeof(S) == 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = ((bits >> i) & 1u) ? one : 0u;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint64_t v = ((bits >> i) & 1u) ? one : S(0);
+      out[2 * i] = static_cast<uint32_t>(v);
+      out[2 * i + 1] = static_cast<uint32_t>(v >> 32);
+    }
+  }
+  if (m == PER) {
+    __builtin_nontemporal_store(out, reinterpret_cast<u4 *>(dst + e));
+  } else {
+    for (int i = 0; i < m; ++i) dst[e + i] = ((bits >> i) & 1u) ? one : S(0);
+  }
+}
+
+// outputs that do not start on 16 bytes
 template <typename S>
 __global__ __launch_bounds__(256) void unpack_generic(const int32_t *__restrict__ words, S *__restrict__ dst,
                                                       int64_t total, int64_t n, int64_t W, S one) {
@@ -134,6 +266,15 @@ __device__ __forceinline__ int64_t out_index(int64_t row, const LeadInfo &li) {
   return idx;
 }
 
+// a finished count as the kernel's output: itself, or the rate count / denom
+template <typename OUT>
+__device__ __forceinline__ OUT finish(int64_t c, OUT denom) {
+  if constexpr (sizeof(OUT) == 8 && OUT(0.5) == OUT(0))
+    return c;
+  else
+    return static_cast<OUT>(c) / denom;
+}
+
 __device__ __forceinline__ int64_t wave_sum(int64_t v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
@@ -142,9 +283,10 @@ __device__ __forceinline__ int64_t wave_sum(int64_t v) {
 
 // One wave per row.  DIRECT: out[row] = count (every leading dim kept);
 // otherwise atomically accumulate into the kept-dims index (out zeroed).
-template <bool DIRECT>
+template <bool DIRECT, typename OUT>
 __global__ __launch_bounds__(256) void row_counts_wave(const int32_t *__restrict__ words, int64_t rows, int64_t W,
-                                                       uint32_t last_mask, LeadInfo li, int64_t *__restrict__ out) {
+                                                       uint32_t last_mask, LeadInfo li, OUT *__restrict__ out,
+                                                       OUT denom) {
   const int lane = static_cast<int>(threadIdx.x & (kWave - 1));
   const int64_t row = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
   if (row >= rows) return;
@@ -158,7 +300,7 @@ __global__ __launch_bounds__(256) void row_counts_wave(const int32_t *__restrict
   c = wave_sum(c);
   if (lane == 0) {
     if constexpr (DIRECT) {
-      out[row] = c;
+      out[row] = finish<OUT>(c, denom);
     } else {
       atomicAdd(reinterpret_cast<unsigned long long *>(out + out_index(row, li)), static_cast<unsigned long long>(c));
     }
@@ -166,9 +308,10 @@ __global__ __launch_bounds__(256) void row_counts_wave(const int32_t *__restrict
 }
 
 // One lane per row, for short rows (W < 16).
-template <bool DIRECT>
+template <bool DIRECT, typename OUT>
 __global__ __launch_bounds__(256) void row_counts_lane(const int32_t *__restrict__ words, int64_t rows, int64_t W,
-                                                       uint32_t last_mask, LeadInfo li, int64_t *__restrict__ out) {
+                                                       uint32_t last_mask, LeadInfo li, OUT *__restrict__ out,
+                                                       OUT denom) {
   const int64_t row = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (row >= rows) return;
   const int32_t *rw = words + row * W;
@@ -179,7 +322,7 @@ __global__ __launch_bounds__(256) void row_counts_lane(const int32_t *__restrict
     c += __popc(w);
   }
   if constexpr (DIRECT) {
-    out[row] = c;
+    out[row] = finish<OUT>(c, denom);
   } else {
     atomicAdd(reinterpret_cast<unsigned long long *>(out + out_index(row, li)), static_cast<unsigned long long>(c));
   }
@@ -194,9 +337,10 @@ __global__ __launch_bounds__(256) void row_counts_lane(const int32_t *__restrict
 // integer sums are order-independent).
 constexpr int kBlkWaves = 16;
 
+template <typename OUT>
 __global__ __launch_bounds__(1024) void row_counts_block(const int32_t *__restrict__ words, int64_t W,
                                                          uint32_t last_mask, int64_t P, int64_t Q, int64_t AQ,
-                                                         int64_t slice, int atomic, int64_t *__restrict__ out) {
+                                                         int64_t slice, int atomic, OUT *__restrict__ out, OUT denom) {
   __shared__ int64_t part[kBlkWaves];
   const int lane = static_cast<int>(threadIdx.x & 63), q = static_cast<int>(threadIdx.x >> 6);
   const int64_t o = blockIdx.x;
@@ -230,7 +374,7 @@ __global__ __launch_bounds__(1024) void row_counts_block(const int32_t *__restri
     if (atomic)
       atomicAdd(reinterpret_cast<unsigned long long *>(out + o), static_cast<unsigned long long>(t));
     else
-      out[o] = t;
+      out[o] = finish<OUT>(t, denom);
   }
 }
 
@@ -244,9 +388,9 @@ __global__ __launch_bounds__(256) void fill_i64(int64_t *__restrict__ p, int64_t
 // inside the block's row range, 16 rows' loads issued before any is used.
 // Bit counts are accumulated SWAR-style: acc[j] holds, in its 4 bytes, the
 // counts of bits j, j+8, j+16, j+24.  A block spans at most 8 * 255 rows,
-// so no byte passes 255 before the wave's counts are unpacked.  The 8
-// waves are then reduced through LDS; a block covering all R rows stores,
-// otherwise it atomically adds (out zeroed).
+// so no byte of a wave's counts passes 255.  The 8 waves' counts are then
+// summed through LDS; a block covering all R rows stores, otherwise it
+// atomically adds (out zeroed).
 constexpr int kKeepWaves = 8;
 constexpr int kKeepRows = kKeepWaves * 255;  // rows per block
 constexpr int kKeepAhead = 16;               // row loads in flight per lane
@@ -254,7 +398,7 @@ constexpr int kKeepAhead = 16;               // row loads in flight per lane
 __global__ __launch_bounds__(512) void keep_last_counts(const int32_t *__restrict__ words, int64_t R, int64_t KW,
                                                         int64_t W, int64_t n, int64_t *__restrict__ out,
                                                         int atomic) {
-  __shared__ int32_t red[kKeepWaves - 1][32][64];
+  __shared__ uint8_t red[kKeepWaves][32][68];  // [wave][bit][word column], each at most 255
   const int lane = static_cast<int>(threadIdx.x & 63);
   const int q = static_cast<int>(threadIdx.x >> 6);
   const int64_t col = static_cast<int64_t>(blockIdx.x) * 64 + lane;  // (k, w) flattened
@@ -262,7 +406,6 @@ __global__ __launch_bounds__(512) void keep_last_counts(const int32_t *__restric
   const int64_t r_begin = static_cast<int64_t>(blockIdx.y) * kKeepRows;
   const int64_t r_end = (r_begin + kKeepRows < R) ? r_begin + kKeepRows : R;
 
-  int32_t cnt[32];
   uint32_t acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = 0;
@@ -287,28 +430,28 @@ __global__ __launch_bounds__(512) void keep_last_counts(const int32_t *__restric
 #pragma unroll
   for (int j = 0; j < 8; ++j)
 #pragma unroll
-    for (int y = 0; y < 4; ++y) cnt[8 * y + j] = static_cast<int32_t>((acc[j] >> (8 * y)) & 0xffu);
-  if (q > 0) {
-#pragma unroll
-    for (int b = 0; b < 32; ++b) red[q - 1][b][lane] = cnt[b];
-  }
+    for (int y = 0; y < 4; ++y) red[q][8 * y + j][lane] = static_cast<uint8_t>(acc[j] >> (8 * y));
   __syncthreads();
-  if (q == 0 && active) {
-    for (int o = 0; o < kKeepWaves - 1; ++o)
+  // the block's 64 words x 32 bits in output order, lanes along the bits:
+  // coalesced stores (one wave adding up and each lane storing its own
+  // word's 32 counts: 32768 rows of 8192 bits 31.6 -> 25.9 us)
 #pragma unroll
-      for (int b = 0; b < 32; ++b) cnt[b] += red[o][b][lane];
-    const int64_t k = col / W;
-    const int64_t w = col - k * W;
+  for (int u = 0; u < 2048 / (64 * kKeepWaves); ++u) {
+    const int i = u * 64 * kKeepWaves + static_cast<int>(threadIdx.x);
+    const int wc = i >> 5, bit = i & 31;
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * 64 + wc;
+    if (c >= KW) continue;
+    int32_t sum = 0;
 #pragma unroll
-    for (int b = 0; b < 32; ++b) {
-      const int64_t j = w * 32 + b;
-      if (j < n) {
-        int64_t *dst = out + k * n + j;
-        if (atomic)
-          atomicAdd(reinterpret_cast<unsigned long long *>(dst), static_cast<unsigned long long>(cnt[b]));
-        else
-          *dst = cnt[b];
-      }
+    for (int o = 0; o < kKeepWaves; ++o) sum += red[o][bit][wc];
+    const int64_t k = c / W;
+    const int64_t j = (c - k * W) * 32 + bit;
+    if (j < n) {
+      int64_t *dst = out + k * n + j;
+      if (atomic)
+        atomicAdd(reinterpret_cast<unsigned long long *>(dst), static_cast<unsigned long long>(sum));
+      else
+        *dst = sum;
     }
   }
 }
@@ -326,25 +469,39 @@ template <class E>
 int pack_typed(const void *src, int32_t *words, int64_t rows, int64_t n, hipStream_t s) {
   const int64_t W = (n + 31) / 32;
   const int64_t total = rows * W;
-  const int64_t waves = (total + 63) / 64;
-  const dim3 grid(blocks(waves * 64));
-  const auto *p = static_cast<const typename E::T *>(src);
-  if (n % 32 == 0)
-    pack_kernel<E, true><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
-  else
-    pack_kernel<E, false><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+  constexpr int size = sizeof(typename E::T);
+  if constexpr (size <= 2) {
+    const auto *p = static_cast<const uint8_t *>(src);
+    const dim3 grid(blocks(total));
+    if (n * size % 16 == 0 && myelin::aligned(src, 16))
+      pack_words<size, 16><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+    else if (n * size % 8 == 0 && myelin::aligned(src, 8))
+      pack_words<size, 8><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+    else
+      pack_words<size, 4><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+  } else {
+    const int64_t waves = (total + 63) / 64;
+    const dim3 grid(blocks(waves * 64));
+    const auto *p = static_cast<const typename E::T *>(src);
+    if (n % 32 == 0)
+      pack_kernel<E, true><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+    else
+      pack_kernel<E, false><<<grid, dim3(256), 0, s>>>(p, words, total, W, n);
+  }
   return myelin::launched("pack");
 }
 
 template <typename S>
 int unpack_typed(const int32_t *words, void *dst, int64_t rows, int64_t n, S one, hipStream_t s) {
-  const int64_t W = (n + 31) / 32;
+  const int64_t W = (n + 31) / 32, total = rows * n;
   S *d = static_cast<S *>(dst);
-  if (n % 32 == 0 && myelin::aligned(dst, 4 * sizeof(S))) {
-    const int64_t quads = rows * n / 4;
-    unpack_aligned<S><<<dim3(blocks(quads)), dim3(256), 0, s>>>(words, d, quads, one);
+  if (myelin::aligned(dst, 16)) {
+    const dim3 grid(blocks((total + 16 / sizeof(S) - 1) / (16 / sizeof(S))));
+    if (n % 32 == 0)
+      unpack_kernel<S, true><<<grid, dim3(256), 0, s>>>(words, d, total, n, W, one);
+    else
+      unpack_kernel<S, false><<<grid, dim3(256), 0, s>>>(words, d, total, n, W, one);
   } else {
-    const int64_t total = rows * n;
     unpack_generic<S><<<dim3(blocks(total)), dim3(256), 0, s>>>(words, d, total, n, W, one);
   }
   return myelin::launched("unpack");
@@ -388,11 +545,18 @@ extern "C" int myelin_unpack(const int32_t *words, void *dst, int dtype, int64_t
   }
 }
 
-extern "C" int myelin_packed_counts(const int32_t *words, int ndim_lead, const int64_t *lead_shape,
-                                    uint32_t reduce_mask, int64_t n, int64_t *out, myelin_stream_t stream) {
+namespace {
+
+// Counts (OUT int64) or rates count / denom (float, double) over dims that
+// include the last.  `counts` is where counts are summed that several
+// workgroups add to (the output itself for OUT int64).
+template <typename OUT>
+int counts_impl(const int32_t *words, int ndim_lead, const int64_t *lead_shape, uint32_t reduce_mask, int64_t n,
+                OUT *out, OUT denom, int64_t *counts, hipStream_t s) {
+  constexpr bool RATE = !(sizeof(OUT) == 8 && OUT(0.5) == OUT(0));
   if (ndim_lead < 0 || ndim_lead > 8) return myelin::invalid("packed_counts: 0..8 leading dims supported");
   if (n < 1) return myelin::invalid("packed_counts: n must be >= 1");
-  if (out == nullptr || (ndim_lead > 0 && lead_shape == nullptr)) return myelin::invalid("packed_counts: null pointer");
+  if (out == nullptr || counts == nullptr || (ndim_lead > 0 && lead_shape == nullptr)) return myelin::invalid("packed_counts: null pointer");
   LeadInfo li{};
   li.ndim = ndim_lead;
   int64_t rows = 1, kept = 1;
@@ -407,7 +571,6 @@ extern "C" int myelin_packed_counts(const int32_t *words, int ndim_lead, const i
       kept *= lead_shape[d];
     }
   }
-  hipStream_t s = myelin::as_hip(stream);
   const uint32_t lead_mask = ndim_lead > 0 ? ((1u << ndim_lead) - 1u) : 0u;
   const bool direct = (reduce_mask & lead_mask) == 0;
   // kept leading dims [d0, d1] contiguous (or none kept): out = (row / Q) % P
@@ -432,38 +595,76 @@ extern "C" int myelin_packed_counts(const int32_t *words, int ndim_lead, const i
   int64_t S = 1;
   if (block_ok) {
     S = cdiv64(256, kept);
+    // up to 128 KB of words an output, one workgroup sums them sooner than
+    // several with a zeroing launch before them (50 outputs of 300 rows of
+    // 73 words: 5.2 + 4.7 -> 6 us)
+    if (AQ * ((n + 31) / 32) <= 32768) S = 1;
     const int64_t by_rows = cdiv64(AQ, 64);
     if (S > by_rows) S = by_rows;
     if (S > 65535) S = 65535;
     if (S < 1) S = 1;
   }
-  if (!direct && (!block_ok || S > 1)) {
-    fill_i64<<<dim3(blocks(kept)), dim3(256), 0, s>>>(out, kept);
+  // several workgroups add to an output: zeroed counts, and for rates the
+  // division after them
+  const bool shared = !direct && (!block_ok || S > 1);
+  const auto divide = [&]() {
+    if constexpr (RATE) {
+      if (kept > 0) rate_kernel<OUT><<<dim3(blocks(kept)), dim3(256), 0, s>>>(counts, out, kept, denom);
+    }
+    return myelin::launched("packed_counts");
+  };
+  if (shared || rows == 0) {
+    if (kept == 0) return MYELIN_OK;
+    fill_i64<<<dim3(blocks(kept)), dim3(256), 0, s>>>(counts, kept);
     if (int rc = myelin::launched("packed_counts zero")) return rc;
   }
-  if (rows == 0) return MYELIN_OK;
+  if (rows == 0) return divide();
   if (words == nullptr) return myelin::invalid("packed_counts: null words");
   const int64_t W = (n + 31) / 32;
   const int rem = static_cast<int>(n % 32);
   const uint32_t last_mask = rem ? ((1u << rem) - 1u) : 0xffffffffu;
   if (block_ok) {
     const int64_t slice = cdiv64(AQ, S);
-    row_counts_block<<<dim3(static_cast<unsigned>(kept), static_cast<unsigned>(S)), dim3(1024), 0, s>>>(
-        words, W, last_mask, P, Q, AQ, slice, S > 1 ? 1 : 0, out);
+    const dim3 grid(static_cast<unsigned>(kept), static_cast<unsigned>(S)), block(1024);
+    if (S > 1)
+      row_counts_block<int64_t><<<grid, block, 0, s>>>(words, W, last_mask, P, Q, AQ, slice, 1, counts, 1);
+    else
+      row_counts_block<OUT><<<grid, block, 0, s>>>(words, W, last_mask, P, Q, AQ, slice, 0, out, denom);
   } else if (W >= 16) {
     const dim3 grid(blocks(rows * 64));
     if (direct)
-      row_counts_wave<true><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out);
+      row_counts_wave<true, OUT><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out, denom);
     else
-      row_counts_wave<false><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out);
+      row_counts_wave<false, int64_t><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, counts, 1);
   } else {
     const dim3 grid(blocks(rows));
     if (direct)
-      row_counts_lane<true><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out);
+      row_counts_lane<true, OUT><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out, denom);
     else
-      row_counts_lane<false><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, out);
+      row_counts_lane<false, int64_t><<<grid, dim3(256), 0, s>>>(words, rows, W, last_mask, li, counts, 1);
   }
+  if (shared) return divide();
   return myelin::launched("packed_counts");
+}
+
+}  // namespace
+
+extern "C" int myelin_packed_counts(const int32_t *words, int ndim_lead, const int64_t *lead_shape,
+                                    uint32_t reduce_mask, int64_t n, int64_t *out, myelin_stream_t stream) {
+  return counts_impl<int64_t>(words, ndim_lead, lead_shape, reduce_mask, n, out, 1, out, myelin::as_hip(stream));
+}
+
+extern "C" int myelin_packed_rates(const int32_t *words, int ndim_lead, const int64_t *lead_shape,
+                                   uint32_t reduce_mask, int64_t n, int64_t denominator, int64_t *counts, void *out,
+                                   int dtype, myelin_stream_t stream) {
+  hipStream_t s = myelin::as_hip(stream);
+  if (dtype == MYELIN_DT_F32)
+    return counts_impl<float>(words, ndim_lead, lead_shape, reduce_mask, n, static_cast<float *>(out),
+                              static_cast<float>(denominator), counts, s);
+  if (dtype == MYELIN_DT_F64)
+    return counts_impl<double>(words, ndim_lead, lead_shape, reduce_mask, n, static_cast<double *>(out),
+                               static_cast<double>(denominator), counts, s);
+  return myelin::invalid("packed_rates: dtype must be F32 or F64");
 }
 
 extern "C" int myelin_packed_counts_keep_last(const int32_t *words, int64_t R, int64_t K, int64_t n, int64_t *out,

@@ -129,8 +129,7 @@ def packed_spike_counts(packed: PackedSpikes, dim: CountDim = -1) -> torch.Tenso
 
     _validate_packed_spikes(packed)
     _lib.require_device(packed.data, "packed.data")
-    shape = packed.original_shape
-    nd = len(shape)
+    nd = len(packed.original_shape)
     if dim is None:
         dims = tuple(range(nd))
     else:
@@ -140,23 +139,35 @@ def packed_spike_counts(packed: PackedSpikes, dim: CountDim = -1) -> torch.Tenso
                 "packed_spike_counts requires reducing the packed/original last dimension; "
                 "use packed_spike_count for dense-like reductions that keep that dimension"
             )
-    lead = shape[:-1]
-    mask = 0
-    for d in dims:
-        if d != nd - 1:
-            mask |= 1 << d
-    kept = tuple(s for i, s in enumerate(lead) if not (mask >> i) & 1)
+    kept, call = _reduction(packed, dims)
     out = torch.empty(kept, dtype=torch.int64, device=packed.data.device)
-    words = packed.data.contiguous()
-    lead_arr = (ctypes.c_int64 * max(1, len(lead)))(*lead)
+    call("myelin_packed_counts", _lib.ptr(out))
+    return out
+
+
+def _reduction(packed: PackedSpikes, dims: tuple[int, ...]):
+    """(shape kept, call) of a reduction over ``dims``, the last among them;
+    ``call(name, *args)`` runs the entry point on its words, leading shape,
+    mask and row length, the given arguments and the stream."""
+
+    shape = packed.original_shape
+    lead = shape[:-1]
     if len(lead) > 8:
         raise ValueError("at most 8 leading dimensions are supported")
-    with _device_of(words):
-        _lib.call(
-            "myelin_packed_counts", _lib.ptr(words), len(lead), ctypes.addressof(lead_arr), mask, shape[-1],
-            _lib.ptr(out), _lib.stream(words.device),
-        )
-    return out
+    mask = 0
+    for d in dims:
+        if d != len(lead):
+            mask |= 1 << d
+    kept = tuple(s for i, s in enumerate(lead) if not (mask >> i) & 1)
+    words = packed.data.contiguous()
+    lead_arr = (ctypes.c_int64 * max(1, len(lead)))(*lead)
+
+    def call(name, *args):
+        with _device_of(words):
+            _lib.call(name, _lib.ptr(words), len(lead), ctypes.addressof(lead_arr), mask, shape[-1], *args,
+                      _lib.stream(words.device))
+
+    return kept, call
 
 
 def _counts_keep_last(packed: PackedSpikes, dims: tuple[int, ...]) -> torch.Tensor:
@@ -195,13 +206,24 @@ def packed_spike_rate(
 ) -> torch.Tensor:
     """``count(dim).to(dtype) / prod(reduced sizes)`` (packing.py:145-162)."""
 
-    counts = packed_spike_count(packed, dim=dim)
     nd = len(packed.original_shape)
     dims = tuple(range(nd)) if dim is None else _normalize_count_dims(dim, ndim=nd)
     denominator = 1
     for index in dims:
         denominator *= packed.original_shape[index]
-    if dtype not in (torch.float32, torch.float64):
+    rate_dtype = dtype in (torch.float32, torch.float64)
+    if nd - 1 in dims and rate_dtype:
+        # counted and divided in one launch where one workgroup has all of
+        # an output's words
+        _validate_packed_spikes(packed)
+        _lib.require_device(packed.data, "packed.data")
+        kept, call = _reduction(packed, dims)
+        counts = torch.empty(kept, dtype=torch.int64, device=packed.data.device)
+        out = torch.empty(kept, dtype=dtype, device=packed.data.device)
+        call("myelin_packed_rates", denominator, _lib.ptr(counts), _lib.ptr(out), _lib.DT[dtype])
+        return out
+    counts = packed_spike_count(packed, dim=dim)
+    if not rate_dtype:
         raise ValueError("packed_spike_rate supports dtype float32 or float64 on the HIP path")
     out = torch.empty(counts.shape, dtype=dtype, device=counts.device)
     with _device_of(counts):
