@@ -38,7 +38,8 @@ namespace {
 
 using myelin::kWave;
 
-typedef float f2 __attribute__((ext_vector_type(2)));
+// two neurons of a lane; rows of an odd length start on any dword
+typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 template <int V>
@@ -353,24 +354,32 @@ __global__ __launch_bounds__(256) void fwd_dense_generic(FwdArgs p) {
   if constexpr (ALIF) st<V>(p.a_final + base, a);
 }
 
-// U steps starting at t0, all inside [0, T): straight-line code.
-template <bool ALIF, int RULE, int V, int U>
-__device__ __forceinline__ void fwd_block(const FwdArgs &p, int64_t base, int64_t t0, const float (&cur)[U][V],
-                                          float (&m)[V], float (&a)[V]) {
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    float sp[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) sp[v] = neuron_step<ALIF, RULE>(m[v], a[v], cur[u][v], p);
-    st_stream<V>(p.spikes + (t0 + u) * p.BN + base, sp);
-  }
-}
-
 template <bool ALIF, int V>
 __device__ __forceinline__ void fwd_ckpt(const FwdArgs &p, int64_t base, int64_t k, const float (&m)[V],
                                          const float (&a)[V]) {
   st<V>(p.ckpt_m + k * p.BN + base, m);
   if constexpr (ALIF) st<V>(p.ckpt_a + k * p.BN + base, a);
+}
+
+// checkpoints fall on multiples of this many steps of a block of U: the
+// block's start, and in blocks of 32 every 16 steps as well
+constexpr int ckpt_grain(int U) { return U > 16 ? 16 : U; }
+
+// U steps starting at t0, all inside [0, T): straight-line code.
+template <bool ALIF, int RULE, int V, int U>
+__device__ __forceinline__ void fwd_block(const FwdArgs &p, int64_t base, int64_t t0, const float (&cur)[U][V],
+                                          float (&m)[V], float (&a)[V], bool ck, int64_t &next_ck, int64_t &k) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u % ckpt_grain(U) == 0 && ck && t0 + u == next_ck) {  // uniform
+      fwd_ckpt<ALIF, V>(p, base, k++, m, a);
+      next_ck += p.chunk;
+    }
+    float sp[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) sp[v] = neuron_step<ALIF, RULE>(m[v], a[v], cur[u][v], p);
+    st_stream<V>(p.spikes + (t0 + u) * p.BN + base, sp);
+  }
 }
 
 // The last T % U steps (rem, uniform) from registers loaded ahead: step
@@ -396,8 +405,10 @@ __device__ __forceinline__ void fwd_tail(const FwdArgs &p, int64_t base, int64_t
 }
 
 // Dense-spike forward, lane owns neurons [V*gid, V*gid + V) of the flat BN
-// axis.  Checkpoints (when requested) fall on block starts (chunk % U == 0,
-// checked by the host), so every full block of U steps is straight-line code:
+// axis; with two neurons a lane and an odd BN the last lane repeats the
+// neuron before its own.  Checkpoints (when requested) fall on multiples of
+// ckpt_grain(U) steps (checked by the host), so every full block of U steps
+// is straight-line code:
 // the compiler keeps the next block's U loads in flight across the current
 // block with exact vmcnt waits.  The last T % U steps are loaded in one batch
 // before the last full block runs, so they wait for one load latency rather
@@ -405,8 +416,9 @@ __device__ __forceinline__ void fwd_tail(const FwdArgs &p, int64_t base, int64_t
 template <bool ALIF, int RULE, int V, int U>
 __global__ __launch_bounds__(256) void fwd_dense(FwdArgs p) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t base = gid * V;
+  int64_t base = gid * V;
   if (base >= p.BN) return;
+  if (V == 2 && base + V > p.BN) base = p.BN - V;
   const int64_t T = p.T, BN = p.BN;
   const bool ck = p.ckpt_m != nullptr;
 
@@ -441,18 +453,10 @@ __global__ __launch_bounds__(256) void fwd_dense(FwdArgs p) {
         for (int v = 0; v < V; ++v) cur[u][v] = nxt[u][v];
 #pragma unroll
       for (int u = 0; u < U; ++u) ld_stream<V>(nxt[u], p.x + (t0 + U + u) * BN + base);
-      if (ck && t0 == next_ck) {
-        fwd_ckpt<ALIF, V>(p, base, k++, m, a);
-        next_ck += p.chunk;
-      }
-      fwd_block<ALIF, RULE, V, U>(p, base, t0, cur, m, a);
+      fwd_block<ALIF, RULE, V, U>(p, base, t0, cur, m, a, ck, next_ck, k);
     }
     load_tail();
-    if (ck && t0 == next_ck) {
-      fwd_ckpt<ALIF, V>(p, base, k++, m, a);
-      next_ck += p.chunk;
-    }
-    fwd_block<ALIF, RULE, V, U>(p, base, t0, nxt, m, a);
+    fwd_block<ALIF, RULE, V, U>(p, base, t0, nxt, m, a, ck, next_ck, k);
   } else {
     load_tail();
   }
@@ -462,9 +466,18 @@ __global__ __launch_bounds__(256) void fwd_dense(FwdArgs p) {
 }
 
 // Packed-spike forward: lanes map to (b, word, bit) so that each half-wave
-// owns one output word; a wave ballot yields two words per step.  Neurons
-// past N in the last word of a row are inactive (their bits are 0).
-template <bool ALIF, int RULE, int U>
+// owns one output word; a wave ballot yields two words per step.  Lanes past
+// N in the last word of a row, or past the last row, run the chain of neuron
+// N - 1 or batch row B - 1 and their bits are 0, so loads and steps have no
+// lane test.  PAIR: the wave's two words are one aligned 8-byte store.
+//
+// Bound by the loads in flight: a step's load is 256 bytes a wave, so the
+// loop runs as fwd_dense's, full blocks of U steps as straight-line code with
+// the next block's loads outstanding, and the last T mod U steps loaded in
+// one batch before the last full block.  (Guarded blocks of 8 steps before:
+// LIF [200, 48, 3000] 61.2 -> 38.4 us, [256, 128, 4096] 170 -> 132 us, 3.3 ->
+// 4.2 TB/s.)
+template <bool ALIF, int RULE, int U, bool PAIR>
 __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t g = gid >> 5;  // global word index over [B, W]
@@ -472,61 +485,76 @@ __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
   const int64_t b = g / p.W;
   const int64_t n = (g - b * p.W) * 32 + bit;
   const bool active = (b < p.B) && (n < p.N);
-  const int64_t flat = b * p.N + n;
+  const int64_t flat = (b < p.B ? b : p.B - 1) * p.N + (n < p.N ? n : p.N - 1);
   const int64_t T = p.T, BN = p.BN;
   const int64_t words_per_step = p.B * p.W;
-  // rows of an even word count from an 8-byte aligned base: the wave's two
-  // words (g_wave is even) are one aligned 8-byte store
-  const bool pair = words_per_step % 2 == 0 && (reinterpret_cast<uintptr_t>(p.packed) & 7) == 0;
   const int lane = static_cast<int>(threadIdx.x & (kWave - 1));
   // the wave's first word; waves start at multiples of 64 lanes, i.e. even
   // words (wave-uniform: made a scalar)
   const int64_t g_v = (gid - lane) >> 5;
   const int64_t g_wave = static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g_v)))) |
                          (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g_v >> 32))) << 32);
+  if (g_wave >= words_per_step) return;  // uniform
+  const float *x = p.x + flat;
+  int32_t *row = p.packed + g_wave;
+  const bool ck = p.ckpt_m != nullptr;
+  int64_t next_ck = 0;
+  float *ck_m = p.ckpt_m + flat, *ck_a = p.ckpt_a + flat;
 
-  float m = active ? p.m0[flat] : 0.0f;
-  float a = (ALIF && active) ? p.a0[flat] : 0.0f;
-
-  float nxt[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) nxt[u] = (active && u < T) ? __builtin_nontemporal_load(p.x + u * BN + flat) : 0.0f;
-
-  int64_t cc = 0;
-  for (int64_t t0 = 0; t0 < T; t0 += U) {
-    float cur[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t t = t0 + U + u;
-      if (t < T && active) nxt[u] = __builtin_nontemporal_load(p.x + t * BN + flat);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t t = t0 + u;
-      if (t < T) {
-        if (p.ckpt_m != nullptr && cc == 0 && active) {
-          const int64_t k = t / p.chunk;
-          p.ckpt_m[k * BN + flat] = m;
-          if constexpr (ALIF) p.ckpt_a[k * BN + flat] = a;
-        }
-        cc = (cc + 1 == p.chunk) ? 0 : cc + 1;
-        bool s = false;
-        if (active) s = neuron_step<ALIF, RULE>(m, a, cur[u], p) != 0.0f;
-        const uint64_t bits = __ballot(s);
-        int32_t *row = p.packed + t * words_per_step;
-        if (pair) {
-          // the wave's two words as one 8-byte store, the same value from
-          // every lane: no lane-selected branch a step
-          if (g_wave < words_per_step) *reinterpret_cast<uint64_t *>(row + g_wave) = bits;
-        } else {
-          if (lane == 0 && g_wave < words_per_step) row[g_wave] = static_cast<int32_t>(bits & 0xffffffffu);
-          if (lane == 32 && g_wave + 1 < words_per_step) row[g_wave + 1] = static_cast<int32_t>(bits >> 32);
-        }
+  float m = p.m0[flat];
+  float a = ALIF ? p.a0[flat] : 0.0f;
+  auto step = [&](int64_t t, float xv) {
+    if (ck && t == next_ck) {  // uniform; a lane past B or N repeats its owner's store
+      *ck_m = m;
+      ck_m += BN;
+      if constexpr (ALIF) {
+        *ck_a = a;
+        ck_a += BN;
       }
+      next_ck += p.chunk;
     }
+    const bool s = neuron_step<ALIF, RULE>(m, a, xv, p) != 0.0f;
+    const uint64_t bits = __ballot(active && s);
+    if constexpr (PAIR) {
+      // the same value from every lane: no lane-selected branch a step
+      *reinterpret_cast<uint64_t *>(row) = bits;
+    } else {
+      if (lane == 0) row[0] = static_cast<int32_t>(bits & 0xffffffffu);
+      if (lane == 32 && g_wave + 1 < words_per_step) row[1] = static_cast<int32_t>(bits >> 32);
+    }
+    row += words_per_step;
+  };
+  const int64_t Tm = (T / U) * U;
+  const int rem = static_cast<int>(T - Tm);
+  float tl[U];
+  auto load_tail = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < rem) tl[u] = __builtin_nontemporal_load(x + (Tm + u) * BN);  // uniform
+  };
+  if (Tm > 0) {
+    float nxt[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nxt[u] = __builtin_nontemporal_load(x + u * BN);
+    int64_t t0 = 0;
+    for (; t0 + U < Tm; t0 += U) {
+      float cur[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+#pragma unroll
+      for (int u = 0; u < U; ++u) nxt[u] = __builtin_nontemporal_load(x + (t0 + U + u) * BN);
+#pragma unroll
+      for (int u = 0; u < U; ++u) step(t0 + u, cur[u]);
+    }
+    load_tail();
+#pragma unroll
+    for (int u = 0; u < U; ++u) step(t0 + u, nxt[u]);
+  } else {
+    load_tail();
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (u < rem) step(Tm + u, tl[u]);  // uniform
   if (active) {
     p.m_final[flat] = m;
     if constexpr (ALIF) p.a_final[flat] = a;
@@ -747,8 +775,9 @@ __device__ __forceinline__ void bwd_load_ckpt(const BwdArgs &p, int64_t k, int64
 template <bool ALIF, int C, int SID, int V, bool GS, int FR, bool RZ = false>
 __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t base = gid * V;
+  int64_t base = gid * V;
   if (base >= p.BN) return;
+  if (V == 2 && base + V > p.BN) base = p.BN - V;  // odd BN: the last lane repeats a neuron
   const int64_t T = p.T, BN = p.BN;
   const int64_t Kf = T / C;
   const int rem = static_cast<int>(T - Kf * C);
@@ -787,6 +816,29 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
     bwd_load_ckpt<ALIF, V>(p, k, base, m, a);
 #pragma unroll
     for (int j = 0; j < C; ++j) ld_stream<V>(xb[j], p.x + (k * C + j) * BN + base);
+    if constexpr (C == 16 && V == 1 && GS) {
+      // one neuron per lane (grids too small to fill the chip, bound by the
+      // loads in flight): all of chunk k - 1's loads, x and grad_spikes, are
+      // outstanding while chunk k is walked backwards
+#pragma unroll
+      for (int j = 0; j < C; ++j) ld_stream<V>(gsb[j], p.gs + (k * C + j) * BN + base);
+      for (; k > 0; --k) {
+        const int64_t t0 = k * C;
+        bwd_recompute<ALIF, C, SID, V, false, FR, RZ>(p, C, xb, m, a, pre, cv);
+        __builtin_amdgcn_sched_barrier(0);
+        bwd_load_ckpt<ALIF, V>(p, k - 1, base, m, a);
+        float gn[C][V];
+#pragma unroll
+        for (int j = 0; j < C; ++j) ld_stream<V>(xb[j], p.x + (t0 - C + j) * BN + base);
+#pragma unroll
+        for (int j = 0; j < C; ++j) ld_stream<V>(gn[j], p.gs + (t0 - C + j) * BN + base);
+        __builtin_amdgcn_sched_barrier(0);
+        bwd_reverse<ALIF, C, SID, V, GS, false, FR, RZ>(p, base, t0, C, gsb, pre, cv, gm, ga);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < C; ++j) gsb[j][0] = gn[j][0];
+      }
+    }
     for (; k > 0; --k) {
       const int64_t t0 = k * C;
       if constexpr (C == 16) {
@@ -840,7 +892,7 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (GS) {
+    if constexpr (GS && !(C == 16 && V == 1)) {
 #pragma unroll
       for (int j = 0; j < C; ++j) ld_stream<V>(gsb[j], p.gs + j * BN + base);
     }
@@ -857,6 +909,20 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
 
 int64_t blocks_for(int64_t lanes) { return (lanes + 255) / 256; }
 
+// Whether a recurrence over BN neurons takes one neuron per lane (with more
+// loads in flight) rather than two.  With up to about three waves per SIMD a
+// launch lasts as long as its fullest SIMD (65,536 lanes are one wave on
+// each of the 1,024), and a wave of two neurons a lane takes about 1.5 times
+// one of one: LIF forward / backward, T = 100, 65,536 neurons 10.1 / 16.2 us
+// at one against 14.4 / 20.4 at two; T = 150, 75,924 neurons (two waves on
+// some SIMDs at one) 28.0 / 38.1 against 22.8 / 33.1; T = 128, 196,608
+// neurons 36.6 / 52.9 against 39.7 / 54.5; 249,917 neurons 69 / 97 against
+// 50 / 75.
+bool one_per_lane(int64_t BN) {
+  const int64_t lanes = 1024 * 64, one = (BN + lanes - 1) / lanes, two = (BN + 2 * lanes - 1) / (2 * lanes);
+  return 2 * one <= 3 * two;
+}
+
 template <bool ALIF, int RULE>
 int launch_fwd(const FwdArgs &a, hipStream_t stream) {
   constexpr bool AG = rule_autograd(RULE);
@@ -865,26 +931,30 @@ int launch_fwd(const FwdArgs &a, hipStream_t stream) {
       return myelin::invalid("spike rule %d emits spike values; packed output takes the threshold rules", RULE);
     } else {
       const int64_t lanes = a.B * a.W * 32;
-      fwd_packed<ALIF, RULE, MYELIN_FWD_UNROLL><<<dim3(blocks_for(lanes)), dim3(256), 0, stream>>>(a);
+      const dim3 grid(blocks_for(lanes));
+      // an even word count a step from an 8-byte aligned base: a wave's words
+      // (it starts at an even one) are one aligned pair
+      const bool pair = a.B * a.W % 2 == 0 && myelin::aligned(a.packed, 8);
+      // under four waves per SIMD each wave keeps more steps in flight
+      if (lanes < 4 * 1024 * 64) {
+        if (pair)
+          fwd_packed<ALIF, RULE, 32, true><<<grid, dim3(256), 0, stream>>>(a);
+        else
+          fwd_packed<ALIF, RULE, 32, false><<<grid, dim3(256), 0, stream>>>(a);
+      } else if (pair) {
+        fwd_packed<ALIF, RULE, 16, true><<<grid, dim3(256), 0, stream>>>(a);
+      } else {
+        fwd_packed<ALIF, RULE, 16, false><<<grid, dim3(256), 0, stream>>>(a);
+      }
       return myelin::launched("fwd_packed");
     }
   }
-  // widest vector the pointers and BN allow (at most 2 neurons per lane for
-  // the autograd rules, which are built at 1 and 2)
-  const void *ptrs[] = {a.x, a.m0, a.m_final, a.spikes, a.ckpt_m, ALIF ? a.a0 : nullptr,
-                        ALIF ? a.a_final : nullptr, ALIF ? a.ckpt_a : nullptr};
-  int v = (AG && MYELIN_FWD_VEC > 2) ? 2 : MYELIN_FWD_VEC;
-  while (v > 1) {
-    bool ok = (a.BN % v) == 0;
-    for (const void *q : ptrs)
-      if (q != nullptr && !myelin::aligned(q, 4 * v)) ok = false;
-    if (ok) break;
-    v >>= 1;
-  }
-  // Small grids (under two waves per SIMD at this width) without
-  // checkpoints: one neuron per lane and 32 steps in flight, so a latency-
-  // bound walk over T has twice the lanes and four times the loads outstanding.
-  if (a.ckpt_m == nullptr && (a.BN + v - 1) / v < 2 * 1024 * 64) {
+  // two neurons per lane (their 8-byte accesses need dword alignment only);
+  // for an odd BN a lane repeats a neuron, so the output is not the input
+  const bool in_place = a.spikes == a.x || a.m_final == a.m0 || (ALIF && a.a_final == a.a0);
+  const int v = MYELIN_FWD_VEC == 2 && a.BN >= 2 && (a.BN % 2 == 0 || !in_place) ? 2 : 1;
+  // Few waves: one neuron per lane and 32 steps in flight
+  if (one_per_lane(a.BN) && (a.ckpt_m == nullptr || a.chunk % 16 == 0)) {
     fwd_dense<ALIF, RULE, 1, 4 * MYELIN_FWD_UNROLL><<<dim3(blocks_for(a.BN)), dim3(256), 0, stream>>>(a);
     return myelin::launched("fwd_dense");
   }
@@ -892,24 +962,19 @@ int launch_fwd(const FwdArgs &a, hipStream_t stream) {
   const dim3 grid(blocks_for(lanes));
   constexpr int U = MYELIN_FWD_UNROLL;
   if (a.ckpt_m != nullptr && a.chunk % U != 0) {
-    if constexpr (AG) {
-      fwd_dense_generic<ALIF, RULE, 1, U><<<dim3(blocks_for(a.BN)), dim3(256), 0, stream>>>(a);
-    } else {
-      if (v == 4)
-        fwd_dense_generic<ALIF, RULE, 4, U><<<grid, dim3(256), 0, stream>>>(a);
-      else if (v == 2)
+    if constexpr (!AG) {
+      if (v == 2 && a.BN % 2 == 0) {
         fwd_dense_generic<ALIF, RULE, 2, U><<<grid, dim3(256), 0, stream>>>(a);
-      else
-        fwd_dense_generic<ALIF, RULE, 1, U><<<grid, dim3(256), 0, stream>>>(a);
+        return myelin::launched("fwd_dense_generic");
+      }
     }
+    fwd_dense_generic<ALIF, RULE, 1, U><<<dim3(blocks_for(a.BN)), dim3(256), 0, stream>>>(a);
     return myelin::launched("fwd_dense_generic");
   }
   if (v == 2)
     fwd_dense<ALIF, RULE, 2, U><<<grid, dim3(256), 0, stream>>>(a);
-  else if (v == 1)
+  else
     fwd_dense<ALIF, RULE, 1, U><<<grid, dim3(256), 0, stream>>>(a);
-  else if constexpr (!AG)
-    fwd_dense<ALIF, RULE, 4, U><<<grid, dim3(256), 0, stream>>>(a);
   return myelin::launched("fwd_dense");
 }
 
@@ -954,15 +1019,13 @@ int fwd_entry(FwdArgs &a, int rule, hipStream_t stream) {
 // smooth rule's kernels are built at one neuron per lane only)
 template <bool ALIF, int C, int SID, int FR>
 int launch_bwd_sid(const BwdArgs &a, hipStream_t stream) {
-  const void *ptrs[] = {a.x, a.ckpt_m, a.gs, a.gmT, a.gx, a.gm0, a.ckpt_a, a.gaT, a.ga0};
-  int v = FR >= MYELIN_RULE_SMOOTH ? 1 : MYELIN_BWD_VEC;
-  while (v > 1) {
-    bool ok = (a.BN % v) == 0;
-    for (const void *q : ptrs)
-      if (q != nullptr && !myelin::aligned(q, 4 * v)) ok = false;
-    if (ok) break;
-    v >>= 1;
-  }
+  // two neurons per lane (dword alignment is enough); an odd BN repeats a
+  // neuron, so no output may be an input
+  const bool in_place = a.gx == a.x || a.gx == a.gs || (a.gmT != nullptr && a.gmT == a.gm0) ||
+                        (a.gaT != nullptr && a.gaT == a.ga0);
+  int v = FR < MYELIN_RULE_SMOOTH && MYELIN_BWD_VEC == 2 && a.BN >= 2 && (a.BN % 2 == 0 || !in_place) ? 2 : 1;
+  // few waves: one neuron per lane with a whole chunk's loads outstanding
+  if (C == 16 && one_per_lane(a.BN)) v = 1;
   const bool gs = (SID != MYELIN_SG_NONE) && a.gs != nullptr;
   // without a spike gradient the two-neuron chunk-16 kernel does not fit
   // the register file (about 460 registers); one neuron per lane needs < 80.
