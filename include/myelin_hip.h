@@ -431,41 +431,42 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
                         int64_t cols, int transpose, myelin_stream_t stream);
 
 /*
- * Exact fp32 synapse currents of small-integer inputs (spikes) on the int8
- * MFMA.  myelin_spike_limit(F) is the largest input magnitude the digit
- * products of an F-wide layer hold in 32 bits (0: F too wide).
+ * Exact fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
  *
- * myelin_cast_spikes: x [rows, F] fp32 -> xi [rows, Kp] int8, zeros past F
- * (Kp a multiple of 128, 16-byte aligned), and, unless xb is NULL, xb [rows,
- * F] bf16.  Sets flags[0] if some element is not bf16-exact (as
- * myelin_cast_bf16_checked) and flags[1] if some element is no integer of
- * magnitude <= myelin_spike_limit(F); never clears them.
+ * myelin_cast_spikes: x [rows, F] fp32 -> words [Kw / 4][rows][4]: words 4 s
+ * to 4 s + 3 of each row's Kw (bit i of word w the element 32 w + i, zeros
+ * past F) for stage s (Kw a multiple of 4, at most 2032; 16-byte aligned),
+ * and, unless xb is NULL, xb [rows, F] bf16.  Sets flags[0] if some element
+ * is not bf16-exact (as myelin_cast_bf16_checked) and flags[1] if some
+ * element is neither 0 nor 1; never clears them.
  *
  * myelin_weight_digits: w [F, N] fp32 -> per column n a power of two
  * scale[n] and w = scale[n] * (d3 2^24 + d2 2^16 + d1 2^8 + d0), balanced
  * base-256 digits, exact for weights down to 2^-6 of the column's largest
- * and within 2^-30 of that below; digits [ceil(N/32), 4 planes, 32, Kp]
- * int8, zeros past F and N.  Sets flags[1] if a column is not finite or its
+ * and within 2^-30 of that below; digits [ceil(N/32), Kp / 128, 4
+ * planes, 32, 128] int8, Kp a multiple of 128, zeros past F and N, each 128
+ * in the order of k that myelin_gemm_spikes reads.  Sets flags[1] if a column is not finite or its
  * largest magnitude is below 2^-96.
  *
- * myelin_gemm_spikes: C [M, N] = xi w (+ bias), every output the exact sum
- * of the digit products rounded once to fp32 (twice past 2^10 column
- * maxima), then scaled and biased: independent of order, tiles and rows.
- * Meaningful only where the two calls above left flags[1] clear.
+ * myelin_gemm_spikes: C [M, N] = bits w (+ bias) over M rows of words
+ * [Kp / 128][x_rows][4] (from row r of a cast on: words + 4 r, x_rows the
+ * cast's rows), every output the exact sum of the digit products rounded once to fp32
+ * (twice past 2^10 column maxima), then scaled and biased: independent of
+ * order, tiles and rows.  Meaningful only where the two calls above left
+ * flags[1] clear.
  * Replaces: as myelin_gemm_f32 (the fp32 synapse GEMMs when the layer input
  *   is spikes).
  */
-int64_t myelin_spike_limit(int64_t F);
-int myelin_cast_spikes(const float *x, int8_t *xi, uint16_t *xb, int64_t rows,
-                       int64_t F, int64_t Kp, int *flags,
+int myelin_cast_spikes(const float *x, int32_t *words, uint16_t *xb,
+                       int64_t rows, int64_t F, int64_t Kw, int *flags,
                        myelin_stream_t stream);
 int myelin_weight_digits(const float *w, int8_t *digits, float *scale,
                          int64_t F, int64_t N, int64_t Kp, int *flags,
                          myelin_stream_t stream);
-int myelin_gemm_spikes(const int8_t *xi, const int8_t *digits,
-                       const float *scale, const float *bias, float *C,
-                       int64_t M, int64_t N, int64_t Kp, int64_t ldc,
-                       myelin_stream_t stream);
+int myelin_gemm_spikes(const int32_t *words, int64_t x_rows,
+                       const int8_t *digits, const float *scale,
+                       const float *bias, float *C, int64_t M, int64_t N,
+                       int64_t Kp, int64_t ldc, myelin_stream_t stream);
 
 /*
  * Reverse recurrence over C steps of a saved pre-reset trace [C, BN]:

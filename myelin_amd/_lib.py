@@ -68,7 +68,7 @@ SIGNATURES: dict[str, list] = {
     "myelin_cast_bf16_checked": [_P, _P, _I64, _P, _P],
     "myelin_cast_spikes": [_P] * 3 + [_I64] * 3 + [_P] * 2,
     "myelin_weight_digits": [_P] * 3 + [_I64] * 3 + [_P] * 2,
-    "myelin_gemm_spikes": [_P] * 5 + [_I64] * 4 + [_P],
+    "myelin_gemm_spikes": [_P, _I64] + [_P] * 4 + [_I64] * 4 + [_P],
     "myelin_split_bf16x3": [_P, _P, _I64, _I64, _INT, _P],
     "myelin_gemm_parts": [_P, _P, _INT, _I64, _P, _P] + [_I64] * 6 + [_INT] * 3 + [_P, _I64, _P],
     "myelin_gemm_parts_col_sum": [_P, _P, _INT, _I64, _P, _P] + [_I64] * 6 + [_INT] * 3 + [_P, _I64, _P, _P, _I64,
@@ -112,8 +112,6 @@ def load() -> ctypes.CDLL:
             lib.myelin_gemm_workspace_elems.restype = ctypes.c_int64
             lib.myelin_narrow_bits_fits.argtypes = [_I64, _I64, _INT]
             lib.myelin_narrow_bits_fits.restype = ctypes.c_int
-            lib.myelin_spike_limit.argtypes = [_I64]
-            lib.myelin_spike_limit.restype = ctypes.c_int64
             for name, argtypes in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.argtypes = argtypes

@@ -1,21 +1,19 @@
-// Exact fp32 synapse currents of integer-valued inputs (spikes) on the int8
-// MFMA.
+// Exact fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
 //
 // An fp32 weight column is written as a 31-bit fixed-point number against
 // its own largest magnitude: w = scale * q, |q| <= 2^30, scale a power of
 // two, and q as four balanced base-256 digits q = d3 2^24 + d2 2^16 + d1 2^8
 // + d0.  Weights down to 2^-6 of their column's largest keep every bit of
 // their fp32 value, and smaller ones are off by at most 2^-30 of it.  With
-// inputs that are small integers, each digit plane's product is an integer
-// sum without rounding; the planes are joined and rounded once per output.
-// So an output does not depend on the order, the tiles or the rows it is
-// computed with, and lies within about half an ulp of the exact sum
-// (measured on 8192 x 4096 currents of 1024 inputs at 5 % activity: 3.0e-8
-// of the largest from float64; the three-plane bf16 split 6.8e-8, an fp32
-// GEMM 5e-7).
+// 0/1 inputs each digit plane's product is an integer sum without rounding;
+// the planes are joined and rounded once per output.  So an output does not
+// depend on the order, the tiles or the rows it is computed with, and lies
+// within about half an ulp of the exact sum (8192 x 4096 currents of 1024
+// inputs at 10 % activity: 3.6e-8 of their 2-norm from float64, an fp32 GEMM
+// 1.9e-7).
 //
-// Cost: four int8 planes at twice the bf16 rate against three bf16 planes:
-// 2/3 of the matrix time, half the input bytes.
+// Cost: four int8 planes at twice the bf16 rate against three bf16 planes,
+// 2/3 of the matrix time, with one bit per input instead of two bytes.
 
 #include "common.h"
 
@@ -27,7 +25,8 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kPlanes = 4;   // base-256 digits per weight
-constexpr int kStage = 128;  // k per LDS stage (bytes of a row)
+constexpr int kStage = 128;  // k per LDS stage (bytes of a digit row)
+constexpr int64_t kMaxK = 508 * 128;  // 128 K 257 < 2^31: two digit sums joined stay in 32 bits
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -44,31 +43,34 @@ __device__ __forceinline__ bool bf16_exact(float v) {
 
 struct CastArgs {
   const float *x;
-  int8_t *xi;
+  uint32_t *words;
   uint16_t *xb;
   int *flags;
   int64_t rows;
-  int F, Kp, lim;
+  int F, Kw;
 };
 
-// x [rows, F] fp32 -> xi [rows, Kp] int8 (zeros past F) and, if xb is given,
-// xb [rows, F] bf16.  flags[0] is set where a value is not bf16-exact,
-// flags[1] where one is no integer of magnitude <= lim; neither is cleared.
+// x [rows, F] fp32 -> words [Kw / 4][rows][4], bit i of word w of a row
+// (stage w / 4) the element 32 w + i, zeros past F, and if xb is given xb
+// [rows, F] bf16.  flags[0] is set where a value is not bf16-exact, flags[1] where one
+// is neither 0 nor 1; neither is cleared.
 // Bound by memory: each lane takes groups of four elements of a row, lane
-// after lane, so every load and store instruction of a wave is contiguous.
+// after lane, so every load and store instruction of a wave is contiguous;
+// eight lanes' four bits are joined to a word by lane exchanges.
 template <bool VEC>
 __global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
   constexpr int U = 4;  // groups per lane
-  const uint32_t per = static_cast<uint32_t>(p.Kp) / 4;
+  const uint32_t per = static_cast<uint32_t>(p.Kw) * 8;
   const int64_t total = p.rows * per;
   const int64_t g0 = static_cast<int64_t>(blockIdx.x) * (256 * U) + threadIdx.x;
+  const int lane = threadIdx.x & 63;
   float v[U][4];
   int64_t row[U];
   int col[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t g = g0 + u * 256;
-    row[u] = g / per;
+    row[u] = total <= 0x7fffffff ? static_cast<int64_t>(static_cast<uint32_t>(g) / per) : g / per;
     col[u] = static_cast<int>(g - row[u] * per) * 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[u][e] = 0.0f;
@@ -85,24 +87,25 @@ __global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
       }
     }
   }
-  bool inexact = false, wide = false;
-  const float lim = static_cast<float>(p.lim);
+  bool inexact = false, other = false;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (g0 + u * 256 >= total) continue;
-    uint32_t q = 0;
+    const bool in = g0 + u * 256 < total;  // the same for a word's eight lanes
+    uint32_t bits = 0;
     uint16_t h[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float f = v[u][e], r = __builtin_rintf(f);
+      const float f = v[u][e];
       inexact = inexact || !bf16_exact(f);
-      const bool ok = r == f && __builtin_fabsf(f) <= lim;  // false for NaN
-      wide = wide || !ok;
-      q |= static_cast<uint32_t>(static_cast<uint8_t>(ok ? static_cast<int>(r) : 0)) << (8 * e);
+      other = other || !(f == 0.0f || f == 1.0f);
+      bits |= (f != 0.0f ? 1u : 0u) << e;
       h[e] = to_bf16(f);
     }
-    *reinterpret_cast<uint32_t *>(p.xi + row[u] * p.Kp + col[u]) = q;
-    if (p.xb != nullptr && col[u] < p.F) {
+    bits <<= 4 * (lane & 7);
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), d));
+    if (in && (lane & 7) == 0) p.words[((col[u] / 128) * p.rows + row[u]) * 4 + (col[u] / 32 & 3)] = bits;
+    if (in && p.xb != nullptr && col[u] < p.F) {
       uint16_t *dst = p.xb + row[u] * p.F + col[u];
       if constexpr (VEC) {
         typedef uint16_t h4 __attribute__((ext_vector_type(4)));
@@ -114,15 +117,23 @@ __global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
       }
     }
   }
-  const bool any0 = __ballot(inexact) != 0, any1 = __ballot(wide) != 0;
-  if ((threadIdx.x & 63) == 0) {
+  const bool any0 = __ballot(inexact) != 0, any1 = __ballot(other) != 0;
+  if (lane == 0) {
     if (any0) p.flags[0] = 1;
     if (any1) p.flags[1] = 1;
   }
 }
 
-// w [F, N] -> digits [ceil(N / 32)][4 planes][32 neurons][Kp] int8 (zeros
-// past F and N) and scale [N].  flags[1] is set where a column holds a
+// The k of byte p (0..15) of 16-byte piece c of a 128-k stage of a digit row:
+// piece c is what lanes of half c & 1 multiply in k step c / 2, and their
+// input bits are byte-wise masks of one word (see bits_fragment).
+__device__ __forceinline__ int piece_k(int c, int p) {
+  return 64 * (c >> 2) + 32 * (c & 1) + 8 * (p & 3) + 4 * ((c >> 1) & 1) + (p >> 2);
+}
+
+// w [F, N] -> digits [ceil(N / 32)][Kp / 128][4 planes][32 neurons][128] int8
+// (zeros past F and N; the 128 k of a stage in the order of piece_k) and
+// scale [N].  flags[1] is set where a column holds a
 // non-finite value or its largest magnitude is outside [2^-96, 2^128).
 // A workgroup writes `chunk` k of 32 neurons: it first finds the columns'
 // maxima over all F (re-read from L2 by each of a column's workgroups: one
@@ -174,15 +185,15 @@ __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ 
       tile[c][r + 32 * u] = (in && f < F) ? static_cast<int>(__builtin_rintf(w[static_cast<int64_t>(f) * N + n] * up)) : 0;
     }
     __syncthreads();
-    // thread -> plane, neuron, 16 k
-    const int pl = threadIdx.x >> 8, nn = (threadIdx.x >> 3) & 31, kc = (threadIdx.x & 7) * 16;
+    // thread -> plane, neuron, piece of 16 k
+    const int pl = threadIdx.x >> 8, nn = (threadIdx.x >> 3) & 31, c16 = threadIdx.x & 7;
     uint32_t out[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint32_t word = 0;
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        int v = tile[nn][kc + 4 * i + b], d = 0;
+        int v = tile[nn][piece_k(c16, 4 * i + b)], d = 0;
         for (int s = 0; s <= pl; ++s) {  // balanced digit pl
           d = static_cast<int8_t>(v & 0xff);
           v = (v - d) >> 8;
@@ -192,55 +203,84 @@ __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ 
       out[i] = word;
     }
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<u4 *>(q + ((static_cast<int64_t>(blockIdx.x) * kPlanes + pl) * 32 + nn) * Kp + k0 + kc) =
+    *reinterpret_cast<u4 *>(q + static_cast<int64_t>(blockIdx.x) * 128 * Kp + static_cast<int64_t>(k0) * 128 +
+                            (pl * 32 + nn) * kStage + 16 * c16) =
         u4{out[0], out[1], out[2], out[3]};
     __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------------------
-// C[M, N] = (x digits) joined, scaled (+ bias).
+// C[M, N] = (bits x digits) joined, scaled (+ bias).
 //
 // The four digit planes of 32 neurons are 128 "virtual" columns that one
 // wave owns: its tile is 32 WM rows x 128 virtual columns, WM x 4 blocks of
 // 32 x 32 (v_mfma_i32_32x32x32_i8: a lane's fragment is 16 bytes of k, as in
-// the bf16 kernels), so an input fragment read from LDS feeds four MFMAs and
-// the planes of an output element end in the same lane and register index:
-// they are joined without a second accumulator set.  WGM x WGN waves share a
-// stage of 128 k of their rows and virtual columns, staged by direct global
-// -> LDS loads of 16 bytes (rows unpadded, 16-byte pieces swizzled as
-// position c ^ swz(row), two stages).
+// the bf16 kernels), so an input fragment feeds four MFMAs and the planes of
+// an output element end in the same lane and register index: they are joined
+// without a second accumulator set.  WGM x WGN waves share a stage of 128 k
+// of their rows and virtual columns, staged by direct global -> LDS loads of
+// 16 bytes (digit rows unpadded, 16-byte pieces at position c ^ swz(row); a
+// row's 128 input bits are one piece).
 //
-// Persistent: each workgroup walks tiles (one workgroup per CU on the large
-// tile), and the first stage of its next tile is loaded during the last
-// stage and the epilogue of this one; K is short here (1024 inputs are eight
-// stages), so a tile started cold would spend a third of its life filling
-// the pipe.
+// Measured at 8192 x 4096 x 1024 (MFMA time at peak 55 us), with parts
+// switched off: 75 us without loads and stores, 53 without MFMAs and stores,
+// and the stores about 30, which added up instead of overlapping.  What
+// helped:
+// - Two workgroups per CU (256 rows x 32 neurons each, four waves) instead of
+//   one of eight waves: one's stores and stage waits under the other's
+//   MFMAs, 160 -> 142 us.
+// - Inputs as bits, 20 KB a stage and workgroup, widened in registers: a lane
+//   of half h takes one word for two k steps, and dword j of its fragment in
+//   step s is (word >> (4 s + j)) & 0x01010101, two operations for four k;
+//   the digits are stored in that order of k.  With byte inputs the smaller
+//   tiles cost more (176 us) than they hid.
+// - Operands stored stage by stage, so that a tile's stage is contiguous: at
+//   a row pitch of 1,024 bytes a stage's pieces meet a quarter of the L2
+//   channels.  142 -> 137 us.
+// - No scheduling hints between MFMAs and LDS reads (with them 137, without
+//   132 us): the other workgroup fills the waits.
+//
+// Persistent: each workgroup walks tiles, and the first NS - 1 stages of its
+// next tile are loaded during the last stages of this one, before the
+// epilogue's stores: K is short here (1024 inputs are eight stages), and the
+// vector memory counter retires in order, so loads behind the stores would
+// wait for them.
 // ---------------------------------------------------------------------------
 struct SpikeArgs {
-  const int8_t *x;  // [M, Kp]
-  const int8_t *q;  // digits
+  const uint32_t *x;  // [Kp / 128][x_rows][4] words, M rows of each stage
+  const int8_t *q;    // digits
   const float *scale, *bias;
   float *C;
-  int64_t M, N, ldc;
+  int64_t M, N, ldc, x_rows;
   int Kp;
 };
 
-// position of 16-byte piece c of row r of a stage: c ^ swz(r).  A function of
-// r & 31, so the 32-row blocks of a wave share it, distinct over any 8
-// aligned rows and, with the row's bank half, over any 16: fragment reads
-// (32 rows of one piece per half-wave) meet no bank conflict
+// position of 16-byte piece c of digit row r of a stage: c ^ swz(r).  A
+// function of r & 31, so the 32-row blocks of a wave share it, distinct over
+// any 8 aligned rows and, with the row's bank half, over any 16: fragment
+// reads (32 rows of one piece per half-wave) meet no bank conflict
 __device__ __forceinline__ int swz(int r) { return (r ^ ((r >> 3) & 3)) & 7; }
 
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-template <int WM, int WGM, int WGN>
+// The fragment of k step s (0 or 1) of the two that a word covers.
+__device__ __forceinline__ i32x4 bits_fragment(uint32_t word, int s) {
+  i32x4 f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) f[j] = static_cast<int>((word >> (4 * s + j)) & 0x01010101u);
+  return f;
+}
+
+template <int WM, int WGM, int WGN, int NS>
 __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(2))) void spike_gemm(SpikeArgs g) {
   constexpr int NT = 64 * WGM * WGN;
   constexpr int BM = 32 * WM * WGM, BV = 128 * WGN;
-  constexpr int TILE = (BM + BV) * kStage;
-  constexpr int NPA = BM * 8 / NT, NPB = BV * 8 / NT;
-  __shared__ __attribute__((aligned(1024))) char lds[2 * TILE];
+  constexpr int TA = BM * 16, TILE = TA + BV * kStage;  // bytes of a stage's bits, of a stage
+  constexpr int NPB = BV * 8 / NT;                      // digit pieces per thread
+  constexpr int WA = BM / 64;                           // waves that load the bits, one piece a lane
+  static_assert(WA <= NT / 64, "one piece of bits per lane at most");
+  __shared__ __attribute__((aligned(1024))) char lds[NS * TILE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w / WGN, wn = w % WGN;
   const uint32_t tiles_m = static_cast<uint32_t>((g.M + BM - 1) / BM);
@@ -263,70 +303,65 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
     m0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(fst + in % gs)) * BM;
     n0 = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(in / gs)) * (32 * WGN);
   };
+  auto load16 = [](uint32_t off, const void *base, const char *dst_lds) {
+    const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void *)dst_lds));
+    uint32_t m0_saved;  // M0 (the LDS base of the load) is the compiler's
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+        : "=&s"(m0_saved)
+        : "v"(off), "s"(base), "s"(dst)
+        : "memory");
+  };
 
   // load side: pieces of the tile being loaded, as 32-bit offsets from a
   // uniform base; rows past the edge read the last row
-  uint32_t oa[NPA], ob[NPB];
-  const int8_t *ba = nullptr, *bb = nullptr;
+  uint32_t oa = 0, ob[NPB];
+  const char *ba = nullptr, *bb = nullptr;
   uint32_t lt = first + slot;
-  int ls = 0, lbuf = 0;
+  int ls = 0, lbuf = 0, ahead = 0;  // next stage to load, its buffer; stages loaded or in flight, not yet used
   auto point = [&]() {
     int64_t m0, n0;
     place(lt, m0, n0);
-    ba = g.x + m0 * g.Kp;
-    bb = g.q + n0 * kPlanes * g.Kp;
+    ba = reinterpret_cast<const char *>(g.x) + m0 * 16;
+    bb = reinterpret_cast<const char *>(g.q) + n0 * kPlanes * g.Kp;
     const int64_t lim_a = g.M - m0, lim_b = vrows - n0 * kPlanes;
-#pragma unroll
-    for (int e = 0; e < NPA; ++e) {
-      const int idx = e * NT + tid, row = idx >> 3;
-      const uint32_t rc = static_cast<uint32_t>(row < lim_a ? row : lim_a - 1);
-      oa[e] = rc * static_cast<uint32_t>(g.Kp) + 16 * ((idx & 7) ^ swz(row));
-    }
+    oa = static_cast<uint32_t>(tid < lim_a ? tid : lim_a - 1) * 16u;
 #pragma unroll
     for (int e = 0; e < NPB; ++e) {
       const int idx = e * NT + tid, row = idx >> 3;
-      const uint32_t rc = static_cast<uint32_t>(row < lim_b ? row : lim_b - 1);
-      ob[e] = rc * static_cast<uint32_t>(g.Kp) + 16 * ((idx & 7) ^ swz(row));
+      const uint32_t gi = row < lim_b ? static_cast<uint32_t>(row) >> 7 : 0u;
+      ob[e] = gi * 128u * static_cast<uint32_t>(g.Kp) + (static_cast<uint32_t>(row) & 127u) * kStage + 16 * ((idx & 7) ^ swz(row));
     }
   };
   auto issue = [&]() {
     if (lt >= last) return;  // uniform
     if (ls == 0) point();
-    char *tile = lds + lbuf * TILE;
-    const int8_t *pa = ba + ls * kStage, *pb = bb + ls * kStage;
+    const char *tile = lds + lbuf * TILE;
+    if (w < WA) load16(oa, ba + static_cast<int64_t>(ls) * g.x_rows * 16, tile + w * 1024);
 #pragma unroll
-    for (int e = 0; e < NPA + NPB; ++e) {
-      const int eo = e < NPA ? e : e - NPA;
-      const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-          (lds_void *)(tile + (e < NPA ? 0 : BM * kStage) + (eo * NT + w * 64) * 16)));
-      const uint32_t o = e < NPA ? oa[e] : ob[eo];
-      const int8_t *base = e < NPA ? pa : pb;
-      uint32_t m0_saved;  // M0 (the LDS base of the load) is the compiler's
-      asm volatile(
-          "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-          : "=&s"(m0_saved)
-          : "v"(o), "s"(base), "s"(dst)
-          : "memory");
-    }
-    lbuf ^= 1;
+    for (int e = 0; e < NPB; ++e) load16(ob[e], bb + ls * 128 * kStage, tile + TA + (e * NT + w * 64) * 16);
+    lbuf = lbuf == NS - 1 ? 0 : lbuf + 1;
+    ++ahead;
     if (++ls == nst) {
       ls = 0;
       lt += slots;
     }
   };
 
-  // fragment byte offsets in a stage; the 32-row blocks of a wave lie 32
-  // rows apart
-  int fa[4], fb[4];
+  // byte offsets in a stage: the lane's word of its row's four (the word of
+  // k steps 2, 3 lies 8 bytes on), and its digit fragments (32-row blocks lie
+  // 32 rows apart)
+  const int fa = (32 * WM * wm + (lane & 31)) * 16 + 4 * (lane >> 5);
+  int fb[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     const int c = 2 * ks + (lane >> 5), r = lane & 31;
-    fa[ks] = (32 * WM * wm + r) * kStage + ((c ^ swz(r)) << 4);
-    fb[ks] = (BM + 128 * wn + r) * kStage + ((c ^ swz(r)) << 4);
+    fb[ks] = TA + (128 * wn + r) * kStage + ((c ^ swz(r)) << 4);
   }
 
-  issue();
-  int buf = 0;
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i) issue();
+  int buf = 0, landed = 0;  // the stage's buffer; stages known to have landed
   for (uint32_t t = first + slot; t < last; t += slots) {
     i32x16 acc[WM][kPlanes];
 #pragma unroll
@@ -336,47 +371,57 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
     for (int s = 0; s < nst; ++s) {
-      // this stage's loads (and, of the first stage of a later tile, none:
-      // the epilogue before it has waited); the barrier makes every wave's
-      // pieces visible, and retires its LDS reads of the other buffer, which
-      // the loads issued after it overwrite
-      if (s > 0 || t == first + slot) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // this stage's loads: all but the NS - 2 later stages' in flight, or
+      // all at the end, or none where the epilogue before has waited.  The
+      // barrier makes every wave's pieces visible, and retires the LDS reads
+      // of the buffer that the loads issued after it overwrite.
+      if (landed > 0)
+        --landed;
+      else if (ahead < NS - 1)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      else if (w < WA)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NPB + 1) * (NS - 2)) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NPB * (NS - 2)) : "memory");
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       const char *cur = lds + buf * TILE;
-      i32x4 a[2][WM], b[2][kPlanes];
+      uint32_t bits[2][WM];
+      i32x4 b[2][kPlanes];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) bits[h][i] = *reinterpret_cast<const uint32_t *>(cur + fa + 512 * i + 8 * h);
       auto rd = [&](int ks, int set) {
 #pragma unroll
-        for (int i = 0; i < WM; ++i) a[set][i] = *reinterpret_cast<const i32x4 *>(cur + fa[ks] + 32 * kStage * i);
+        for (int j = 0; j < kPlanes; ++j)
+          b[set][j] = *reinterpret_cast<const i32x4 *>(cur + fb[ks] + 32 * kStage * j);
+      };
+      i32x4 a[2][WM];
+      auto widen = [&](int ks, int set) {
 #pragma unroll
-        for (int j = 0; j < kPlanes; ++j) b[set][j] = *reinterpret_cast<const i32x4 *>(cur + fb[ks] + 32 * kStage * j);
+        for (int i = 0; i < WM; ++i) a[set][i] = bits_fragment(bits[ks >> 1][i], ks & 1);
       };
       rd(0, 0);
+      --ahead;
       issue();
+      widen(0, 0);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        if (ks + 1 < 4) rd(ks + 1, (ks + 1) & 1);
+        if (ks + 1 < 4) {
+          rd(ks + 1, (ks + 1) & 1);
+          widen(ks + 1, (ks + 1) & 1);
+        }
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
           for (int j = 0; j < kPlanes; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[ks & 1][i], b[ks & 1][j], acc[i][j], 0, 0, 0);
-        if (ks + 1 < 4) {
-          // the next k step's fragment reads one after each MFMA: left to
-          // itself the scheduler issues them after the last
-          constexpr int NR = WM + kPlanes, NM = WM * kPlanes;
-#pragma unroll
-          for (int z = 0; z < (NR < NM ? NR : NM); ++z) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, NR > NM ? 2 : 1, 0);
-          }
-          if constexpr (NM > NR) __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
-        }
       }
-      buf ^= 1;
+      buf = buf == NS - 1 ? 0 : buf + 1;
     }
-    // the next tile's first stage has landed before this tile's stores are
-    // issued, so its first stage needs no wait behind them
+    // the next tile's first stages land before this tile's stores are issued
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    landed = ahead;
     int64_t m0, n0;
     place(t, m0, n0);
     const int64_t n = n0 + 32 * wn + (lane & 31);
@@ -390,8 +435,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
       for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          // hi 2^16 + lo, both exact in 32 bits (the host bounds K |x|);
-          // hi is exact in fp32 while the sum is under 2^10 column maxima
+          // hi 2^16 + lo, both exact in 32 bits; hi is exact in fp32 while
+          // the sum is under 2^10 column maxima
           const int lo = (acc[i][1][r] << 8) + acc[i][0][r];
           const int hi = (acc[i][3][r] << 8) + acc[i][2][r];
           float v = __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo)) * sc;
@@ -404,33 +449,26 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
-template <int WM, int WGM, int WGN>
+template <int WM, int WGM, int WGN, int NS>
 int launch_spike(const SpikeArgs &g, int per_cu, hipStream_t s) {
   const int64_t tiles = cdiv(g.M, 32 * WM * WGM) * cdiv(g.N, 32 * WGN);
   const int64_t wgs = tiles < 256 * per_cu ? tiles : 256 * per_cu;
-  spike_gemm<WM, WGM, WGN><<<dim3(static_cast<unsigned>(wgs)), dim3(64 * WGM * WGN), 0, s>>>(g);
+  spike_gemm<WM, WGM, WGN, NS><<<dim3(static_cast<unsigned>(wgs)), dim3(64 * WGM * WGN), 0, s>>>(g);
   return myelin::launched("gemm_spikes");
 }
 
 }  // namespace
 
-// the largest input magnitude whose joined digit sums stay in 32 bits:
-// K |x| 128 257 < 2^31
-extern "C" int64_t myelin_spike_limit(int64_t F) {
-  const int64_t kp = cdiv(F < 1 ? 1 : F, kStage) * kStage, lim = 65000 / kp;
-  return lim > 127 ? 127 : lim;
-}
-
-extern "C" int myelin_cast_spikes(const float *x, int8_t *xi, uint16_t *xb, int64_t rows, int64_t F, int64_t Kp,
+extern "C" int myelin_cast_spikes(const float *x, int32_t *words, uint16_t *xb, int64_t rows, int64_t F, int64_t Kw,
                                   int *flags, myelin_stream_t stream) {
   if (rows < 0 || F < 1) return myelin::invalid("cast_spikes: rows must be >= 0 and F >= 1");
-  if (Kp % kStage != 0 || Kp < F || Kp > 65000) return myelin::invalid("cast_spikes: bad row pitch");
+  if (F > kMaxK || Kw % 4 != 0 || Kw * 32 < F || Kw * 32 > kMaxK) return myelin::invalid("cast_spikes: bad row pitch");
   if (rows == 0) return MYELIN_OK;
-  if (x == nullptr || xi == nullptr || flags == nullptr) return myelin::invalid("cast_spikes: null pointer");
-  if (!myelin::aligned(xi, 16)) return myelin::invalid("cast_spikes: xi must be 16-byte aligned");
-  const int64_t blocks = cdiv(rows * (Kp / 4), 1024);
+  if (x == nullptr || words == nullptr || flags == nullptr) return myelin::invalid("cast_spikes: null pointer");
+  if (!myelin::aligned(words, 16)) return myelin::invalid("cast_spikes: words must be 16-byte aligned");
+  const int64_t blocks = cdiv(rows * Kw * 8, 1024);
   if (blocks > 0x7fffffff) return myelin::invalid("cast_spikes: too many elements");
-  const CastArgs a{x, xi, xb, flags, rows, static_cast<int>(F), static_cast<int>(Kp), static_cast<int>(myelin_spike_limit(F))};
+  const CastArgs a{x, reinterpret_cast<uint32_t *>(words), xb, flags, rows, static_cast<int>(F), static_cast<int>(Kw)};
   const dim3 grid(static_cast<unsigned>(blocks));
   if (F % 4 == 0 && myelin::aligned(x, 16) && (xb == nullptr || myelin::aligned(xb, 8)))
     cast_spikes<true><<<grid, dim3(256), 0, myelin::as_hip(stream)>>>(a);
@@ -442,7 +480,7 @@ extern "C" int myelin_cast_spikes(const float *x, int8_t *xi, uint16_t *xb, int6
 extern "C" int myelin_weight_digits(const float *w, int8_t *digits, float *scale, int64_t F, int64_t N, int64_t Kp,
                                     int *flags, myelin_stream_t stream) {
   if (F < 1 || N < 1) return myelin::invalid("weight_digits: F and N must be positive");
-  if (Kp % kStage != 0 || Kp < F || Kp > 65000) return myelin::invalid("weight_digits: bad row pitch");
+  if (Kp % kStage != 0 || Kp < F || Kp > kMaxK) return myelin::invalid("weight_digits: bad row pitch");
   if (w == nullptr || digits == nullptr || scale == nullptr || flags == nullptr)
     return myelin::invalid("weight_digits: null pointer");
   if (!myelin::aligned(digits, 16)) return myelin::invalid("weight_digits: digits must be 16-byte aligned");
@@ -458,22 +496,25 @@ extern "C" int myelin_weight_digits(const float *w, int8_t *digits, float *scale
   return myelin::launched("weight_digits");
 }
 
-extern "C" int myelin_gemm_spikes(const int8_t *xi, const int8_t *digits, const float *scale, const float *bias,
-                                  float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc, myelin_stream_t stream) {
+extern "C" int myelin_gemm_spikes(const int32_t *words, int64_t x_rows, const int8_t *digits, const float *scale,
+                                  const float *bias, float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc,
+                                  myelin_stream_t stream) {
   if (M < 0 || N < 0) return myelin::invalid("gemm_spikes: negative size");
-  if (Kp < kStage || Kp % kStage != 0 || Kp > 65000) return myelin::invalid("gemm_spikes: bad row pitch");
+  if (x_rows < M) return myelin::invalid("gemm_spikes: x_rows < M");
+  if (Kp < kStage || Kp % kStage != 0 || Kp > kMaxK) return myelin::invalid("gemm_spikes: bad row pitch");
   if (ldc < N) return myelin::invalid("gemm_spikes: ldc < N");
   if (M == 0 || N == 0) return MYELIN_OK;
-  if (xi == nullptr || digits == nullptr || scale == nullptr || C == nullptr)
+  if (words == nullptr || digits == nullptr || scale == nullptr || C == nullptr)
     return myelin::invalid("gemm_spikes: null pointer");
-  if (!myelin::aligned(xi, 16) || !myelin::aligned(digits, 16))
+  if (!myelin::aligned(words, 16) || !myelin::aligned(digits, 16))
     return myelin::invalid("gemm_spikes: operands must be 16-byte aligned");
   if (ldc >= (int64_t{1} << 27)) return myelin::invalid("gemm_spikes: rows too long");
   if (cdiv(M, 128) * cdiv(N, 32) > 0x7fffffff) return myelin::invalid("gemm_spikes: output too large");
-  const SpikeArgs g{xi, digits, scale, bias, C, M, N, ldc, static_cast<int>(Kp)};
+  const SpikeArgs g{reinterpret_cast<const uint32_t *>(words), digits, scale, bias, C, M, N, ldc, x_rows,
+                    static_cast<int>(Kp)};
   hipStream_t s = myelin::as_hip(stream);
-  // 256 rows x 64 neurons (eight waves, 128 KB of LDS, one workgroup per CU)
-  // where that fills the chip, else 128 x 32 (four waves, two per CU)
-  if (cdiv(M, 256) * cdiv(N, 64) >= 256) return launch_spike<2, 4, 2>(g, 1, s);
-  return launch_spike<1, 4, 1>(g, 2, s);
+  // 256 rows x 32 neurons, two workgroups per CU, where that fills the chip;
+  // else 128 rows (3200 x 256 x 784, 200 of them: 8.8 us)
+  if (cdiv(M, 256) * cdiv(N, 32) >= 512) return launch_spike<2, 4, 1, 3>(g, 2, s);
+  return launch_spike<1, 4, 1, 4>(g, 2, s);
 }

@@ -150,21 +150,26 @@ class _LazyBf16:
         return self._last[1]
 
 
-def _cast_spikes(x, pitch, flags, stream, bf16=True):
-    """(int8 copy of x ``[..., F]`` in rows of ``pitch`` bytes, its bf16 copy
-    or None); flags as myelin_cast_spikes."""
+# widest input of the int8 products: two digit sums joined stay in 32 bits
+_DIGITS_MAX_F = 508 * 128
 
-    F = x.shape[-1]
-    xi = torch.empty((*x.shape[:-1], pitch), dtype=torch.int8, device=x.device)
+
+def _cast_spikes(x, flags, stream, bf16=True):
+    """(bits of x ``[T, B, F]`` as int32 words ``[ceil(F / 128), T, B, 4]``,
+    its bf16 copy or None); flags as myelin_cast_spikes."""
+
+    T, B, F = x.shape
+    stages = -(-F // 128)
+    words = torch.empty((stages, T, B, 4), dtype=torch.int32, device=x.device)
     xb = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if bf16 else None
-    _lib.call("myelin_cast_spikes", _lib.ptr(x), _lib.ptr(xi), _lib.ptr(xb), x.numel() // F, F, pitch,
+    _lib.call("myelin_cast_spikes", _lib.ptr(x), _lib.ptr(words), _lib.ptr(xb), T * B, F, 4 * stages,
               _lib.ptr(flags), stream)
-    return xi, xb
+    return words, xb
 
 
 class _Digits:
     """An fp32 weight ``[F, N]`` as the four int8 digit planes and the column
-    scales myelin_gemm_spikes reads (the ``wt`` of an int8 input)."""
+    scales myelin_gemm_spikes reads (the ``wt`` of an input of words)."""
 
     def __init__(self, q: torch.Tensor, scale: torch.Tensor):
         self.q = q
@@ -174,7 +179,7 @@ class _Digits:
 class _Split:
     """The fp32 synapse on the int8 or the bf16 MFMA, exactly.
 
-    An input of small integers (spikes) times W runs as four int8 products
+    An input of zeros and ones (spikes) times W runs as four int8 products
     with the base-256 digits of W, summed without rounding and rounded once
     (``myelin_gemm_spikes``).  An input whose every value is a bf16 value
     runs as three bf16 products, ``x @ W = x @ W_hi + x @ W_mid + x @ W_lo``
@@ -182,8 +187,8 @@ class _Split:
     is exact and only the fp32 summation rounds.  Per multiply-add the first
     costs 2/3 of the second, and that a fifth of the fp32 engine.
 
-    Construction launches the checked copies of x (``xi`` int8 and ``xb``
-    bf16; without ``bf16`` only ``xi``), both forms of W and an asynchronous
+    Construction launches the checked copies of x (``words``, its bits, and
+    ``xb`` bf16; without ``bf16`` only the words), both forms of W and an asynchronous
     copy of the check's flags to pinned host memory; ``exact()`` and
     ``operands()`` wait for those flags, the bf16 planes of W being formed
     meanwhile.
@@ -198,7 +203,7 @@ class _Split:
         dev = x.device
         flags = torch.zeros(2, dtype=torch.int32, device=dev)
         self.x = x
-        self.xi = self.xb = self.digits = None
+        self.words = self.xb = self.digits = None
         if lean:
             # no whole bf16 copy: check x slice by slice into one scratch
             # buffer (the flag is only ever set), and cast per chunk later
@@ -209,13 +214,13 @@ class _Split:
                 part = x[t0:t0 + step]
                 _lib.call("myelin_cast_bf16_checked", _lib.ptr(part), _lib.ptr(scratch), part.numel(), _lib.ptr(flags),
                           stream)
-        elif ints and _lib.load().myelin_spike_limit(F) > 0:
-            pitch = -(-F // 128) * 128
-            self.xi, self.xb = _cast_spikes(x, pitch, flags, stream, bf16=bf16)
-            # a weight the digits cannot hold raises the int8 flag as well
-            q = torch.empty((-(-N // 32), 4, 32, pitch), dtype=torch.int8, device=dev)
+        elif ints and F <= _DIGITS_MAX_F:
+            self.words, self.xb = _cast_spikes(x, flags, stream, bf16=bf16)
+            # a weight the digits cannot hold raises the words' flag as well
+            kp = 128 * self.words.shape[0]
+            q = torch.empty((-(-N // 32), 128, kp), dtype=torch.int8, device=dev)
             self.digits = _Digits(q, torch.empty(N, dtype=torch.float32, device=dev))
-            _lib.call("myelin_weight_digits", _lib.ptr(w), _lib.ptr(q), _lib.ptr(self.digits.scale), F, N, pitch,
+            _lib.call("myelin_weight_digits", _lib.ptr(w), _lib.ptr(q), _lib.ptr(self.digits.scale), F, N, kp,
                       _lib.ptr(flags), stream)
         else:
             self.xb = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
@@ -241,18 +246,18 @@ class _Split:
 
     def operands(self):
         """(xs, wt, xg): the currents' operands on the engine that takes this
-        input -- int8 and digits, bf16 and planes, or the fp32 input and None
-        -- and what the weight gradient's GEMM reads (the bf16 copy if the
+        input -- words and digits, bf16 and planes, or the fp32 input and
+        None -- and what the weight gradient's GEMM reads (the bf16 copy if the
         input is exact in it, else x; None on digits without ``bf16``)."""
 
-        inexact, wide = self._answer()
+        inexact, other = self._answer()
         if inexact:
             return self.x, None, self.x
-        if self.digits is not None and not wide:
-            return self.xi, self.digits, self.xb
+        if self.digits is not None and not other:
+            return self.words, self.digits, self.xb
         if self.xb is None:
             flags = torch.empty(2, dtype=torch.int32, device=self.x.device)  # known to hold: not read
-            self.xb = _cast_spikes(self.x, self.xi.shape[-1], flags, _lib.stream(self.x.device))[1]
+            self.xb = _cast_spikes(self.x, flags, _lib.stream(self.x.device))[1]
         return self.xb, self.w3, self.xb
 
 
@@ -297,7 +302,7 @@ def _split_eligible(prec: int, T: int, B: int, F: int, N: int, ints: bool = True
     if prec != _lib.PREC["fp32"] or N <= 32 or F % 8 != 0 or N % 8 != 0 or T * B * F * N < _SPLIT_MIN_MACS:
         return False
     # the bf16 products alone: the shapes the fused kernel does not take
-    if _fused(B, N) and not (ints and _lib.load().myelin_spike_limit(F) > 0):
+    if _fused(B, N) and not (ints and F <= _DIGITS_MAX_F):
         return False
     return not torch.cuda.is_current_stream_capturing()
 
@@ -416,7 +421,8 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
 
     ``x`` is fp32 with ``w [F, N]`` fp32, or bf16 (bf16 synapse) with ``wt``,
     the bf16 transposed weight ``[N, F]``; or an exact split's operands: bf16
-    with ``wt`` its planes ``[3, N, F]``, or int8 with ``wt`` a _Digits.
+    with ``wt`` its planes ``[3, N, F]``, or words (see _cast_spikes) with
+    ``wt`` a _Digits.
     Fused (one launch, currents stay in LDS) when N >= 64 and the fused grid
     has >= 1024 workgroups, except on the exact split.
     Otherwise each workgroup would walk many chunks serially, so the steps
@@ -438,16 +444,11 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     on the one stream).
     """
 
-    if x_bits is not None:
-        T, B = x_bits.shape[:2]
-        F = w.shape[0]
-    else:
-        T, B, F = x.shape
     digits = wt if isinstance(wt, _Digits) else None
+    T, B = x_bits.shape[:2] if x_bits is not None else x.shape[1:3] if digits is not None else x.shape[:2]
+    F = w.shape[0]
     half = x_bits is None and digits is None and x.dtype == torch.bfloat16
     parts = half and wt.ndim == 3  # exact split: wt holds the planes [3, N, F]
-    if digits is not None:
-        F = w.shape[0]
     N = wt.shape[-2] if half else w.shape[1]
     if digits is None and not parts and _fused(B, N):
         if pre_from not in (None, t0):
@@ -509,8 +510,8 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
             _gemm(x_bits[c0:c1], w, cur, rows, N, F, x_bits.shape[2], N, N, False, False, False, prec, s, bias=b,
                   a_bits=True, split=not exact)
         elif digits is not None:
-            _lib.call("myelin_gemm_spikes", _lib.ptr(x[c0:c1]), _lib.ptr(digits.q), _lib.ptr(digits.scale),
-                      _lib.ptr(b), _lib.ptr(cur), rows, N, x.shape[2], N, s)
+            _lib.call("myelin_gemm_spikes", _lib.ptr(x[:, c0:c1]), T * B, _lib.ptr(digits.q),
+                      _lib.ptr(digits.scale), _lib.ptr(b), _lib.ptr(cur), rows, N, digits.q.shape[2], N, s)
         elif parts:
             _gemm_parts(x[c0:c1], wt, 3, N * F, cur, rows, N, F, F, F, N, False, True, False, s, bias=b,
                         split=not exact)
@@ -700,7 +701,7 @@ def linear_backward(xs, w, b, pre, ckpt, wt, g_m, g_out, decay, threshold, reset
     split's operand with its ``wt`` (see _lif_fwd); ``xg`` is what dW's GEMM
     reads where that is not ``xs``; ``g_out`` is dL/dspikes ``[T, B, N]`` or, with ``rate``, dL/drates ``[B, N]``."""
 
-    T, B = xs.shape[:2]
+    T, B = xs.shape[1:3] if isinstance(wt, _Digits) else xs.shape[:2]
     x_bits = xs if bits_f is not None else None
     F, N = w.shape
     BN = B * N

@@ -1,6 +1,6 @@
-"""Exact synapse currents of small-integer inputs on the int8 MFMA
-(myelin_cast_spikes, myelin_weight_digits, myelin_gemm_spikes) against
-float64, at the edges of its tiles, stages and digit ranges."""
+"""Exact synapse currents of spikes on the int8 MFMA (myelin_cast_spikes,
+myelin_weight_digits, myelin_gemm_spikes) against float64, at the edges of
+its tiles and stages and of the digits' range."""
 
 from __future__ import annotations
 
@@ -20,56 +20,59 @@ def _print_case(**kw):
 
 
 def _operands(x, w):
-    """(xi, xb, digits, scale, flags) of x [M, F] and w [F, N] on the GPU."""
+    """(words, xb, digits, scale, flags) of x [M, F] and w [F, N] on the GPU."""
 
     (M, F), N = x.shape, w.shape[1]
-    kp = -(-F // 128) * 128
+    stages = -(-F // 128)
+    kp = 128 * stages
     stream = _lib.stream(x.device)
-    xi = torch.full((M, kp), 77, dtype=torch.int8, device=DEV)
+    words = torch.full((stages, M, 4), 77, dtype=torch.int32, device=DEV)
     xb = torch.empty((M, F), dtype=torch.bfloat16, device=DEV)
     flags = torch.zeros(2, dtype=torch.int32, device=DEV)
-    q = torch.full((-(-N // 32), 4, 32, kp), 77, dtype=torch.int8, device=DEV)
+    q = torch.full((-(-N // 32), 128, kp), 77, dtype=torch.int8, device=DEV)
     scale = torch.empty(N, device=DEV)
-    _lib.call("myelin_cast_spikes", x.data_ptr(), xi.data_ptr(), xb.data_ptr(), M, F, kp, flags.data_ptr(), stream)
+    _lib.call("myelin_cast_spikes", x.data_ptr(), words.data_ptr(), xb.data_ptr(), M, F, 4 * stages, flags.data_ptr(),
+              stream)
     _lib.call("myelin_weight_digits", w.data_ptr(), q.data_ptr(), scale.data_ptr(), F, N, kp, flags.data_ptr(), stream)
-    return xi, xb, q, scale, flags
+    return words, xb, q, scale, flags
 
 
-def _product(xi, q, scale, bias, N):
-    out = torch.full((xi.shape[0], N), float("nan"), device=DEV)
-    _lib.call("myelin_gemm_spikes", xi.data_ptr(), q.data_ptr(), scale.data_ptr(), _lib.ptr(bias), out.data_ptr(),
-              xi.shape[0], N, xi.shape[1], N, _lib.stream(out.device))
+def _product(words, q, scale, bias, N):
+    out = torch.full((words.shape[1], N), float("nan"), device=DEV)
+    _lib.call("myelin_gemm_spikes", words.data_ptr(), words.stride(0) // 4, q.data_ptr(), scale.data_ptr(),
+              _lib.ptr(bias), out.data_ptr(), words.shape[1], N, q.shape[2], N, _lib.stream(out.device))
     return out
 
 
-# small tiles of 128 rows x 32 neurons, large ones of 256 x 64 from 256 of
-# them on (the last two); one stage of 128 inputs, remainders of each
+# tiles of 128 rows x 32 neurons, and of 256 rows from 512 of them on (the
+# last two); one stage of 128 inputs, remainders of each
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,F", [(1, 33, 1), (127, 64, 127), (128, 65, 128), (129, 96, 129), (300, 31, 1000),
                                    (20011, 300, 72), (65600, 40, 257)])
-@pytest.mark.parametrize("ints", [False, True])
-def test_digit_products_match_float64(M, N, F, ints):
-    _print_case(test="digits", M=M, N=N, F=F, ints=ints)
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_digit_products_match_float64(M, N, F, with_bias):
+    _print_case(test="digits", M=M, N=N, F=F, with_bias=with_bias)
     g = seeded(M + N + F)
-    lim = _lib.load().myelin_spike_limit(F)
-    x = torch.randint(-lim, lim + 1, (M, F), generator=g).float() if ints else (torch.rand(M, F, generator=g) < 0.1).float()
+    x = (torch.rand(M, F, generator=g) < (0.1 if with_bias else 0.9)).float()
     # columns of very different size, small weights beside large ones
     w = torch.randn(F, N, generator=g) * torch.exp2(torch.randint(-40, 40, (N,), generator=g).float())
     w = w * torch.exp2(-torch.randint(0, 12, (F, N), generator=g).float())
     w[:, N // 2] = 0.0
-    bias = torch.randn(N, generator=g) if ints else None
+    bias = torch.randn(N, generator=g) if with_bias else None
     xd, wd, bd = x.to(DEV), w.to(DEV), None if bias is None else bias.to(DEV)
-    xi, xb, q, scale, flags = _operands(xd, wd)
+    words, xb, q, scale, flags = _operands(xd, wd)
     assert flags.tolist() == [0, 0]
-    assert torch.equal(xb.float(), xd) and torch.equal(xi[:, :F].float(), xd)
-    assert F == xi.shape[1] or int(xi[:, F:].abs().max()) == 0
-    got = _product(xi, q, scale, bd, N)
+    packed = myelin.pack_spikes(xd).data
+    rows = words.permute(1, 0, 2).reshape(M, -1)
+    assert torch.equal(xb.float(), xd) and torch.equal(rows[:, :packed.shape[1]], packed)
+    assert not bool(rows[:, packed.shape[1]:].any())
+    got = _product(words, q, scale, bd, N)
     ref = xd.double() @ wd.double()
     # weights: rounded to multiples of 2^(e - 30), 2^(e - 1) <= column max <
     # 2^e, so each within 2^(e - 31) <= 2^-30 column max; the sum is rounded
     # at most twice to fp32 (2^-24 each), then the bias sum
     colmax = wd.double().abs().max(0).values
-    tol = ref.abs() * 2.0**-23 + xd.double().abs().sum(1, keepdim=True) * colmax * 2.0**-30
+    tol = ref.abs() * 2.0**-23 + xd.double().sum(1, keepdim=True) * colmax * 2.0**-30
     if bd is not None:
         ref = ref + bd.double()
         tol = tol + ref.abs() * 2.0**-24
@@ -77,19 +80,18 @@ def test_digit_products_match_float64(M, N, F, ints):
     assert bool((off <= tol).all()), f"largest error {float((off / tol.clamp_min(1e-300)).max()):.2f} of the bound"
     # a row does not depend on the rows computed with it
     r0 = M // 3
-    assert torch.equal(_product(xi[r0:r0 + 130].contiguous(), q, scale, bd, N), got[r0:r0 + 130])
+    assert torch.equal(_product(words[:, r0:r0 + 130], q, scale, bd, N), got[r0:r0 + 130])
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case,expect", [("spikes", [0, 0]), ("wide", [0, 1]), ("half", [0, 1]), ("real", [1, 1]),
+@pytest.mark.parametrize("case,expect", [("spikes", [0, 0]), ("two", [0, 1]), ("minus", [0, 1]), ("half", [0, 1]), ("real", [1, 1]),
                                          ("nan", [1, 1]), ("w_inf", [0, 1]), ("w_nan", [0, 1]), ("w_tiny", [0, 1])])
 def test_flags_say_what_the_digits_cannot_hold(case, expect):
     _print_case(test="digit_flags", case=case)
     g = seeded(5)
     x = (torch.rand(70, 300, generator=g) < 0.1).float()
     w = torch.randn(300, 40, generator=g)
-    lim = _lib.load().myelin_spike_limit(300)
-    x[69, 299] = {"wide": lim + 1.0, "half": 0.5, "real": 0.3, "nan": float("nan")}.get(case, 1.0)
+    x[69, 299] = {"two": 2.0, "minus": -1.0, "half": 0.5, "real": 0.3, "nan": float("nan")}.get(case, 1.0)
     if case == "w_tiny":
         w[:, 39] = 1e-35
     elif case.startswith("w_"):
@@ -134,13 +136,16 @@ def test_fused_shape_layer_takes_the_engine_its_input_allows(monkeypatch, value)
 
 def test_host_validation():
     with pytest.raises(ValueError, match="row pitch"):
-        _lib.call("myelin_cast_spikes", 16, 16, None, 4, 200, 200, 16, None)
+        _lib.call("myelin_cast_spikes", 16, 16, None, 4, 200, 6, 16, None)
     with pytest.raises(ValueError, match="null pointer"):
-        _lib.call("myelin_cast_spikes", 16, 16, None, 4, 200, 256, None, None)
+        _lib.call("myelin_cast_spikes", 16, 16, None, 4, 200, 8, None, None)
     with pytest.raises(ValueError, match="aligned"):
         _lib.call("myelin_weight_digits", 16, 8, 16, 200, 4, 256, 16, None)
-    with pytest.raises(ValueError, match="ldc"):
-        _lib.call("myelin_gemm_spikes", 16, 16, 16, None, 16, 4, 64, 128, 32, None)
     with pytest.raises(ValueError, match="row pitch"):
-        _lib.call("myelin_gemm_spikes", 16, 16, 16, None, 16, 4, 64, 64, 64, None)
-    assert _lib.load().myelin_spike_limit(64) == 127 and _lib.load().myelin_spike_limit(70000) == 0
+        _lib.call("myelin_weight_digits", 16, 16, 16, 70000, 4, 70016, 16, None)
+    with pytest.raises(ValueError, match="ldc"):
+        _lib.call("myelin_gemm_spikes", 16, 4, 16, 16, None, 16, 4, 64, 128, 32, None)
+    with pytest.raises(ValueError, match="row pitch"):
+        _lib.call("myelin_gemm_spikes", 16, 4, 16, 16, None, 16, 4, 64, 64, 64, None)
+    with pytest.raises(ValueError, match="x_rows"):
+        _lib.call("myelin_gemm_spikes", 16, 3, 16, 16, None, 16, 4, 64, 128, 64, None)
