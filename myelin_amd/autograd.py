@@ -14,10 +14,12 @@ re-reads ``x`` once to recompute each chunk.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Any
 
 import torch
+from torch.autograd import forward_ad
 
 from myelin_amd import _lib
 
@@ -27,6 +29,60 @@ from myelin_amd import _lib
 # chunk at a time so its registers stay near those of 8.  ALIF [256, 128,
 # 4096] fast_sigmoid: forward 190.5 -> 183.5 us, backward 270 -> 268 us.
 BWD_CHUNK = 16
+
+
+_native = None
+
+
+def native():
+    """The C++ form of the Functions below (csrc/autograd.cpp), bound to the
+    loaded library once."""
+
+    global _native
+    if _native is None:
+        try:
+            from myelin_amd import _autograd
+        except ImportError as e:
+            raise ImportError(f"myelin_amd/_autograd.so is not built or does not load ({e}); "
+                              "run `python -m myelin_amd.build`") from e
+        lib = _lib.load()
+        addr = [ctypes.cast(getattr(lib, n), ctypes.c_void_p).value
+                for n in ("myelin_lif_fwd_f32", "myelin_lif_bwd_f32", "myelin_alif_fwd_f32", "myelin_alif_bwd_f32",
+                          "myelin_last_error")]
+        _autograd.bind(*addr, _lib.MyelinHipError)
+        _native = _autograd
+    return _native
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain(*tensors: torch.Tensor) -> bool:
+    """The C++ Functions take these tensors: no subclass, no compiler or jit
+    tracing, function transform (vmap, grad, jvp) or forward-mode level, for
+    which the Python Functions' own rules and errors hold."""
+
+    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
+            and all(type(t) in _PLAIN for t in tensors))
+
+
+def lif(x, m0, decay, threshold, reset, slope, rule, sid):
+    """(final membrane, spikes) of HipLIFFunction."""
+
+    if plain(x, m0):
+        return native().lif(x, m0, decay, threshold, reset, slope, rule, sid, BWD_CHUNK)
+    with torch.cuda.device(x.device):
+        return HipLIFFunction.apply(x, m0, decay, threshold, reset, slope, rule, sid)
+
+
+def alif(x, m0, a0, decay, rho, threshold, beta, reset, slope, rule, sid):
+    """(final membrane, final adaptation, spikes) of HipALIFFunction."""
+
+    if plain(x, m0, a0):
+        return native().alif(x, m0, a0, decay, rho, threshold, beta, reset, slope, rule, sid, BWD_CHUNK)
+    with torch.cuda.device(x.device):
+        return HipALIFFunction.apply(x, m0, a0, decay, rho, threshold, beta, reset, slope, rule, sid)
 
 
 def _chunks(T: int) -> int:

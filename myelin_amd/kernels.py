@@ -20,8 +20,8 @@ from typing import Literal
 
 import torch
 
-from myelin_amd import _lib
-from myelin_amd.autograd import BWD_CHUNK, HipALIFFunction, HipLIFFunction
+from myelin_amd import _lib, autograd
+from myelin_amd.autograd import BWD_CHUNK
 from myelin_amd.checkpointing import CheckpointSize, resolve_checkpoint_size
 from myelin_amd.neurons import ALIFParams, ALIFState, LIFParams, LIFState
 from myelin_amd.packing import PackedSpikes, packed_last_dim_size
@@ -100,11 +100,8 @@ def lif_forward(
                   T, B, N, _f32(params.decay), _f32(params.threshold), _f32(params.reset), 0.0,
                   _lib.RULE_THRESHOLD, BWD_CHUNK, _lib.stream(x.device))
         return LIFState(membrane=m), spikes
-    with torch.cuda.device(inputs.device):
-        m, spikes = HipLIFFunction.apply(
-            x, m0, _f32(params.decay), _f32(params.threshold), _f32(params.reset),
-            0.0, _lib.RULE_THRESHOLD, _lib.SG_NONE,
-        )
+    m, spikes = autograd.lif(x, m0, _f32(params.decay), _f32(params.threshold), _f32(params.reset), 0.0,
+                             _lib.RULE_THRESHOLD, _lib.SG_NONE)
     return LIFState(membrane=m), spikes
 
 
@@ -171,12 +168,9 @@ def alif_forward(
                   _f32(params.threshold), _f32(params.beta), _f32(params.reset), 0.0, _lib.RULE_THRESHOLD,
                   BWD_CHUNK, _lib.stream(x.device))
         return ALIFState(membrane=m, adaptation=a), spikes
-    with torch.cuda.device(inputs.device):
-        m, a, spikes = HipALIFFunction.apply(
-            x, m0, a0, _f32(params.decay), _f32(params.adaptation_decay),
-            _f32(params.threshold), _f32(params.beta), _f32(params.reset), 0.0,
-            _lib.RULE_THRESHOLD, _lib.SG_NONE,
-        )
+    m, a, spikes = autograd.alif(x, m0, a0, _f32(params.decay), _f32(params.adaptation_decay),
+                                 _f32(params.threshold), _f32(params.beta), _f32(params.reset), 0.0,
+                                 _lib.RULE_THRESHOLD, _lib.SG_NONE)
     return ALIFState(membrane=m, adaptation=a), spikes
 
 
@@ -230,11 +224,8 @@ def surrogate_lif_forward(
     _check_inputs(inputs)
     m0 = _check_state(initial_state.membrane, inputs, "membrane")
     rule, code = _surrogate_codes(sid, hard_forward, backend == "torch" or not hard_forward)
-    with torch.cuda.device(inputs.device):
-        m, spikes = HipLIFFunction.apply(
-            inputs.contiguous(), m0, _f32(params.decay), _f32(params.threshold), _f32(params.reset),
-            _f32(surrogate_slope), rule, code,
-        )
+    m, spikes = autograd.lif(inputs.contiguous(), m0, _f32(params.decay), _f32(params.threshold),
+                             _f32(params.reset), _f32(surrogate_slope), rule, code)
     return LIFState(membrane=m), spikes
 
 
@@ -267,12 +258,9 @@ def surrogate_alif_forward(
     a0 = _check_state(initial_state.adaptation, inputs, "adaptation")
     autograd_order = backend in ("auto", "torch") or not hard_forward
     rule, code = _surrogate_codes(sid, hard_forward, autograd_order)
-    with torch.cuda.device(inputs.device):
-        m, a, spikes = HipALIFFunction.apply(
-            inputs.contiguous(), m0, a0, _f32(params.decay), _f32(params.adaptation_decay),
-            _f32(params.threshold), _f32(params.beta), _f32(params.reset), _f32(surrogate_slope),
-            rule, code,
-        )
+    m, a, spikes = autograd.alif(inputs.contiguous(), m0, a0, _f32(params.decay), _f32(params.adaptation_decay),
+                                 _f32(params.threshold), _f32(params.beta), _f32(params.reset),
+                                 _f32(surrogate_slope), rule, code)
     return ALIFState(membrane=m, adaptation=a), spikes
 
 
