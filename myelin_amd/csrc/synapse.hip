@@ -1363,14 +1363,20 @@ __device__ __forceinline__ void store_kvec(typename Prec<PREC>::T *dst, const fl
 // k-vectors.  S = uint16_t (bf16 bits, bf16 MFMA only): KC pieces are one
 // 16-byte load of 8 k copied as is; an MN thread loads a 4 x 8 block as
 // eight 8-byte rows and regroups the 16-bit halves into four 8-k vectors.
-// Alignment: fp32 rows 16 bytes (ld % 4 == 0); bf16 KC rows 16 bytes
-// (ld % 8 == 0), bf16 MN rows 8 bytes (ld % 4 == 0).  The per-piece
-// addresses are computed once.  fast() loads a whole KS-wide stage with no
+// Alignment: fp32 none beyond the element's (the 16-byte global loads take
+// any 4-byte address, so odd widths run at this engine's rate: 10179 x 963 x
+// 1024 271 -> 212 us against the 64 x 64 engine, its dX 386 -> 203, its dW
+// 297 -> 190); bf16 KC rows 16 bytes
+// (ld % 8 == 0), bf16 MN rows 8 bytes (ld % 4 == 0).  An fp32 MN block that
+// straddles the last column moves left to end there: it rewrites columns of
+// its neighbour with the same values.  The per-piece addresses are computed
+// once.  fast() loads a whole KS-wide stage with no
 // guards (rows / columns past the tile edge come from a clamped in-range
 // address); slow() guards every element and zero-fills (the partial last
 // stage).
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u4_any __attribute__((ext_vector_type(4), aligned(4)));  // four floats at any element
 
 template <int PREC, bool KC, typename S, int D, int ROWS = kBig, int NT = 256>
 struct BigLoader {
@@ -1414,6 +1420,7 @@ struct BigLoader {
       const int tt = tid % MNB;
       mn0_ = (tt % (ROWS / 4)) * 4;
       kk[0] = (tt / (ROWS / 4)) * (H ? 8 : KQ);
+      if (!H && mn_lim >= 4 && mn0_ < mn_lim && mn0_ + 3 >= mn_lim) mn0_ = static_cast<int>(mn_lim) - 4;
       ok[0] = mn0_ + 3 < mn_lim;
       const int64_t mc = ok[0] ? mn0_ : ((mn_lim - 4) & ~static_cast<int64_t>(3));
       q[0] = base + kk[0] * ld + mn0 + mc;
@@ -1435,7 +1442,7 @@ struct BigLoader {
         } else {
 #pragma unroll
           for (int h = 0; h < KQ; h += 4) {
-            const u4 t = *reinterpret_cast<const u4 *>(src + h);
+            const u4_any t = *reinterpret_cast<const u4_any *>(src + h);
             v[d][e * KQ + h] = t.x;
             v[d][e * KQ + h + 1] = t.y;
             v[d][e * KQ + h + 2] = t.z;
@@ -1455,7 +1462,7 @@ struct BigLoader {
       } else {
 #pragma unroll
         for (int j = 0; j < KQ; ++j) {
-          const u4 t = *reinterpret_cast<const u4 *>(src + j * ld);
+          const u4_any t = *reinterpret_cast<const u4_any *>(src + j * ld);
           v[d][4 * j] = t.x;
           v[d][4 * j + 1] = t.y;
           v[d][4 * j + 2] = t.z;
@@ -3411,23 +3418,60 @@ void launch_gemm_v(const GemmArgs &g, int ta, int tb, dim3 grid, hipStream_t s) 
 #define MYELIN_SPLIT_WANT 512  // tile GEMMs split K below this many output tiles
 #endif
 
+// k-steps of the busiest CU: rounds of 256 workgroups times the k of each,
+// with 64 more for a workgroup's first loads and its stores
+inline int64_t tile_rounds(int64_t workgroups, int64_t k) { return cdiv(workgroups, 256) * (k + 64); }
+
 // K splits for an output of `tiles` workgroups: split when the output alone
-// gives under `want` workgroups and K is long.
+// gives under `want` workgroups and K is long, into as many as reach `want`
+// or, for fp32 products, as stay within it, whichever has fewer k-steps (320
+// x 1856 x 5568, 45 tiles: 12 splits leave 28 workgroups for a third round,
+// 104 us, 11 none, 86; the bf16 products' counts are those their kernels
+// were measured with).
 template <int PREC>
 int64_t plan_splits(int64_t tiles, int64_t K, int64_t want) {
   constexpr int KS = Prec<PREC>::KS;
   if (tiles >= want || K < 8 * KS) return 1;
   int64_t splits = cdiv(want, tiles);
+  const int64_t under = want / tiles;
+  if (PREC == 0 && under < splits && tile_rounds(tiles * under, K / under) < tile_rounds(tiles * splits, K / splits)) splits = under;
   const int64_t max_by_k = K / (4 * KS);
   if (splits > max_by_k) splits = max_by_k;
   if (splits > 64) splits = 64;
   return splits < 1 ? 1 : splits;
 }
 
+// K splits an fp32-operand GEMM takes at `edge`-wide tiles, and the k of each
+template <int PREC>
+int64_t tile_splits(const GemmArgs &g, int64_t edge, int64_t ws_elems, int64_t &kchunk) {
+  constexpr int KS = Prec<PREC>::KS;
+  int64_t splits = g.ws != nullptr ? plan_splits<PREC>(cdiv(g.N, edge) * cdiv(g.M, edge), g.K, MYELIN_SPLIT_WANT) : 1;
+  while (splits > 1 && splits * g.M * g.N > ws_elems) --splits;
+  kchunk = cdiv(cdiv(g.K, splits), KS) * KS;
+  splits = cdiv(g.K, kchunk);
+  return splits < 1 ? 1 : splits;
+}
+
 // fp32 operands: the 128 x 128 kernel takes outputs of at least one full
-// tile per side whose operands allow 16-byte loads
-bool use_big(const GemmArgs &g) {
-  return g.M >= kBig && g.N >= kBig && al16(g.A) && al16(g.B) && g.lda % 4 == 0 && g.ldb % 4 == 0;
+// tile per side, unless the 64 x 64 one has its busiest CU done sooner: a
+// k-step of its tiles costs 3/8 (a quarter of the products, with twice the
+// LDS reads for each).  Split planes are written and read once more, 6500
+// elements in the time of one of 8 units of a k-step.  3200 x 256 x 784, 50
+// tiles or 200: 64.8 and 31.5 us; 12800 x 2048 x 784, 1600 tiles: 392 us on
+// 128 x 128.  Without a K split both sum in the same order: same bits.
+// A last tile of one to three rows of an operand that is contiguous along
+// them has no four to load at once: it would walk K element by element.
+template <int PREC>
+bool use_big(const GemmArgs &g, int ta, int tb, int64_t ws_elems) {
+  if (g.M < kBig || g.N < kBig) return false;
+  if ((ta && cdiv(g.M, kBig) * kBig - g.M > kBig - 4) || (!tb && cdiv(g.N, kBig) * kBig - g.N > kBig - 4)) return false;
+  if (PREC != 0) return true;
+  auto cost = [&](int64_t edge, int64_t unit) {
+    int64_t k;
+    const int64_t splits = tile_splits<PREC>(g, edge, ws_elems, k);
+    return tile_rounds(cdiv(g.M, edge) * cdiv(g.N, edge) * splits, k) * unit + (splits > 1 ? splits * g.M * g.N / 6500 : 0);
+  };
+  return cost(kBig, 8) <= cost(kTile, 3);
 }
 
 // bf16 operands (128 x 128 kernel only): k-contiguous rows 16-byte aligned,
@@ -3762,7 +3806,7 @@ int launch_gemm(GemmArgs g, int ta, int tb, bool half, int64_t ws_elems, hipStre
       launch_smallk<PREC, false>(g, ta, tb, grid, s);
     return myelin::launched("gemm (small K)");
   }
-  const bool big = !bits && (half || use_big(g));
+  const bool big = !bits && (half || use_big<PREC>(g, ta, tb, ws_elems));
   if constexpr (PREC == 1) {
     // the 256 x 256 mn-contiguous tiles pay only with a K split (their
     // grid is under one round of the chip): plan it first, and take the
@@ -3804,11 +3848,7 @@ int launch_gemm(GemmArgs g, int ta, int tb, bool half, int64_t ws_elems, hipStre
   const int64_t edge = big ? kBig : kTile;
   const int64_t tiles = cdiv(g.N, edge) * cdiv(g.M, edge);
   if (!big && cdiv(g.M, kTile) > 65535) return myelin::invalid("gemm: M too large (%lld)", (long long)g.M);
-  int64_t splits = g.ws != nullptr ? plan_splits<PREC>(tiles, g.K, MYELIN_SPLIT_WANT) : 1;
-  while (splits > 1 && splits * g.M * g.N > ws_elems) --splits;
-  g.kchunk = cdiv(cdiv(g.K, splits), KS) * KS;
-  splits = cdiv(g.K, g.kchunk);
-  if (splits < 1) splits = 1;
+  const int64_t splits = tile_splits<PREC>(g, edge, ws_elems, g.kchunk);
   g.splits = static_cast<int>(splits);
   if (big) {
     const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits));
