@@ -3429,12 +3429,12 @@ inline int64_t tile_rounds(int64_t workgroups, int64_t k) { return cdiv(workgrou
 // 104 us, 11 none, 86; the bf16 products' counts are those their kernels
 // were measured with).
 template <int PREC>
-int64_t plan_splits(int64_t tiles, int64_t K, int64_t want) {
+int64_t plan_splits(int64_t tiles, int64_t K, int64_t want, bool within = PREC == 0) {
   constexpr int KS = Prec<PREC>::KS;
   if (tiles >= want || K < 8 * KS) return 1;
   int64_t splits = cdiv(want, tiles);
   const int64_t under = want / tiles;
-  if (PREC == 0 && under < splits && tile_rounds(tiles * under, K / under) < tile_rounds(tiles * splits, K / splits)) splits = under;
+  if (within && under < splits && tile_rounds(tiles * under, K / under) < tile_rounds(tiles * splits, K / splits)) splits = under;
   const int64_t max_by_k = K / (4 * KS);
   if (splits > max_by_k) splits = max_by_k;
   if (splits > 64) splits = 64;
@@ -4001,7 +4001,7 @@ extern "C" int64_t myelin_gemm_workspace_elems(int64_t M, int64_t N, int64_t K, 
   int64_t most = N <= 32 ? narrow_splits(K) : 1;
   for (int64_t edge : {static_cast<int64_t>(kTile), static_cast<int64_t>(kBig)}) {
     const int64_t tiles = cdiv(M, edge) * cdiv(N, edge);
-    const int64_t s = precision == MYELIN_PREC_BF16 ? plan_splits<1>(tiles, K, MYELIN_SPLIT_WANT) : plan_splits<0>(tiles, K, MYELIN_SPLIT_WANT);
+    const int64_t s = precision == MYELIN_PREC_BF16 ? plan_splits<1>(tiles, K, MYELIN_SPLIT_WANT) : plan_splits<0>(tiles, K, MYELIN_SPLIT_WANT, false);
     if (s > most) most = s;
   }
   if (precision == MYELIN_PREC_BF16) {
