@@ -467,9 +467,11 @@ __global__ __launch_bounds__(256) void fwd_dense(FwdArgs p) {
 
 // Packed-spike forward: lanes map to (b, word, bit) so that each half-wave
 // owns one output word; a wave ballot yields two words per step.  Lanes past
-// N in the last word of a row, or past the last row, run the chain of neuron
-// N - 1 or batch row B - 1 and their bits are 0, so loads and steps have no
-// lane test.  PAIR: the wave's two words are one aligned 8-byte store.
+// N in the last word of a row run the chain of neuron N - 1, which is in
+// their half-wave, and their bits are 0, so loads and steps have no lane
+// test; half-waves past the last row leave at once (the rows' own lanes are
+// in other workgroups, whose m_final, where it is m0, they would read).
+// PAIR: the wave's two words are one aligned 8-byte store.
 //
 // Bound by the loads in flight: a step's load is 256 bytes a wave, so the
 // loop runs as fwd_dense's, full blocks of U steps as straight-line code with
@@ -484,8 +486,8 @@ __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
   const int bit = static_cast<int>(gid & 31);
   const int64_t b = g / p.W;
   const int64_t n = (g - b * p.W) * 32 + bit;
-  const bool active = (b < p.B) && (n < p.N);
-  const int64_t flat = (b < p.B ? b : p.B - 1) * p.N + (n < p.N ? n : p.N - 1);
+  const bool active = n < p.N;
+  const int64_t flat = b * p.N + (n < p.N ? n : p.N - 1);
   const int64_t T = p.T, BN = p.BN;
   const int64_t words_per_step = p.B * p.W;
   const int lane = static_cast<int>(threadIdx.x & (kWave - 1));
@@ -494,7 +496,7 @@ __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
   const int64_t g_v = (gid - lane) >> 5;
   const int64_t g_wave = static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g_v)))) |
                          (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g_v >> 32))) << 32);
-  if (g_wave >= words_per_step) return;  // uniform
+  if (b >= p.B) return;
   const float *x = p.x + flat;
   int32_t *row = p.packed + g_wave;
   const bool ck = p.ckpt_m != nullptr;
@@ -504,7 +506,7 @@ __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
   float m = p.m0[flat];
   float a = ALIF ? p.a0[flat] : 0.0f;
   auto step = [&](int64_t t, float xv) {
-    if (ck && t == next_ck) {  // uniform; a lane past B or N repeats its owner's store
+    if (ck && t == next_ck) {  // uniform; a lane past N repeats its owner's store
       *ck_m = m;
       ck_m += BN;
       if constexpr (ALIF) {
@@ -520,7 +522,7 @@ __global__ __launch_bounds__(256) void fwd_packed(FwdArgs p) {
       *reinterpret_cast<uint64_t *>(row) = bits;
     } else {
       if (lane == 0) row[0] = static_cast<int32_t>(bits & 0xffffffffu);
-      if (lane == 32 && g_wave + 1 < words_per_step) row[1] = static_cast<int32_t>(bits >> 32);
+      if (lane == 32) row[1] = static_cast<int32_t>(bits >> 32);
     }
     row += words_per_step;
   };

@@ -3296,7 +3296,7 @@ struct CurCursor {
 template <bool PRE, bool SPK, bool PK, int RULE, bool CK>
 __device__ __forceinline__ void cur_step(const CurArgs &p, int64_t t, float c, bool act, int64_t BN, int64_t gw,
                                          int lane, float &m, float &cnt, CurCursor &o) {
-  // (stores from every lane: a lane past B or N repeats its owner's)
+  // (stores from every lane: a lane past N repeats its owner's)
   if constexpr (CK) {
     if (t == o.next_ck) {
       *o.ck = m;
@@ -3322,10 +3322,10 @@ __device__ __forceinline__ void cur_step(const CurArgs &p, int64_t t, float c, b
     if (p.B * p.W % 2 == 0 && (reinterpret_cast<uintptr_t>(p.packed) & 7) == 0) {
       // the wave's two words as one 8-byte store, the same value from every
       // lane (gw is even and wave-uniform): no lane-selected branch a step
-      if (gw < p.B * p.W) *reinterpret_cast<uint64_t *>(o.pk + gw) = bits;
+      *reinterpret_cast<uint64_t *>(o.pk + gw) = bits;
     } else {
-      if (lane == 0 && gw < p.B * p.W) o.pk[gw] = static_cast<int32_t>(bits & 0xffffffffu);
-      if (lane == 32 && gw + 1 < p.B * p.W) o.pk[gw + 1] = static_cast<int32_t>(bits >> 32);
+      if (lane == 0) o.pk[gw] = static_cast<int32_t>(bits & 0xffffffffu);
+      if (lane == 32) o.pk[gw + 1] = static_cast<int32_t>(bits >> 32);
     }
     o.pk += p.B * p.W;
   }
@@ -3338,16 +3338,19 @@ __global__ __launch_bounds__(256) void lif_currents_fwd(CurArgs p) {
   const int bit = static_cast<int>(gid & 31);
   const int64_t b = g / p.W;
   const int64_t n = (g - b * p.W) * 32 + bit;
-  const bool act = (b < p.B) && (n < p.N);
-  // lanes past B or N run the chain of batch row B - 1 / neuron N - 1 and
-  // store the same values to the same addresses as the lane that owns it,
+  const bool act = n < p.N;
+  // lanes past N run the chain of neuron N - 1 and store the same values to
+  // the same addresses as the lane that owns it, which is in their half-wave,
   // so a step stores without a lane test
-  const int64_t flat = (b < p.B ? b : p.B - 1) * p.N + (n < p.N ? n : p.N - 1), BN = p.B * p.N;
+  const int64_t flat = b * p.N + (n < p.N ? n : p.N - 1), BN = p.B * p.N;
   const int lane = static_cast<int>(threadIdx.x & 63);
   // the wave's first packed word (wave-uniform: made a scalar)
   const int64_t gw_v = (gid - lane) >> 5;
   const int64_t gw = static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(gw_v)))) |
                      (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(gw_v >> 32))) << 32);
+  // half-waves past the last row leave here: the rows' own lanes are in other
+  // workgroups, and where m_final is m0 those may have written it already
+  if (b >= p.B) return;
   float m = p.m0 != nullptr ? p.m0[flat] : 0.0f;
   float cnt = p.counts != nullptr ? p.counts[flat] : 0.0f;
   // checkpoint rows are counted from ck_origin: row k holds the state before
