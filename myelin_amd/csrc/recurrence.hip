@@ -24,14 +24,8 @@
 
 #include "common.h"
 
-#ifndef MYELIN_FWD_VEC
-#define MYELIN_FWD_VEC 2
-#endif
 #ifndef MYELIN_FWD_UNROLL
 #define MYELIN_FWD_UNROLL 8
-#endif
-#ifndef MYELIN_BWD_VEC
-#define MYELIN_BWD_VEC 2
 #endif
 
 namespace {
@@ -774,7 +768,8 @@ __device__ __forceinline__ void bwd_load_ckpt(const BwdArgs &p, int64_t k, int64
 // full chunks then run as straight-line code, software-pipelined: the
 // checkpoint and x of chunk k-1 are loaded while chunk k is walked
 // backwards, and grad_spikes of chunk k while chunk k is recomputed.
-template <bool ALIF, int C, int SID, int V, bool GS, int FR, bool RZ = false>
+// AHEAD: all of a chunk's loads outstanding (one neuron per lane, chunk 16).
+template <bool ALIF, int C, int SID, int V, bool GS, int FR, bool RZ = false, bool AHEAD = false>
 __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   int64_t base = gid * V;
@@ -818,10 +813,12 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
     bwd_load_ckpt<ALIF, V>(p, k, base, m, a);
 #pragma unroll
     for (int j = 0; j < C; ++j) ld_stream<V>(xb[j], p.x + (k * C + j) * BN + base);
-    if constexpr (C == 16 && V == 1 && GS) {
-      // one neuron per lane (grids too small to fill the chip, bound by the
-      // loads in flight): all of chunk k - 1's loads, x and grad_spikes, are
-      // outstanding while chunk k is walked backwards
+    if constexpr (AHEAD) {
+      // one wave per SIMD, bound by the loads in flight: all of chunk k - 1's
+      // loads, x and grad_spikes, are outstanding while chunk k is walked
+      // backwards (LIF, T = 100, 32,768 neurons 14.2 -> 13.1 us; with two
+      // waves the registers cost more: 69,633 neurons, multi-Gaussian 29.0 ->
+      // 32.7)
 #pragma unroll
       for (int j = 0; j < C; ++j) ld_stream<V>(gsb[j], p.gs + (k * C + j) * BN + base);
       for (; k > 0; --k) {
@@ -894,7 +891,7 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (GS && !(C == 16 && V == 1)) {
+    if constexpr (GS && !AHEAD) {
 #pragma unroll
       for (int j = 0; j < C; ++j) ld_stream<V>(gsb[j], p.gs + j * BN + base);
     }
@@ -911,17 +908,58 @@ __global__ __launch_bounds__(256) void bwd_chunked(BwdArgs p) {
 
 int64_t blocks_for(int64_t lanes) { return (lanes + 255) / 256; }
 
-// Whether a recurrence over BN neurons takes one neuron per lane (with more
-// loads in flight) rather than two.  With up to about three waves per SIMD a
-// launch lasts as long as its fullest SIMD (65,536 lanes are one wave on
-// each of the 1,024), and a wave of two neurons a lane takes about 1.5 times
-// one of one: LIF forward / backward, T = 100, 65,536 neurons 10.1 / 16.2 us
-// at one against 14.4 / 20.4 at two; T = 150, 75,924 neurons (two waves on
-// some SIMDs at one) 28.0 / 38.1 against 22.8 / 33.1; T = 128, 196,608
-// neurons 36.6 / 52.9 against 39.7 / 54.5; 249,917 neurons 69 / 97 against
-// 50 / 75.
-bool one_per_lane(int64_t BN) {
-  const int64_t lanes = 1024 * 64, one = (BN + lanes - 1) / lanes, two = (BN + 2 * lanes - 1) / (2 * lanes);
+constexpr int64_t kWaveLanes = 1024 * 64;  // lanes of one wave on each of the 1,024 SIMDs
+
+// How much of a step is arithmetic.  kLight: the threshold and surrogate
+// rules, and derivatives of a few operations; kMedium: some 20 operations;
+// kBusy: an exponential as well; kHeavy: torch's atan evaluated in the
+// reference's order, tens of operations; kErf: its erf, hundreds.
+enum Work { kLight, kMedium, kBusy, kHeavy, kErf };
+
+// of an autograd rule's forward
+constexpr Work forward_work(int rule) {
+  if (!rule_autograd(rule)) return kLight;
+  return rule % 16 == MYELIN_SG_MULTI_GAUSSIAN ? kErf : rule % 16 == MYELIN_SG_ATAN ? kHeavy : kLight;
+}
+
+// of a backward with surrogate SID, in the autograd order where FR != 0
+constexpr Work backward_work(int sid, int fr) {
+  if (sid == MYELIN_SG_MULTI_GAUSSIAN) return fr != 0 ? kErf : kBusy;
+  if (sid == MYELIN_SG_SIGMOID) return fr != 0 ? kBusy : kMedium;
+  if (fr == 0 || sid == MYELIN_SG_TRIANGULAR) return kLight;
+  return sid == MYELIN_SG_ATAN ? kHeavy : kMedium;
+}
+
+// Whether a recurrence over BN neurons takes one neuron per lane rather than
+// two.  With up to about three waves per SIMD a launch lasts as long as its
+// fullest SIMD, and a wave of two neurons a lane takes about 1.5 times one of
+// one where loads bound it: LIF forward / closed-form backward, T = 100,
+// 65,536 neurons 10.1 / 16.2 us at one against 14.4 / 20.4 at two, 81,921
+// neurons (two waves on some SIMDs at one) 18.8 / 28 against 16.7 / 23,
+// 163,840 neurons forward 24.5 against 28.9, 249,917 neurons 52 / 75 against
+// 43 / 61.  The wave that a SIMD gets beside its only one counts once 1/32 of
+// the SIMDs have one: up to there it runs beside others (65,537 neurons at
+// one 12.4 / 18.4 against 15.6 / 21.4, 131,073 at two 22.1 / 32 against 28.7 /
+// 37).
+// Where arithmetic bounds it two neurons take twice as long as one, and one
+// stays the better while the two's grid has rounds to fill: backward of
+// kBusy up to three waves (multi-Gaussian, 98,305 neurons 32.2 against 36.5,
+// 180,225 55 against 57, 212,993 74 against 61), kHeavy up to seven (139,264
+// neurons 63 against 81, 458,752 141 against 157, 655,363 248 against 231;
+// forward 45 against 58, 104 against 110, 173 against 162), kErf at any size
+// (backward 177 against 352 at 65,536 neurons, 655,363 8 % less).
+// kMedium lies between: as kBusy where a wave's 256 bytes of a row are two
+// whole lines (sigmoid, 81,920 neurons 23 against 25, 163,840 38 against 44),
+// otherwise as kLight with the extra waves counting from 1/8 (T = 150, 75,924
+// neurons 39.6 against 36.0; 69,633 neurons, ALIF, autograd-order fast
+// sigmoid 27.0 against 28.6).
+bool one_per_lane(int64_t BN, Work work) {
+  if (work == kErf) return true;
+  if (work == kHeavy) return BN <= 7 * kWaveLanes;
+  if (work == kBusy || (work == kMedium && BN % 32 == 0)) return BN <= 3 * kWaveLanes;
+  const int64_t slack = kWaveLanes / (work == kLight ? 32 : 8);
+  if (BN <= kWaveLanes + slack) return true;
+  const int64_t one = (BN + kWaveLanes - 1) / kWaveLanes, two = (BN + 2 * (kWaveLanes - slack) - 1) / (2 * kWaveLanes);
   return 2 * one <= 3 * two;
 }
 
@@ -951,15 +989,20 @@ int launch_fwd(const FwdArgs &a, hipStream_t stream) {
       return myelin::launched("fwd_packed");
     }
   }
-  // two neurons per lane (their 8-byte accesses need dword alignment only);
-  // for an odd BN a lane repeats a neuron, so the output is not the input
-  const bool in_place = a.spikes == a.x || a.m_final == a.m0 || (ALIF && a.a_final == a.a0);
-  const int v = MYELIN_FWD_VEC == 2 && a.BN >= 2 && (a.BN % 2 == 0 || !in_place) ? 2 : 1;
-  // Few waves: one neuron per lane and 32 steps in flight
-  if (one_per_lane(a.BN) && (a.ckpt_m == nullptr || a.chunk % 16 == 0)) {
+  // One neuron per lane: 32 steps in flight, or 8 where arithmetic bounds the
+  // step and several waves share a SIMD (autograd-order atan, T = 100, 69,633
+  // neurons 33.8 -> 33.2 us, 262,145 76 -> 71; multi-Gaussian, 81,921 neurons
+  // 133 -> 120).
+  constexpr Work work = forward_work(RULE);
+  const bool one = one_per_lane(a.BN, work);
+  if (one && (work < kHeavy || a.BN <= kWaveLanes) && (a.ckpt_m == nullptr || a.chunk % 16 == 0)) {
     fwd_dense<ALIF, RULE, 1, 4 * MYELIN_FWD_UNROLL><<<dim3(blocks_for(a.BN)), dim3(256), 0, stream>>>(a);
     return myelin::launched("fwd_dense");
   }
+  // two neurons per lane (their 8-byte accesses need dword alignment only);
+  // for an odd BN a lane repeats a neuron, so the output is not the input
+  const bool in_place = a.spikes == a.x || a.m_final == a.m0 || (ALIF && a.a_final == a.a0);
+  const int v = a.BN >= 2 && (a.BN % 2 == 0 || !in_place) && !(one && work >= kHeavy) ? 2 : 1;
   const int64_t lanes = (a.BN + v - 1) / v;
   const dim3 grid(blocks_for(lanes));
   constexpr int U = MYELIN_FWD_UNROLL;
@@ -1025,9 +1068,13 @@ int launch_bwd_sid(const BwdArgs &a, hipStream_t stream) {
   // neuron, so no output may be an input
   const bool in_place = a.gx == a.x || a.gx == a.gs || (a.gmT != nullptr && a.gmT == a.gm0) ||
                         (a.gaT != nullptr && a.gaT == a.ga0);
-  int v = FR < MYELIN_RULE_SMOOTH && MYELIN_BWD_VEC == 2 && a.BN >= 2 && (a.BN % 2 == 0 || !in_place) ? 2 : 1;
-  // few waves: one neuron per lane with a whole chunk's loads outstanding
-  if (C == 16 && one_per_lane(a.BN)) v = 1;
+  int v = FR < MYELIN_RULE_SMOOTH && a.BN >= 2 && (a.BN % 2 == 0 || !in_place) ? 2 : 1;
+  // (ALIF's multi-Gaussian in the autograd order: two neurons take 1.8 times
+  // one's, 81,920 neurons 331 us against 363, 262,145 967 against 895)
+  constexpr Work work = backward_work(SID, FR);
+  const int64_t ones = (a.BN + kWaveLanes - 1) / kWaveLanes, twos = (ones + 1) / 2;
+  const bool one = ALIF && FR != 0 && SID == MYELIN_SG_MULTI_GAUSSIAN ? 4 * ones <= 7 * twos : one_per_lane(a.BN, work);
+  if (C == 16 && one) v = 1;
   const bool gs = (SID != MYELIN_SG_NONE) && a.gs != nullptr;
   // without a spike gradient the two-neuron chunk-16 kernel does not fit
   // the register file (about 460 registers); one neuron per lane needs < 80.
@@ -1055,8 +1102,12 @@ int launch_bwd_sid(const BwdArgs &a, hipStream_t stream) {
     }
   } else {
     if (gs) {
-      if constexpr (SID != MYELIN_SG_NONE)
-        bwd_chunked<ALIF, C, SID, 1, true, FR><<<grid, dim3(256), 0, stream>>>(a);
+      if constexpr (SID != MYELIN_SG_NONE) {
+        if (C == 16 && a.BN <= kWaveLanes)
+          bwd_chunked<ALIF, C, SID, 1, true, FR, false, C == 16><<<grid, dim3(256), 0, stream>>>(a);
+        else
+          bwd_chunked<ALIF, C, SID, 1, true, FR><<<grid, dim3(256), 0, stream>>>(a);
+      }
     } else {
       bwd_chunked<ALIF, C, SID, 1, false, FR><<<grid, dim3(256), 0, stream>>>(a);
     }
