@@ -3427,12 +3427,14 @@ inline int64_t tile_rounds(int64_t workgroups, int64_t k) { return cdiv(workgrou
 
 // K splits for an output of `tiles` workgroups: split when the output alone
 // gives under `want` workgroups and K is long, into as many as reach `want`
-// or, for fp32 products, as stay within it, whichever has fewer k-steps (320
-// x 1856 x 5568, 45 tiles: 12 splits leave 28 workgroups for a third round,
-// 104 us, 11 none, 86; the bf16 products' counts are those their kernels
-// were measured with).
+// or, for fp32 products on 128 x 128 tiles (`within`), as stay within it,
+// whichever has fewer k-steps (320 x 1856 x 5568, 45 tiles: 12 splits leave
+// 28 workgroups for a third round, 104 us, 11 none, 86).  64 x 64 tiles share
+// a CU, so fewer of them only leave it idle (1280 x 513 x 785: 3 splits 38
+// us, 2 splits 44); the bf16 products' counts are those their kernels were
+// measured with.
 template <int PREC>
-int64_t plan_splits(int64_t tiles, int64_t K, int64_t want, bool within = PREC == 0) {
+int64_t plan_splits(int64_t tiles, int64_t K, int64_t want, bool within = false) {
   constexpr int KS = Prec<PREC>::KS;
   if (tiles >= want || K < 8 * KS) return 1;
   int64_t splits = cdiv(want, tiles);
@@ -3448,7 +3450,8 @@ int64_t plan_splits(int64_t tiles, int64_t K, int64_t want, bool within = PREC =
 template <int PREC>
 int64_t tile_splits(const GemmArgs &g, int64_t edge, int64_t ws_elems, int64_t &kchunk) {
   constexpr int KS = Prec<PREC>::KS;
-  int64_t splits = g.ws != nullptr ? plan_splits<PREC>(cdiv(g.N, edge) * cdiv(g.M, edge), g.K, MYELIN_SPLIT_WANT) : 1;
+  int64_t splits = g.ws != nullptr ? plan_splits<PREC>(cdiv(g.N, edge) * cdiv(g.M, edge), g.K, MYELIN_SPLIT_WANT,
+                                                       PREC == 0 && edge == kBig) : 1;
   while (splits > 1 && splits * g.M * g.N > ws_elems) --splits;
   kchunk = cdiv(cdiv(g.K, splits), KS) * KS;
   splits = cdiv(g.K, kchunk);
@@ -3459,22 +3462,39 @@ int64_t tile_splits(const GemmArgs &g, int64_t edge, int64_t ws_elems, int64_t &
 // tile per side, unless the 64 x 64 one has its busiest CU done sooner: a
 // k-step of its tiles costs 3/8 (a quarter of the products, with twice the
 // LDS reads for each).  Split planes are written and read once more, 6500
-// elements in the time of one of 8 units of a k-step.  3200 x 256 x 784, 50
+// elements in the time of one of 8 units of a k-step.  Tiles of two operands
+// that are contiguous along m and n start 40 k-steps later (5120 x 201 x 333:
+// 29.0 us on 40 x 2 of them, 25.8 on 64 x 64 ones).  3200 x 256 x 784, 50
 // tiles or 200: 64.8 and 31.5 us; 12800 x 2048 x 784, 1600 tiles: 392 us on
 // 128 x 128.  Without a K split both sum in the same order: same bits.
+// On the bf16 MFMA operands with 16-byte rows take the 128 x 128 tiles, and
+// others where 64 x 64 ones would fill more than one round of the chip (two,
+// where K runs down the rows of A) with at least 128 k: 640 x 201 x 333, 40
+// of them, 16.2 us against 19.7 on 128 x 128, 1001 x 1001 x 300, 256 of them,
+// 12.1 against 18.9; 999 x 999 x 999, 512 with the splits, 41 against 28, 6400
+// x 701 x 1001 149 against 60.
 // A last tile of one to three rows of an operand that is contiguous along
-// them has no four to load at once: it would walk K element by element.
+// them has no four to load at once: it would walk K element by element.  It
+// does so only where the 64 x 64 grid cannot hold the rows.
 template <int PREC>
 bool use_big(const GemmArgs &g, int ta, int tb, int64_t ws_elems) {
   if (g.M < kBig || g.N < kBig) return false;
+  if (cdiv(g.M, kTile) > 65535) return true;
   if ((ta && cdiv(g.M, kBig) * kBig - g.M > kBig - 4) || (!tb && cdiv(g.N, kBig) * kBig - g.N > kBig - 4)) return false;
-  if (PREC != 0) return true;
-  auto cost = [&](int64_t edge, int64_t unit) {
+  if constexpr (PREC != 0) {
+    if (al16(g.A) && al16(g.B) && g.lda % 4 == 0 && g.ldb % 4 == 0) return true;
     int64_t k;
-    const int64_t splits = tile_splits<PREC>(g, edge, ws_elems, k);
-    return tile_rounds(cdiv(g.M, edge) * cdiv(g.N, edge) * splits, k) * unit + (splits > 1 ? splits * g.M * g.N / 6500 : 0);
-  };
-  return cost(kBig, 8) <= cost(kTile, 3);
+    const int64_t small = cdiv(g.M, kTile) * cdiv(g.N, kTile) * tile_splits<PREC>(g, kTile, ws_elems, k);
+    return g.K >= 128 && (ta ? small >= 512 : small > 256);
+  } else {
+    auto cost = [&](int64_t edge, int64_t unit, int64_t late) {
+      int64_t k;
+      const int64_t splits = tile_splits<PREC>(g, edge, ws_elems, k);
+      return tile_rounds(cdiv(g.M, edge) * cdiv(g.N, edge) * splits, k + late) * unit +
+             (splits > 1 ? splits * g.M * g.N / 6500 : 0);
+    };
+    return cost(kBig, 8, ta && !tb ? 40 : 0) <= cost(kTile, 3, 0);
+  }
 }
 
 // bf16 operands (128 x 128 kernel only): k-contiguous rows 16-byte aligned,
@@ -4004,7 +4024,7 @@ extern "C" int64_t myelin_gemm_workspace_elems(int64_t M, int64_t N, int64_t K, 
   int64_t most = N <= 32 ? narrow_splits(K) : 1;
   for (int64_t edge : {static_cast<int64_t>(kTile), static_cast<int64_t>(kBig)}) {
     const int64_t tiles = cdiv(M, edge) * cdiv(N, edge);
-    const int64_t s = precision == MYELIN_PREC_BF16 ? plan_splits<1>(tiles, K, MYELIN_SPLIT_WANT) : plan_splits<0>(tiles, K, MYELIN_SPLIT_WANT, false);
+    const int64_t s = precision == MYELIN_PREC_BF16 ? plan_splits<1>(tiles, K, MYELIN_SPLIT_WANT) : plan_splits<0>(tiles, K, MYELIN_SPLIT_WANT);
     if (s > most) most = s;
   }
   if (precision == MYELIN_PREC_BF16) {
