@@ -413,8 +413,9 @@ int myelin_cast_transpose_bf16(const float *x, uint16_t *xb, int64_t n,
 
 /*
  * myelin_cast_bf16 that also sets *inexact = 1 (never clears it) when some
- * element is not a bf16 value the MFMA multiplies exactly (its rounding
- * changes it, or it is a nonzero denormal).  No counterpart in the
+ * element is not a bf16 value that products with the planes of a split
+ * weight multiply exactly (its rounding changes it, it is a nonzero
+ * denormal, or infinite: a plane may be zero).  No counterpart in the
  * reference.
  */
 int myelin_cast_bf16_checked(const float *src, uint16_t *dst, int64_t n,

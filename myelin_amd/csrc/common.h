@@ -57,4 +57,13 @@ __device__ __forceinline__ float div_by(float x, float b, float y) {
   return __builtin_fmaf(e, y, q0);
 }
 
+// v is a bf16 value whose products with the three planes of a split weight
+// the MFMA forms exactly: its bf16 rounding returns it, and it is zero or
+// normal (denormals may be flushed) and finite (a plane may be zero).
+__device__ __forceinline__ bool bf16_exact(float v) {
+  const float a = __builtin_fabsf(v);
+  return static_cast<float>(static_cast<__bf16>(v)) == v &&
+         (a == 0.0f || (a >= 1.17549435e-38f && a < __builtin_huge_valf()));
+}
+
 }  // namespace myelin

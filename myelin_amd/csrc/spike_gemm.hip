@@ -35,12 +35,6 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 
-// v survives its bf16 rounding and is zero or normal
-__device__ __forceinline__ bool bf16_exact(float v) {
-  const float a = __builtin_fabsf(v);
-  return static_cast<float>(static_cast<__bf16>(v)) == v && (a == 0.0f || a >= 1.17549435e-38f);
-}
-
 struct CastArgs {
   const float *x;
   uint32_t *words;
@@ -96,7 +90,7 @@ __global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float f = v[u][e];
-      inexact = inexact || !bf16_exact(f);
+      inexact = inexact || !myelin::bf16_exact(f);
       other = other || !(f == 0.0f || f == 1.0f);
       bits |= (f != 0.0f ? 1u : 0u) << e;
       h[e] = to_bf16(f);

@@ -2967,13 +2967,6 @@ __global__ __launch_bounds__(acc_fwd::NT) __attribute__((amdgpu_waves_per_eu(2))
     }
 }
 
-// v is a bf16 value the MFMA multiplies exactly: its bf16 rounding returns
-// it, and it is zero or normal (denormals may be flushed)
-__device__ __forceinline__ bool bf16_exact(float v) {
-  const float a = __builtin_fabsf(v);
-  return static_cast<float>(static_cast<__bf16>(v)) == v && (a == 0.0f || a >= 1.17549435e-38f);
-}
-
 struct PreBwdArgs {
   const float *pre;     // [C, BN]
   const float *gs;      // [C, BN] or null
@@ -4801,14 +4794,14 @@ __global__ __launch_bounds__(256) void cast_bf16_checked(const float *__restrict
   if (i + 8 <= n) {
     const f4 a = *reinterpret_cast<const f4 *>(src + i);
     const f4 b = *reinterpret_cast<const f4 *>(src + i + 4);
-    bad = !(bf16_exact(a.x) && bf16_exact(a.y) && bf16_exact(a.z) && bf16_exact(a.w) && bf16_exact(b.x) &&
-            bf16_exact(b.y) && bf16_exact(b.z) && bf16_exact(b.w));
+    bad = !(myelin::bf16_exact(a.x) && myelin::bf16_exact(a.y) && myelin::bf16_exact(a.z) && myelin::bf16_exact(a.w) && myelin::bf16_exact(b.x) &&
+            myelin::bf16_exact(b.y) && myelin::bf16_exact(b.z) && myelin::bf16_exact(b.w));
     const u4 o{to_bf16(a.x) | (unsigned)to_bf16(a.y) << 16, to_bf16(a.z) | (unsigned)to_bf16(a.w) << 16,
                to_bf16(b.x) | (unsigned)to_bf16(b.y) << 16, to_bf16(b.z) | (unsigned)to_bf16(b.w) << 16};
     *reinterpret_cast<u4 *>(dst + i) = o;
   } else {
     for (int64_t j = i; j < n; ++j) {
-      bad = bad || !bf16_exact(src[j]);
+      bad = bad || !myelin::bf16_exact(src[j]);
       dst[j] = to_bf16(src[j]);
     }
   }
