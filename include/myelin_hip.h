@@ -432,7 +432,7 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
                         int64_t cols, int transpose, myelin_stream_t stream);
 
 /*
- * Exact fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
+ * fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
  *
  * myelin_cast_spikes: x [rows, F] fp32 -> words [Kw / 4][rows][4]: words 4 s
  * to 4 s + 3 of each row's Kw (bit i of word w the element 32 w + i, zeros
@@ -446,8 +446,10 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
  * base-256 digits, exact for weights down to 2^-6 of the column's largest
  * and within 2^-30 of that below; digits [ceil(N/32), Kp / 128, 4
  * planes, 32, 128] int8, Kp a multiple of 128, zeros past F and N, each 128
- * in the order of k that myelin_gemm_spikes reads.  Sets flags[1] if a column is not finite or its
- * largest magnitude is below 2^-96.
+ * in the order of k that myelin_gemm_spikes reads.  Sets flags[1] if a
+ * column is not finite, its largest magnitude is below 2^-96, or more than a
+ * few of its weights are so far below its largest that the digits hold them
+ * less well than an fp32 product would (the shares: csrc/spike_gemm.hip).
  *
  * myelin_gemm_spikes: C [M, N] = bits w (+ bias) over M rows of words
  * [Kp / 128][x_rows][4] (from row r of a cast on: words + 4 r, x_rows the

@@ -1,16 +1,17 @@
-// Exact fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
+// fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
 //
 // An fp32 weight column is written as a 31-bit fixed-point number against
 // its own largest magnitude: w = scale * q, |q| <= 2^30, scale a power of
 // two, and q as four balanced base-256 digits q = d3 2^24 + d2 2^16 + d1 2^8
 // + d0.  Weights down to 2^-6 of their column's largest keep every bit of
-// their fp32 value, and smaller ones are off by at most 2^-30 of it.  With
-// 0/1 inputs each digit plane's product is an integer sum without rounding;
-// the planes are joined and rounded once per output.  So an output does not
-// depend on the order, the tiles or the rows it is computed with, and lies
-// within about half an ulp of the exact sum (8192 x 4096 currents of 1024
-// inputs at 10 % activity: 3.6e-8 of their 2-norm from float64, an fp32 GEMM
-// 1.9e-7).
+// their fp32 value; smaller ones are off by at most 2^-30 of it, so columns
+// with more than a few much smaller ones are turned away (weight_digits).
+// With 0/1 inputs each digit plane's product is an integer sum without
+// rounding; the planes are joined and rounded once per output (twice past
+// 2^10 column maxima).  So an output does not depend on the order, the tiles
+// or the rows it is computed with, and lies within half an ulp of the digits'
+// sum (8192 x 4096 currents of 1024 inputs at 10 % activity: 3.6e-8 of their
+// 2-norm from float64, an fp32 GEMM 1.9e-7).
 //
 // Cost: four int8 planes at twice the bf16 rate against three bf16 planes,
 // 2/3 of the matrix time, with one bit per input instead of two bytes.
@@ -26,6 +27,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kPlanes = 4;   // base-256 digits per weight
 constexpr int kStage = 128;  // k per LDS stage (bytes of a digit row)
+constexpr int kSlack = 6;    // small weights a column may hold beyond their shares (see weight_digits)
 constexpr int64_t kMaxK = 508 * 128;  // 128 K 257 < 2^31: two digit sums joined stay in 32 bits
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -127,8 +129,20 @@ __device__ __forceinline__ int piece_k(int c, int p) {
 
 // w [F, N] -> digits [ceil(N / 32)][Kp / 128][4 planes][32 neurons][128] int8
 // (zeros past F and N; the 128 k of a stage in the order of piece_k) and
-// scale [N].  flags[1] is set where a column holds a
-// non-finite value or its largest magnitude is outside [2^-96, 2^128).
+// scale [N].  flags[1] is set where a column holds a non-finite value, its
+// largest magnitude is outside [2^-96, 2^128), or its weights span too wide a
+// range for one scale (below).
+//
+// The range: a weight below 2^-7 of 2^e (the power of two above its column's
+// largest) is rounded, by at most 2^-31 of 2^e.  An fp32 product's own error
+// is about 2^-24 of the sum of the magnitudes that spike, so the digits are as
+// good where most of those are above 2^-7 of 2^e -- whichever inputs spike,
+// and also where the largest weights' inputs are silent.  So of the weights
+// in a chunk of a column that the digits round, at most a quarter may be,
+// a 16th be below 2^-10 and a 256th below 2^-14 of 2^e (and kSlack more, as
+// chance has it: of 128 normal or Laplace weights 3 to 15, 1 to 2 and 0.1).
+// One weight 100 times the rest of its column raised the error of its currents
+// from 1.2e-7, fp32's, to 7.7e-7 without this, 10^6 times to 6e-3.
 // A workgroup writes `chunk` k of 32 neurons: it first finds the columns'
 // maxima over all F (re-read from L2 by each of a column's workgroups: one
 // launch instead of a reduction and a second pass), then turns tiles of 128
@@ -137,6 +151,7 @@ __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ 
                                                       float *__restrict__ scale, int *__restrict__ flags, int F, int N,
                                                       int Kp, int chunk) {
   __shared__ uint32_t red[32][33];
+  __shared__ uint64_t small[32][33];
   __shared__ int tile[32][kStage + 1];
   const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
   const int64_t n = static_cast<int64_t>(blockIdx.x) * 32 + c;
@@ -171,12 +186,21 @@ __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ 
     if (bad) flags[1] = 1;
   }
   const int k_begin = blockIdx.y * chunk, k_end = k_begin + chunk < Kp ? k_begin + chunk : Kp;
+  uint64_t count = 0;  // of the column's weights in this chunk: three sums of 21 bits
   for (int k0 = k_begin; k0 < k_end; k0 += kStage) {
 #pragma unroll
     for (int u = 0; u < kStage / 32; ++u) {
       const int f = k0 + r + 32 * u;
-      // exact: |w| up is at most 2^30 and a power of two times w
-      tile[c][r + 32 * u] = (in && f < F) ? static_cast<int>(__builtin_rintf(w[static_cast<int64_t>(f) * N + n] * up)) : 0;
+      const float v = (in && f < F) ? w[static_cast<int64_t>(f) * N + n] : 0.0f;
+      // |w| up is at most 2^30 and a power of two times w: exact but for the
+      // integer rounding of magnitudes under 2^23
+      const float scaled = v * up, q_f = __builtin_rintf(scaled), mag = __builtin_fabsf(scaled);
+      tile[c][r + 32 * u] = static_cast<int>(q_f);
+      if (v != 0.0f && (scaled != q_f || q_f == 0.0f)) {
+        count += 1;
+        if (mag < 1048576.0f) count += uint64_t{1} << 21;
+        if (mag < 65536.0f) count += uint64_t{1} << 42;
+      }
     }
     __syncthreads();
     // thread -> plane, neuron, piece of 16 k
@@ -201,6 +225,17 @@ __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ 
                             (pl * 32 + nn) * kStage + 16 * c16) =
         u4{out[0], out[1], out[2], out[3]};
     __syncthreads();
+  }
+  small[r][c] = count;
+  __syncthreads();
+  if (r == 0 && in && up != 0.0f) {
+    uint64_t sum = 0;
+#pragma unroll 8
+    for (int i = 0; i < 32; ++i) sum += small[i][c];
+    const int weights = (k_end < F ? k_end : F) - k_begin, mask = (1 << 21) - 1;
+    const int rounded = static_cast<int>(sum) & mask, below10 = static_cast<int>(sum >> 21) & mask,
+              below14 = static_cast<int>(sum >> 42);
+    if (rounded > weights / 4 + kSlack || below10 > weights / 16 + kSlack || below14 > weights / 256 + kSlack) flags[1] = 1;
   }
 }
 

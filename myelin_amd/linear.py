@@ -177,11 +177,13 @@ class _Digits:
 
 
 class _Split:
-    """The fp32 synapse on the int8 or the bf16 MFMA, exactly.
+    """The fp32 synapse on the int8 or the bf16 MFMA.
 
     An input of zeros and ones (spikes) times W runs as four int8 products
     with the base-256 digits of W, summed without rounding and rounded once
-    (``myelin_gemm_spikes``).  An input whose every value is a bf16 value
+    (``myelin_gemm_spikes``), where the digits hold W as well as an fp32
+    product would (they are 31 bits of each column's largest weight; columns
+    of too wide a range are turned away).  An input whose every value is a bf16 value
     runs as three bf16 products, ``x @ W = x @ W_hi + x @ W_mid + x @ W_lo``
     with the three bf16 planes of W summing exactly to W, so every product
     is exact and only the fp32 summation rounds.  Per multiply-add the first

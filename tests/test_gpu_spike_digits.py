@@ -54,9 +54,10 @@ def test_digit_products_match_float64(M, N, F, with_bias):
     _print_case(test="digits", M=M, N=N, F=F, with_bias=with_bias)
     g = seeded(M + N + F)
     x = (torch.rand(M, F, generator=g) < (0.1 if with_bias else 0.9)).float()
-    # columns of very different size, small weights beside large ones
+    # columns of very different size, small weights beside large ones (a
+    # column of many more binades is turned away: test_gpu_digit_range)
     w = torch.randn(F, N, generator=g) * torch.exp2(torch.randint(-40, 40, (N,), generator=g).float())
-    w = w * torch.exp2(-torch.randint(0, 12, (F, N), generator=g).float())
+    w = w * torch.exp2(-torch.randint(0, 4, (F, N), generator=g).float())
     w[:, N // 2] = 0.0
     bias = torch.randn(N, generator=g) if with_bias else None
     xd, wd, bd = x.to(DEV), w.to(DEV), None if bias is None else bias.to(DEV)
