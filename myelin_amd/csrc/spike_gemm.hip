@@ -464,10 +464,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
       for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          // hi 2^16 + lo, both exact in 32 bits; hi is exact in fp32 while
+          // the sum is hi 2^16 + lo, both exact in 32 bits; with all but the
+          // low 16 bits of lo carried over lo is exact in fp32, and hi while
           // the sum is under 2^10 column maxima
-          const int lo = (acc[i][1][r] << 8) + acc[i][0][r];
-          const int hi = (acc[i][3][r] << 8) + acc[i][2][r];
+          int lo = (acc[i][1][r] << 8) + acc[i][0][r];
+          int hi = (acc[i][3][r] << 8) + acc[i][2][r];
+          const int carry = (lo + 0x8000) >> 16;
+          hi += carry;
+          lo -= carry << 16;
           float v = __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo)) * sc;
           if (g.bias != nullptr) v = v + bi;
           const float *base = g.C + (mw + 32 * i + acc_row(r, 0)) * g.ldc + n0;

@@ -107,3 +107,29 @@ def test_share_of_small_weights():
             n = 512 // share + 6 + extra
             w[:n, 19999] = value * 0.7  # 0.75 < 1 = 2^e; 0.7 has 24 bits: rounded
             assert _digits_flag(w) == flag, (share, extra)
+
+
+@pytest.mark.parametrize("K", [2003, 65024])
+def test_large_sums_that_cancel(K):
+    """Half of the inputs add 32767 units, which lies in the two low digits,
+    the others take 65536 units off in the two high ones: the low sum alone
+    passes 2^24, the whole stays below it and is returned exactly."""
+
+    _print_case(test="digit_cancel", K=K)
+    n = K // 3
+    w = torch.zeros(K, 32)
+    unit = 2.0**-30
+    w[:2 * n] = 32767 * unit
+    w[2 * n:3 * n] = -65536 * unit
+    w[K - 1] = 0.75  # the column's largest: sets the unit; silent
+    x = torch.ones(1, 4, K)
+    x[..., K - 1] = 0.0
+    x[0, 1, 0] = x[0, 2, 2 * n] = x[0, 3, 1] = x[0, 3, 2 * n + 1] = 0.0
+    xs, wt, _ = _operands(x, w)
+    assert isinstance(wt, L._Digits)
+    pre = torch.empty(1, 4, 32, device=DEV)
+    L._lif_fwd(xs, w.to(DEV), None, None, 0, 1, 0.0, float("inf"), 0.0, 1.0, _lib.RULE_THRESHOLD, _lib.PREC["fp32"],
+               _lib.stream(pre.device), pre=pre, wt=wt)
+    ref = (x.double().reshape(4, K) @ w.double()).reshape(1, 4, 32)
+    assert bool((ref.abs() < 2.0**24 * unit).all())
+    assert torch.equal(pre.cpu().double(), ref)
