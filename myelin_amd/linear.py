@@ -152,6 +152,13 @@ class _LazyBf16:
 
 # widest input of the int8 products: two digit sums joined stay in 32 bits
 _DIGITS_MAX_F = 508 * 128
+# narrowest where the fused kernel could run, which keeps the currents in LDS
+# where the split writes and reads them.  N=4096, T=100, B=256, us fused and
+# split: forward with dense spikes F=128 422 and 525, 192 551 and 562, 256 664
+# and 556, its training step 914 and 1005, 1252 and 1086, 1358 and 1096;
+# packed output F=96 332 and 333, 128 387 and 333, 192 500 and 361
+_DIGITS_MIN_F_FUSED = 192
+_DIGITS_MIN_F_PACKED = 128
 
 
 def _cast_spikes(x, flags, stream, bf16=True):
@@ -293,18 +300,22 @@ def _split_synapse(x, w, stream, lean=False, bf16=True, ints=True):
     return _Split(x, w, stream, lean, bf16, ints)
 
 
-def _split_eligible(prec: int, T: int, B: int, F: int, N: int, ints: bool = True) -> bool:
+def _split_eligible(prec: int, T: int, B: int, F: int, N: int, ints: bool = True, packed: bool = False) -> bool:
     """fp32 synapse wide enough for tiles (narrower outputs stream the input
-    once through the narrow kernels) with enough work to amortise the input
-    check -- and no graph being captured on the current stream: the split's
-    choice needs the input check's flags on the host (``_Split.operands``),
-    a wait that capture does not allow and whose answer a replay could not
-    revisit, so captured layers keep the fp32 engine."""
+    once through the narrow kernels), of widths whose rows the bf16 loaders
+    take (the weight gradient reads the bf16 copy on either route), with
+    enough work to amortise the input check -- and no graph being captured
+    on the current stream: the split's choice needs the input check's flags on
+    the host (``_Split.operands``), a wait that capture does not allow and
+    whose answer a replay could not revisit, so captured layers keep the fp32
+    engine, and may differ in a sum's last bits from the same layer run
+    eagerly.  ``ints``: the int8 products may be tried; ``packed``: the
+    output is packed words only."""
 
     if prec != _lib.PREC["fp32"] or N <= 32 or F % 8 != 0 or N % 8 != 0 or T * B * F * N < _SPLIT_MIN_MACS:
         return False
     # the bf16 products alone: the shapes the fused kernel does not take
-    if _fused(B, N) and not (ints and F <= _DIGITS_MAX_F):
+    if _fused(B, N) and not (ints and (_DIGITS_MIN_F_PACKED if packed else _DIGITS_MIN_F_FUSED) <= F <= _DIGITS_MAX_F):
         return False
     return not torch.cuda.is_current_stream_capturing()
 
@@ -913,7 +924,7 @@ def linear_packed_forward(x, w, b, params, checkpoint: int, precision: str):
     with torch.cuda.device(x.device):
         prec, stream = _lib.PREC[precision], _lib.stream(x.device)
         xs, wt = x, None
-        if _split_eligible(prec, T, B, F, N):
+        if _split_eligible(prec, T, B, F, N, packed=True):
             xs, wt, _ = _split_synapse(x, w, stream, bf16=False).operands()
         _lif_fwd(xs, w, b, None, 0, T, float(params.decay), float(params.threshold), float(params.reset), 10.0,
                  _lib.RULE_THRESHOLD, prec, stream, m_final=m_final, packed=words, ckpt_every=checkpoint, wt=wt)

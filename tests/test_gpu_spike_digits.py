@@ -118,6 +118,7 @@ def test_fused_shape_layer_takes_the_engine_its_input_allows(monkeypatch, value)
     p = myelin.LIFParams(tau_mem=9.0, threshold=0.7, reset=-0.2)
     res, names, real = [], [], _lib.call
     monkeypatch.setattr(_lib, "call", lambda name, *a: names.append(name) or real(name, *a))
+    monkeypatch.setattr(L, "_DIGITS_MIN_F_FUSED", 0)
     for macs in (0, 1 << 62):
         monkeypatch.setattr(L, "_SPLIT_MIN_MACS", macs)
         leaves = [t.to(DEV).requires_grad_() for t in (x, w, b)]
