@@ -434,12 +434,19 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
 /*
  * fp32 synapse currents of spikes (0/1 inputs) on the int8 MFMA.
  *
+ * Two device ints `flags` say whether an input and a weight qualify:
+ * flags[0] that some element of x is not bf16-exact (as
+ * myelin_cast_bf16_checked), flags[1] that some is neither 0 nor 1 or that
+ * the weight's digits would not do.
+ *
+ * myelin_probe_spikes: writes both flags from a sample of x's n elements.
+ *
  * myelin_cast_spikes: x [rows, F] fp32 -> words [Kw / 4][rows][4]: words 4 s
  * to 4 s + 3 of each row's Kw (bit i of word w the element 32 w + i, zeros
  * past F) for stage s (Kw a multiple of 4, at most 2032; 16-byte aligned),
- * and, unless xb is NULL, xb [rows, F] bf16.  Sets flags[0] if some element
- * is not bf16-exact (as myelin_cast_bf16_checked) and flags[1] if some
- * element is neither 0 nor 1; never clears them.
+ * and, unless xb is NULL, xb [rows, F] bf16.  Sets flags as every element
+ * says; never clears them.  Where flags[0] is set already, or flags[1] and
+ * xb is NULL, the outputs may be left unwritten.
  *
  * myelin_weight_digits: w [F, N] fp32 -> per column n a power of two
  * scale[n] and w = scale[n] * (d3 2^24 + d2 2^16 + d1 2^8 + d0), balanced
@@ -450,16 +457,21 @@ int myelin_split_bf16x3(const float *src, uint16_t *dst, int64_t rows,
  * column is not finite, its largest magnitude is below 2^-96, or more than a
  * few of its weights are so far below its largest that the digits hold them
  * less well than an fp32 product would (the shares: csrc/spike_gemm.hip).
+ * Where flags[1] is set already the outputs may be left unwritten.
  *
  * myelin_gemm_spikes: C [M, N] = bits w (+ bias) over M rows of words
  * [Kp / 128][x_rows][4] (from row r of a cast on: words + 4 r, x_rows the
  * cast's rows), every output the exact sum of the digit products rounded once to fp32
  * (twice past 2^10 column maxima), then scaled and biased: independent of
- * order, tiles and rows.  Meaningful only where the two calls above left
+ * order, tiles and rows.  Meaningful only where the calls above left
  * flags[1] clear.
+ * myelin_gemm_spikes_if: the same, and nothing where a flag is set when it
+ * runs, so that it may be launched before the host knows the flags.
  * Replaces: as myelin_gemm_f32 (the fp32 synapse GEMMs when the layer input
  *   is spikes).
  */
+int myelin_probe_spikes(const float *x, int64_t n, int *flags,
+                        myelin_stream_t stream);
 int myelin_cast_spikes(const float *x, int32_t *words, uint16_t *xb,
                        int64_t rows, int64_t F, int64_t Kw, int *flags,
                        myelin_stream_t stream);
@@ -470,6 +482,11 @@ int myelin_gemm_spikes(const int32_t *words, int64_t x_rows,
                        const int8_t *digits, const float *scale,
                        const float *bias, float *C, int64_t M, int64_t N,
                        int64_t Kp, int64_t ldc, myelin_stream_t stream);
+int myelin_gemm_spikes_if(const int *flags, const int32_t *words,
+                          int64_t x_rows, const int8_t *digits,
+                          const float *scale, const float *bias, float *C,
+                          int64_t M, int64_t N, int64_t Kp, int64_t ldc,
+                          myelin_stream_t stream);
 
 /*
  * Reverse recurrence over C steps of a saved pre-reset trace [C, BN]:

@@ -66,9 +66,11 @@ SIGNATURES: dict[str, list] = {
     "myelin_linear_lif_fwd_bf16": [_P] * 10 + [_I64] * 7 + [_F] * 4 + [_INT, _P],
     "myelin_cast_bf16": [_P, _P, _I64, _P],
     "myelin_cast_bf16_checked": [_P, _P, _I64, _P, _P],
+    "myelin_probe_spikes": [_P, _I64] + [_P] * 2,
     "myelin_cast_spikes": [_P] * 3 + [_I64] * 3 + [_P] * 2,
     "myelin_weight_digits": [_P] * 3 + [_I64] * 3 + [_P] * 2,
     "myelin_gemm_spikes": [_P, _I64] + [_P] * 4 + [_I64] * 4 + [_P],
+    "myelin_gemm_spikes_if": [_P, _P, _I64] + [_P] * 4 + [_I64] * 4 + [_P],
     "myelin_split_bf16x3": [_P, _P, _I64, _I64, _INT, _P],
     "myelin_gemm_parts": [_P, _P, _INT, _I64, _P, _P] + [_I64] * 6 + [_INT] * 3 + [_P, _I64, _P],
     "myelin_gemm_parts_col_sum": [_P, _P, _INT, _I64, _P, _P] + [_I64] * 6 + [_INT] * 3 + [_P, _I64, _P, _P, _I64,

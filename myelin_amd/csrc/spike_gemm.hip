@@ -37,6 +37,31 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 
+// flags[0], flags[1] (as cast_spikes sets them) from 64 runs of 64 elements
+// spread over x: real-valued inputs, nearly all of whose elements show it, are
+// known before any pass over them.  (4,096 elements each on a page of its own
+// took 7 to 12 us of address translation.)
+__global__ __launch_bounds__(1024) void probe_spikes(const float *x, int64_t n, int *flags) {
+  const int64_t step = n / 64 > 64 ? n / 64 : 64;
+  float v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = (static_cast<int64_t>(threadIdx.x >> 6) * 4 + u) * step + (threadIdx.x & 63);
+    v[u] = i < n ? x[i] : 0.0f;
+  }
+  bool inexact = false, other = false;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    inexact = inexact || !myelin::bf16_exact(v[u]);
+    other = other || !(v[u] == 0.0f || v[u] == 1.0f);
+  }
+  const int any0 = __syncthreads_or(inexact), any1 = __syncthreads_or(other);
+  if (threadIdx.x == 0) {
+    flags[0] = any0 != 0;
+    flags[1] = any1 != 0;
+  }
+}
+
 struct CastArgs {
   const float *x;
   uint32_t *words;
@@ -55,6 +80,7 @@ struct CastArgs {
 // eight lanes' four bits are joined to a word by lane exchanges.
 template <bool VEC>
 __global__ __launch_bounds__(256) void cast_spikes(CastArgs p) {
+  if (p.flags[0] != 0 || (p.flags[1] != 0 && p.xb == nullptr)) return;  // uniform: nothing here will be read
   constexpr int U = 4;  // groups per lane
   const uint32_t per = static_cast<uint32_t>(p.Kw) * 8;
   const int64_t total = p.rows * per;
@@ -131,7 +157,7 @@ __device__ __forceinline__ int piece_k(int c, int p) {
 // (zeros past F and N; the 128 k of a stage in the order of piece_k) and
 // scale [N].  flags[1] is set where a column holds a non-finite value, its
 // largest magnitude is outside [2^-96, 2^128), or its weights span too wide a
-// range for one scale (below).
+// range for one scale (below); nothing is done where it is set already.
 //
 // The range: a weight below 2^-7 of 2^e (the power of two above its column's
 // largest) is rounded, by at most 2^-31 of 2^e.  An fp32 product's own error
@@ -150,6 +176,10 @@ __device__ __forceinline__ int piece_k(int c, int p) {
 __global__ __launch_bounds__(1024) void weight_digits(const float *__restrict__ w, int8_t *__restrict__ q,
                                                       float *__restrict__ scale, int *__restrict__ flags, int F, int N,
                                                       int Kp, int chunk) {
+  __shared__ int skip;  // one answer for the workgroup: others may set the flag meanwhile
+  if (threadIdx.x == 0) skip = flags[1];
+  __syncthreads();
+  if (skip != 0) return;
   __shared__ uint32_t red[32][33];
   __shared__ uint64_t small[32][33];
   __shared__ int tile[32][kStage + 1];
@@ -280,6 +310,7 @@ struct SpikeArgs {
   const uint32_t *x;  // [Kp / 128][x_rows][4] words, M rows of each stage
   const int8_t *q;    // digits
   const float *scale, *bias;
+  const int *flags;  // or null: return at once where one of the two is set
   float *C;
   int64_t M, N, ldc, x_rows;
   int Kp;
@@ -310,6 +341,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
   constexpr int WA = BM / 64;                           // waves that load the bits, one piece a lane
   static_assert(WA <= NT / 64, "one piece of bits per lane at most");
   __shared__ __attribute__((aligned(1024))) char lds[NS * TILE];
+  if (g.flags != nullptr && (g.flags[0] | g.flags[1]) != 0) return;  // uniform: no launch beside this one writes them
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w / WGN, wn = w % WGN;
   const uint32_t tiles_m = static_cast<uint32_t>((g.M + BM - 1) / BM);
@@ -492,6 +524,13 @@ int launch_spike(const SpikeArgs &g, int per_cu, hipStream_t s) {
 
 }  // namespace
 
+extern "C" int myelin_probe_spikes(const float *x, int64_t n, int *flags, myelin_stream_t stream) {
+  if (n < 0) return myelin::invalid("probe_spikes: negative size");
+  if (flags == nullptr || (n > 0 && x == nullptr)) return myelin::invalid("probe_spikes: null pointer");
+  probe_spikes<<<dim3(1), dim3(1024), 0, myelin::as_hip(stream)>>>(x, n, flags);
+  return myelin::launched("probe_spikes");
+}
+
 extern "C" int myelin_cast_spikes(const float *x, int32_t *words, uint16_t *xb, int64_t rows, int64_t F, int64_t Kw,
                                   int *flags, myelin_stream_t stream) {
   if (rows < 0 || F < 1) return myelin::invalid("cast_spikes: rows must be >= 0 and F >= 1");
@@ -529,9 +568,10 @@ extern "C" int myelin_weight_digits(const float *w, int8_t *digits, float *scale
   return myelin::launched("weight_digits");
 }
 
-extern "C" int myelin_gemm_spikes(const int32_t *words, int64_t x_rows, const int8_t *digits, const float *scale,
-                                  const float *bias, float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc,
-                                  myelin_stream_t stream) {
+namespace {
+
+int gemm_spikes_impl(const int32_t *words, int64_t x_rows, const int8_t *digits, const float *scale, const float *bias,
+                     const int *flags, float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc, hipStream_t s) {
   if (M < 0 || N < 0) return myelin::invalid("gemm_spikes: negative size");
   if (x_rows < M) return myelin::invalid("gemm_spikes: x_rows < M");
   if (Kp < kStage || Kp % kStage != 0 || Kp > kMaxK) return myelin::invalid("gemm_spikes: bad row pitch");
@@ -543,11 +583,25 @@ extern "C" int myelin_gemm_spikes(const int32_t *words, int64_t x_rows, const in
     return myelin::invalid("gemm_spikes: operands must be 16-byte aligned");
   if (ldc >= (int64_t{1} << 27)) return myelin::invalid("gemm_spikes: rows too long");
   if (cdiv(M, 128) * cdiv(N, 32) > 0x7fffffff) return myelin::invalid("gemm_spikes: output too large");
-  const SpikeArgs g{reinterpret_cast<const uint32_t *>(words), digits, scale, bias, C, M, N, ldc, x_rows,
+  const SpikeArgs g{reinterpret_cast<const uint32_t *>(words), digits, scale, bias, flags, C, M, N, ldc, x_rows,
                     static_cast<int>(Kp)};
-  hipStream_t s = myelin::as_hip(stream);
   // 256 rows x 32 neurons, two workgroups per CU, where that fills the chip;
   // else 128 rows (3200 x 256 x 784, 200 of them: 8.8 us)
   if (cdiv(M, 256) * cdiv(N, 32) >= 512) return launch_spike<2, 4, 1, 3>(g, 2, s);
   return launch_spike<1, 4, 1, 4>(g, 2, s);
+}
+
+}  // namespace
+
+extern "C" int myelin_gemm_spikes(const int32_t *words, int64_t x_rows, const int8_t *digits, const float *scale,
+                                  const float *bias, float *C, int64_t M, int64_t N, int64_t Kp, int64_t ldc,
+                                  myelin_stream_t stream) {
+  return gemm_spikes_impl(words, x_rows, digits, scale, bias, nullptr, C, M, N, Kp, ldc, myelin::as_hip(stream));
+}
+
+extern "C" int myelin_gemm_spikes_if(const int *flags, const int32_t *words, int64_t x_rows, const int8_t *digits,
+                                     const float *scale, const float *bias, float *C, int64_t M, int64_t N, int64_t Kp,
+                                     int64_t ldc, myelin_stream_t stream) {
+  if (flags == nullptr) return myelin::invalid("gemm_spikes_if: null pointer");
+  return gemm_spikes_impl(words, x_rows, digits, scale, bias, flags, C, M, N, Kp, ldc, myelin::as_hip(stream));
 }

@@ -190,40 +190,44 @@ class _Split:
     with the base-256 digits of W, summed without rounding and rounded once
     (``myelin_gemm_spikes``), where the digits hold W as well as an fp32
     product would (they are 31 bits of each column's largest weight; columns
-    of too wide a range are turned away).  An input whose every value is a bf16 value
-    runs as three bf16 products, ``x @ W = x @ W_hi + x @ W_mid + x @ W_lo``
-    with the three bf16 planes of W summing exactly to W, so every product
-    is exact and only the fp32 summation rounds.  Per multiply-add the first
-    costs 2/3 of the second, and that a fifth of the fp32 engine.
+    of too wide a range are turned away).  An input whose every value is a
+    bf16 value runs as three bf16 products, ``x @ W = x @ W_hi + x @ W_mid +
+    x @ W_lo`` with the three bf16 planes of W summing exactly to W, so every
+    product is exact and only the fp32 summation rounds.  Per multiply-add the
+    first costs 2/3 of the second, and that a fifth of the fp32 engine.
 
     Construction launches the checked copies of x (``words``, its bits, and
-    ``xb`` bf16; without ``bf16`` only the words), both forms of W and an asynchronous
-    copy of the check's flags to pinned host memory; ``exact()`` and
-    ``operands()`` wait for those flags, the bf16 planes of W being formed
-    meanwhile.
+    ``xb`` bf16; without ``bf16`` only the words), the form of W they are
+    tried with, an asynchronous copy of the check's flags to pinned host
+    memory and, given ``first`` = (bias, steps, exact), the currents of the
+    first steps from them (``head``, see _lif_fwd), which the GPU computes
+    while the host waits; ``exact()`` and ``operands()`` wait for the flags.
+    A sample of x is checked first: on the int8 products' route the launches
+    behind it end at once where it shows real values.  What the check costs
+    those (the launches and the host's wait; us without a check and with):
+    784 -> 2048, T=50, B=256 forward 500 and 529, 1024 -> 2048, T=100, B=128
+    packed 520 and 557, 784 -> 2048, T=50, B=64 packed 146 and 170; what it
+    gives spikes: 501 -> 196, 518 -> 161, 146 -> 77.
 
     ``ints=False`` takes the bf16 products alone, and ``lean`` (the memory
     policy) implies it: no whole copy of x is kept then (``xb`` is a
     _LazyBf16), and a second copy and the digits of W beside the bf16 slices
-    that its weight gradient reads anyway would be its largest buffers."""
+    that its weight gradient reads anyway would be its largest buffers.
+    Otherwise a layer over spikes holds, until its backward, x's bf16 copy,
+    and while it runs the words, 4 (digits) or 6 (planes) bytes a weight and
+    one chunk of currents, also where the fused kernel would keep those in
+    LDS."""
 
-    def __init__(self, x, w, stream, lean=False, bf16=True, ints=True):
-        F, N = w.shape
+    def __init__(self, x, w, stream, lean=False, bf16=True, ints=True, first=None):
+        T, B, F = x.shape
+        N = w.shape[1]
         dev = x.device
-        flags = torch.zeros(2, dtype=torch.int32, device=dev)
-        self.x = x
-        self.words = self.xb = self.digits = None
-        if lean:
-            # no whole bf16 copy: check x slice by slice into one scratch
-            # buffer (the flag is only ever set), and cast per chunk later
-            self.xb = _LazyBf16(x)
-            step = max(1, (1 << 22) // max(1, x[0].numel()))
-            scratch = torch.empty((min(step, x.shape[0]), *x.shape[1:]), dtype=torch.bfloat16, device=dev)
-            for t0 in range(0, x.shape[0], step):
-                part = x[t0:t0 + step]
-                _lib.call("myelin_cast_bf16_checked", _lib.ptr(part), _lib.ptr(scratch), part.numel(), _lib.ptr(flags),
-                          stream)
-        elif ints and F <= _DIGITS_MAX_F:
+        self.x, self.w = x, w
+        self.words = self.xb = self.digits = self._w3 = self.head = None
+        digits = not lean and ints and F <= _DIGITS_MAX_F
+        if digits:
+            flags = torch.empty(2, dtype=torch.int32, device=dev)
+            _lib.call("myelin_probe_spikes", _lib.ptr(x), x.numel(), _lib.ptr(flags), stream)
             self.words, self.xb = _cast_spikes(x, flags, stream, bf16=bf16)
             # a weight the digits cannot hold raises the words' flag as well
             kp = 128 * self.words.shape[0]
@@ -232,15 +236,49 @@ class _Split:
             _lib.call("myelin_weight_digits", _lib.ptr(w), _lib.ptr(q), _lib.ptr(self.digits.scale), F, N, kp,
                       _lib.ptr(flags), stream)
         else:
-            self.xb = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
-            _lib.call("myelin_cast_bf16_checked", _lib.ptr(x), _lib.ptr(self.xb), x.numel(), _lib.ptr(flags), stream)
+            flags = torch.zeros(2, dtype=torch.int32, device=dev)
+            if lean:
+                # no whole bf16 copy: check x slice by slice into one scratch
+                # buffer (the flag is only ever set), and cast per chunk later
+                self.xb = _LazyBf16(x)
+                step = max(1, (1 << 22) // max(1, x[0].numel()))
+                scratch = torch.empty((min(step, T), B, F), dtype=torch.bfloat16, device=dev)
+                for t0 in range(0, T, step):
+                    part = x[t0:t0 + step]
+                    _lib.call("myelin_cast_bf16_checked", _lib.ptr(part), _lib.ptr(scratch), part.numel(),
+                              _lib.ptr(flags), stream)
+            else:
+                self.xb = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
+                _lib.call("myelin_cast_bf16_checked", _lib.ptr(x), _lib.ptr(self.xb), x.numel(), _lib.ptr(flags),
+                          stream)
         self._host = torch.empty(2, dtype=torch.int32, pin_memory=True)
         self._host.copy_(flags, non_blocking=True)
         self._ready = torch.cuda.Event()
         self._ready.record(torch.cuda.current_stream(dev))
-        self.w3 = torch.empty((3, N, F), dtype=torch.bfloat16, device=dev)
-        _lib.call("myelin_split_bf16x3", _lib.ptr(w), _lib.ptr(self.w3), F, N, 1, stream)
         self._flags = None
+        if first is not None:
+            b, steps, exact = first
+            head = torch.empty((steps, B, N), dtype=torch.float32, device=dev)
+            if digits:
+                _lib.call("myelin_gemm_spikes_if", _lib.ptr(flags), _lib.ptr(self.words), T * B, _lib.ptr(q),
+                          _lib.ptr(self.digits.scale), _lib.ptr(b), _lib.ptr(head), steps * B, N, kp, N, stream)
+            else:
+                _gemm_parts(self.xb[0:steps], self.w3, 3, N * F, head, steps * B, N, F, F, F, N, False, True, False,
+                            stream, bias=b, split=not exact)
+            self.head = head
+        elif not digits:
+            self.w3  # (formed while the host waits)
+
+    @property
+    def w3(self):
+        """The three bf16 planes of W^T ``[3, N, F]``, formed when first asked for."""
+
+        if self._w3 is None:
+            F, N = self.w.shape
+            self._w3 = torch.empty((3, N, F), dtype=torch.bfloat16, device=self.w.device)
+            _lib.call("myelin_split_bf16x3", _lib.ptr(self.w), _lib.ptr(self._w3), F, N, 1,
+                      _lib.stream(self.w.device))
+        return self._w3
 
     def _answer(self):
         if self._flags is None:
@@ -257,21 +295,25 @@ class _Split:
         """(xs, wt, xg): the currents' operands on the engine that takes this
         input -- words and digits, bf16 and planes, or the fp32 input and
         None -- and what the weight gradient's GEMM reads (the bf16 copy if the
-        input is exact in it, else x; None on digits without ``bf16``)."""
+        input is exact in it, else x; None on digits without ``bf16``).
+        ``head`` is dropped where it was computed on another engine."""
 
         inexact, other = self._answer()
         if inexact:
+            self.head = None
             return self.x, None, self.x
         if self.digits is not None and not other:
             return self.words, self.digits, self.xb
+        if self.digits is not None:
+            self.head = None
         if self.xb is None:
-            flags = torch.empty(2, dtype=torch.int32, device=self.x.device)  # known to hold: not read
+            flags = torch.zeros(2, dtype=torch.int32, device=self.x.device)  # known to hold: not read back
             self.xb = _cast_spikes(self.x, flags, _lib.stream(self.x.device))[1]
         return self.xb, self.w3, self.xb
 
 
 def _exact_split(wt) -> bool:
-    """``wt`` belongs to an exact split of the fp32 synapse (see _lif_fwd)."""
+    """``wt`` belongs to a split of the fp32 synapse (see _lif_fwd)."""
 
     return isinstance(wt, _Digits) or (wt is not None and wt.ndim == 3)
 
@@ -294,10 +336,10 @@ def _unpack_operands(how, tensors):
     return xs, _Digits(tensors[2], tensors[3]) if digits else tensors[2], xg
 
 
-def _split_synapse(x, w, stream, lean=False, bf16=True, ints=True):
-    """Start the exact split of ``x @ W`` (see _Split)."""
+def _split_synapse(*args, **kwargs):
+    """Start the split of ``x @ W`` (see _Split)."""
 
-    return _Split(x, w, stream, lean, bf16, ints)
+    return _Split(*args, **kwargs)
 
 
 def _split_eligible(prec: int, T: int, B: int, F: int, N: int, ints: bool = True, packed: bool = False) -> bool:
@@ -427,9 +469,15 @@ def _budgets(lean: bool, checkpoint, B: int, N: int) -> tuple[int, int]:
     return _CURRENT_CHUNK_ELEMS, _CURRENT_CHUNK_ELEMS
 
 
+def _chunk_steps(T: int, B: int, N: int, budget: int) -> int:
+    """Steps of a chunk of up to ``budget`` currents (see _lif_fwd)."""
+
+    return max(1, min(T, budget // (B * N)))
+
+
 def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, stream, *, m_final=None,
              spikes=None, pre=None, packed=None, rates=None, ckpt=None, ckpt_every=1, wt=None, exact=False,
-             pre_from=None, x_bits=None, budget=_CURRENT_CHUNK_ELEMS, cur=None):
+             pre_from=None, x_bits=None, budget=_CURRENT_CHUNK_ELEMS, cur=None, head=None):
     """Synaptic currents + LIF recurrence over steps [t0, t1).
 
     ``x`` is fp32 with ``w [F, N]`` fp32, or bf16 (bf16 synapse) with ``wt``,
@@ -455,6 +503,8 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     ``cur``: an fp32 buffer of at least one chunk's currents for the chunked
     route to use instead of allocating its own (when the GEMMs run in turn
     on the one stream).
+    ``head [steps, B, N]``: such a buffer that holds the currents of the
+    first ``steps`` steps already (a _Split's).
     """
 
     digits = wt if isinstance(wt, _Digits) else None
@@ -485,8 +535,13 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
                   _lib.ptr(m_final), _lib.ptr(spikes), _lib.ptr(pre), _lib.ptr(rates), T, B, F, N, t0, t1, decay,
                   threshold, reset, slope, rule, prec, stream)
         return
-    step = max(1, min(t1 - t0, budget // (B * N)))
-    bounds = sorted({*range(t0, t1, step), t1} | ({p0} if t0 < p0 < t1 else set()))
+    step = _chunk_steps(t1 - t0, B, N, budget)
+    cuts = {p0}
+    done_to = t0  # the currents of the steps before it are in head
+    if head is not None:
+        cur, done_to = head, t0 + head.shape[0]
+        cuts.add(done_to)
+    bounds = sorted({*range(t0, t1, step), t1} | {c for c in cuts if t0 < c < t1})
     n = len(bounds) - 1
     # several chunks on the fp32 engine: each chunk's GEMM runs on the side
     # stream one chunk ahead of the recurrence, into two alternating
@@ -537,11 +592,14 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
         c0, c1 = bounds[c], bounds[c + 1]
         i = c % len(curs)
         cur = curs[i]
+        if c1 <= done_to:
+            cur = head[c0 - t0:c1 - t0]
         s_ = side.cuda_stream if overlap else stream
         with torch.cuda.stream(side) if overlap else contextlib.nullcontext():
             if overlap and c >= 2:
                 side.wait_event(used[i])
-            gemm(c0, c1, cur, s_)
+            if c1 > done_to:
+                gemm(c0, c1, cur, s_)
             if overlap:
                 done[i].record(side)
         if overlap:
@@ -640,7 +698,8 @@ class HipLinearLIFFunction(torch.autograd.Function):
         xg = xs
         split = None
         if not half and bits is None and _split_eligible(prec, T, B, F, N, ints=not lean or checkpoint is None):
-            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None, bf16=need)
+            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None, bf16=need,
+                                   first=(b, _chunk_steps(T, B, N, fwd_budget), need and checkpoint is not None))
         m_final = torch.empty((B, N), dtype=x.dtype, device=dev)
         out = torch.empty((B, N) if rate else (T, B, N), dtype=x.dtype, device=dev)
         # spikes: their packed twin too (N / 8 bytes per row more), for a
@@ -648,27 +707,31 @@ class HipLinearLIFFunction(torch.autograd.Function):
         words = torch.empty((T, B, -(-N // 32)), dtype=torch.int32, device=dev) if not rate else None
         if checkpoint is not None and _keep_trace(F, N):
             checkpoint = None
-        if split is not None:
-            xs, wt, xg = split.operands()
-        chunked = not _fused(B, N) or _exact_split(wt)
         pre = ckpt = None
         tail = 0
+        fused = _fused(B, N)
         if need:
             if checkpoint is None:
                 pre = torch.empty((T, B, N), dtype=x.dtype, device=dev)
             else:
                 ckpt = torch.empty((math.ceil(T / checkpoint), B, N), dtype=x.dtype, device=dev)
-                if chunked:
+                if not fused or split is not None:
                     # the backward starts with the last span, whose trace
                     # this forward computes anyway: keep it (the buffer the
                     # backward would fill) instead of recomputing it there
                     span = _span(T, checkpoint, B * N, budget)
                     tail = (math.ceil(T / span) - 1) * span
                     pre = torch.empty((T - tail, B, N), dtype=x.dtype, device=dev)
+        if split is not None:
+            # (asked for after the allocations: the GPU runs the split's
+            # launches meanwhile)
+            xs, wt, xg = split.operands()
+            if fused and checkpoint is not None and not _exact_split(wt):
+                pre, tail = None, 0  # the fused kernel keeps no part of the trace
         _lif_fwd(xs, w, b, None, 0, T, decay, threshold, reset, slope, rule, prec, stream, m_final=m_final,
                  spikes=None if rate else out, pre=pre, packed=words, rates=out if rate else None, ckpt=ckpt,
                  ckpt_every=checkpoint or 1, wt=wt, exact=ckpt is not None, pre_from=tail, x_bits=bits,
-                 budget=fwd_budget)
+                 budget=fwd_budget, head=None if split is None else split.head)
         if words is not None:
             _attach_bits(out, words)
         if bits is not None:
@@ -923,9 +986,13 @@ def linear_packed_forward(x, w, b, params, checkpoint: int, precision: str):
     words = torch.empty((T, B, packed_last_dim_size(N)), dtype=torch.int32, device=x.device)
     with torch.cuda.device(x.device):
         prec, stream = _lib.PREC[precision], _lib.stream(x.device)
-        xs, wt = x, None
+        xs, wt, head = x, None, None
         if _split_eligible(prec, T, B, F, N, packed=True):
-            xs, wt, _ = _split_synapse(x, w, stream, bf16=False).operands()
+            split = _split_synapse(x, w, stream, bf16=False,
+                                   first=(b, _chunk_steps(T, B, N, _CURRENT_CHUNK_ELEMS), False))
+            xs, wt, _ = split.operands()
+            head = split.head
         _lif_fwd(xs, w, b, None, 0, T, float(params.decay), float(params.threshold), float(params.reset), 10.0,
-                 _lib.RULE_THRESHOLD, prec, stream, m_final=m_final, packed=words, ckpt_every=checkpoint, wt=wt)
+                 _lib.RULE_THRESHOLD, prec, stream, m_final=m_final, packed=words, ckpt_every=checkpoint, wt=wt,
+                 budget=_CURRENT_CHUNK_ELEMS, head=head)
     return m_final, PackedSpikes(data=words, original_shape=(T, B, N))

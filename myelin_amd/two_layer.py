@@ -122,18 +122,6 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         # bf16 synapse: the hidden GEMMs read bf16 copies of x and W_h^T
         half = _half(prec, F, H)
         xs, wt = _cast_transpose_bf16(x, wh, stream) if half else (x, None)
-        # spike inputs: the hidden synapse on the exact bf16 products, its
-        # operands asked for below, when the input check has had the time of
-        # the allocations.  (The int8 products take a step at T=2000, B=32,
-        # 1024 -> 4096 -> 20 from 6.20 to 5.93 ms.  Both are exact but for
-        # the last rounding; a superspike adjoint amplifies a last bit over
-        # thousands of steps, and where the hidden layer is nearly silent
-        # the two routes' gradients, each 1.5e-5 from the true one, lie
-        # 2.8e-5 apart: this network keeps the sums its results were
-        # established with.)
-        split = None
-        if not half and _split_eligible(prec, T, B, F, H, ints=False):
-            split = _split_synapse(x, wh, stream, lean=lean, ints=False)
         need = any(ctx.needs_input_grad[:5])
         K = math.ceil(T / C)
         L0 = min(C, T)
@@ -151,6 +139,18 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         # backward's)
         G = max(1, min(K, (_LEAN_FWD_ELEMS if lean else _CURRENT_CHUNK_ELEMS) // (L0 * B * H)))
         LG = min(G * C, T)
+        # spike inputs: the hidden synapse on the exact bf16 products, the
+        # first group's already running while the host learns whether the
+        # input qualifies.  (The int8 products take a step at T=2000, B=32,
+        # 1024 -> 4096 -> 20 from 6.20 to 5.93 ms.  Both are exact but for
+        # the last rounding; a superspike adjoint amplifies a last bit over
+        # thousands of steps, and where the hidden layer is nearly silent
+        # the two routes' gradients, each 1.5e-5 from the true one, lie
+        # 2.8e-5 apart: this network keeps the sums its results were
+        # established with.)
+        split = None
+        if not half and _split_eligible(prec, T, B, F, H, ints=False):
+            split = _split_synapse(x, wh, stream, lean=lean, ints=False, first=(bh, LG, need))
         # the packed variant never forms dense hidden spikes: its readout
         # GEMM reads the words, and as the words of all T are kept, the
         # readout runs once after the hidden layer (one currents GEMM and
@@ -162,8 +162,10 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
         pre_o = torch.empty((T, B, O), device=dev) if keep else None
         words = torch.empty((T, B, (H + 31) // 32), dtype=torch.int32, device=dev) if packed_hidden else None
         xg = xs
+        head = None
         if split is not None:
             xs, wt, xg = split.operands()
+            head, split.head = split.head, None
         for k in range(0, K, G):
             t0 = k * C
             t1 = min(t0 + G * C, T)
@@ -171,7 +173,9 @@ class HipTwoLayerRateFunction(torch.autograd.Function):
             _lif_fwd(xs[t0:t1], wh, bh, m_h, 0, L, decay, threshold, reset, slope, _lib.RULE_THRESHOLD, prec, stream,
                      m_final=m_h, spikes=None if hs is None else hs[:L],
                      packed=None if words is None else words[t0:t1], ckpt=None if ck_h is None else ck_h[k:],
-                     ckpt_every=C, wt=wt, exact=need, budget=LG * B * H)
+                     ckpt_every=C, wt=wt, exact=need, budget=LG * B * H,
+                     head=head)
+            head = None
             if hs is not None:
                 _readout_chunk(cur[:L], hs[:L], wo, bo, m_o, m_o, None if pre_o is None else pre_o[t0:t1], counts,
                                rates if t1 == T else None, ck_o, T, t0, t1, C, decay, threshold, reset, slope, prec,

@@ -116,8 +116,8 @@ def test_fused_shape_layer_takes_the_engine_its_input_allows(monkeypatch, value)
     b = torch.rand(N, generator=g) * 0.1
     gs = torch.randn(T, B, N, generator=g).to(DEV)
     p = myelin.LIFParams(tau_mem=9.0, threshold=0.7, reset=-0.2)
-    res, names, real = [], [], _lib.call
-    monkeypatch.setattr(_lib, "call", lambda name, *a: names.append(name) or real(name, *a))
+    res, routes, operands = [], [], L._Split.operands
+    monkeypatch.setattr(L._Split, "operands", lambda split: routes.append(operands(split)) or routes[-1])
     monkeypatch.setattr(L, "_DIGITS_MIN_F_FUSED", 0)
     for macs in (0, 1 << 62):
         monkeypatch.setattr(L, "_SPLIT_MIN_MACS", macs)
@@ -125,7 +125,8 @@ def test_fused_shape_layer_takes_the_engine_its_input_allows(monkeypatch, value)
         _, s = myelin.linear_surrogate_lif_forward(*leaves, p, surrogate="atan", surrogate_slope=4.0, checkpoint_size=4)
         res.append([s.detach(), *torch.autograd.grad(s, leaves, gs)])
         if macs == 0:
-            assert ("myelin_gemm_spikes" in names) == (value == "spikes")
+            (_, wt, _), = routes
+            assert isinstance(wt, L._Digits) == (value == "spikes") and (wt is None) == (value == "real")
     if value == "real":
         for a, c in zip(*res):
             assert torch.equal(a, c)
