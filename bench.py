@@ -56,6 +56,7 @@ T, B, N = 256, 128, 4096
 HBM_PEAK_GBPS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0
 FP32_PEAK_TFLOPS = 157.3
+INT8_PEAK_TOPS = 5000.0  # dense
 # algorithmic bytes per neuron-step: forward reads x and writes spikes;
 # backward re-reads x, reads dL/ds, writes dL/dx
 FWD_BYTES, BWD_BYTES = 8, 12
@@ -577,19 +578,43 @@ def _workload_long_rate(torch, myelin, args, threads, packed_hidden=False, check
             rates = readout(hidden(x))
         torch.nn.functional.cross_entropy(rates * Tl, labels).backward()
 
-    # the dominant kernel: one forward chunk of the split synapse, 256 steps
-    # x 32 rows = 8192 x 4096 currents over 3 x 1024 bf16 k (the forward's
-    # 2**25-current chunk; the backward's span recomputes run the same kernel)
+    # the engine the hidden currents run on, as the library chooses it: the
+    # modules take the int8 digits of a spike input except under the memory
+    # policy, the packed two-layer network the three bf16 planes
     stream = _lib.stream(dev)
+    lean = checkpoint_size == "memory"
+    ints = not (packed_hidden or lean)
+    engine = "fp32"
+    if lin._split_eligible(_lib.PREC["fp32"], Tl, Bl, F, H, ints=ints):
+        with torch.no_grad():
+            _, wt, _ = lin._split_synapse(x, wh.detach(), stream, lean=lean, ints=ints).operands()
+        engine = "int8" if isinstance(wt, lin._Digits) else "fp32" if wt is None else "bf16x3"
+        del wt
+    # the dominant kernel: one forward chunk of the split synapse, 256 steps
+    # x 32 rows = 8192 x 4096 currents over 4 int8 digit products or 3 x 1024
+    # bf16 k (the forward's 2**25-current chunk; the backward's span recomputes
+    # run the same kernel)
     rows = (lin._CURRENT_CHUNK_ELEMS // (Bl * H)) * Bl
-    xb = x.reshape(Tl * Bl, F)[:rows].to(torch.bfloat16)
-    w3 = torch.empty((3, H, F), dtype=torch.bfloat16, device=dev)
-    _lib.call("myelin_split_bf16x3", wh.data_ptr(), w3.data_ptr(), F, H, 1, stream)
     cur = torch.empty(rows, H, device=dev)
+    if engine == "int8":
+        with torch.no_grad():
+            words, digits, _ = lin._split_synapse(x, wh.detach(), stream, bf16=False).operands()
 
-    def launch():
-        _lib.call("myelin_gemm_parts", xb.data_ptr(), w3.data_ptr(), 3, H * F, bh.data_ptr(), cur.data_ptr(), rows,
-                  H, F, F, F, H, 0, 1, 0, None, 0, stream)
+        def launch():
+            _lib.call("myelin_gemm_spikes", words.data_ptr(), Tl * Bl, digits.q.data_ptr(), digits.scale.data_ptr(),
+                      bh.data_ptr(), cur.data_ptr(), rows, H, digits.q.shape[2], H, stream)
+
+        operands = (words, digits)
+    else:
+        xb = x.reshape(Tl * Bl, F)[:rows].to(torch.bfloat16)
+        w3 = torch.empty((3, H, F), dtype=torch.bfloat16, device=dev)
+        _lib.call("myelin_split_bf16x3", wh.data_ptr(), w3.data_ptr(), F, H, 1, stream)
+
+        def launch():
+            _lib.call("myelin_gemm_parts", xb.data_ptr(), w3.data_ptr(), 3, H * F, bh.data_ptr(), cur.data_ptr(), rows,
+                      H, F, F, F, H, 0, 1, 0, None, 0, stream)
+
+        operands = (xb, w3)
 
     # 41 back-to-back launches under one HIP event pair after 10 warmup
     # launches (the per-dispatch durations a kernel trace averages, without
@@ -601,7 +626,11 @@ def _workload_long_rate(torch, myelin, args, threads, packed_hidden=False, check
         launch()
     kern_ms = _launch_ms(torch, launch, 41)
     kern_pair = _launch_ms_median(torch, launch, 41, warmup=0)
-    del xb, w3, cur
+    del operands, cur, launch
+    if engine == "int8":
+        del words, digits
+    else:
+        del xb, w3
     step()
     torch.cuda.synchronize()
     torch.cuda.reset_peak_memory_stats(dev)
@@ -614,15 +643,16 @@ def _workload_long_rate(torch, myelin, args, threads, packed_hidden=False, check
     flops = 3 * 2 * Tl * Bl * F * H + 4 * 2 * Tl * Bl * H * O
     tflops = flops / (ms * 1e-3) / 1e12
     E = Tl * Bl * H
-    # the input is spikes, so the hidden synapse GEMMs (forward, recompute,
-    # dW) run as the exact three-part bf16 split: 3x their flops on the bf16
-    # MFMA; the readout GEMMs stay fp32
-    split = lin._split_eligible(_lib.PREC["fp32"], Tl, Bl, F, H) and bool(torch.equal(x, x.bfloat16().float()))
-    hidden_flops = 3 * 2 * Tl * Bl * F * H
-    executed = (3 * hidden_flops if split else hidden_flops) + (flops - hidden_flops)
+    # the input is spikes: the hidden synapse GEMMs (forward, recompute, dW)
+    # run as three bf16 products each, or the first two as four int8 products
+    # (whose peak is twice bf16's: counted as half the operations); the
+    # readout GEMMs as fp32 ones
+    gemm = 2 * Tl * Bl * F * H
+    executed = {"fp32": 3, "bf16x3": 9, "int8": 2 * 4 / 2 + 3}[engine] * gemm + (flops - 3 * gemm)
     mfma_tflops = executed / (ms * 1e-3) / 1e12
-    k_flops = 3 * 2 * rows * H * F
+    k_flops = (4 if engine == "int8" else 3) * 2 * rows * H * F
     k_tflops = k_flops / (kern_ms * 1e-3) / 1e12
+    k_peak = INT8_PEAK_TOPS if engine == "int8" else BF16_PEAK_TFLOPS
     ck = ("'memory'=45 (lean: chunk and span buffers of one checkpoint chunk)" if checkpoint_size == "memory"
           else f"{checkpoint_size} (buffers of 2**25 floats)")
     name = (f"two_layer_surrogate_lif_rate_packed_hidden_forward(1024->4096->20, checkpoint {ck}, "
@@ -634,16 +664,20 @@ def _workload_long_rate(torch, myelin, args, threads, packed_hidden=False, check
                  {"workload": name, "T": Tl, "B": Bl, "F": F, "N": H, "readout": O, "gflop_per_step": flops / 1e9},
                  steps=n_steps, warmup=n_warm + 1,
                  roofline={"bound": "mfma",
-                           "kernel": "gemm_dma<256 x 256 tiles, 3 bf16 parts> (one forward chunk of the exact "
-                                     "bf16 split of the fp32 synapse, 8192 x 4096 x 3*1024)",
-                           "achieved": k_tflops, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
-                           "frac": k_tflops / BF16_PEAK_TFLOPS,
-                           "traffic": _traffic("long_rate_T2000_B32_F1024_N4096", "gemm_dma_256x256"),
+                           "kernel": ("spike_gemm<256 x 32 tiles, 4 int8 digits> (one forward chunk of the fp32 "
+                                      "synapse over spikes, 8192 x 4096 x 1024)" if engine == "int8" else
+                                      "gemm_dma<256 x 256 tiles, 3 bf16 parts> (one forward chunk of the exact "
+                                      "bf16 split of the fp32 synapse, 8192 x 4096 x 3*1024)"),
+                           "achieved": k_tflops, "peak": k_peak, "unit": "Top/s" if engine == "int8" else "TFLOP/s",
+                           "frac": k_tflops / k_peak,
+                           "traffic": None if engine == "int8" else
+                           _traffic("long_rate_T2000_B32_F1024_N4096", "gemm_dma_256x256"),
                            "flops_per_launch": k_flops, "kernel_ms": kern_ms,
                            "kernel_ms_event_pair_median": kern_pair},
                  step_mfma_tflops_executed=mfma_tflops, step_mfma_frac_executed=mfma_tflops / BF16_PEAK_TFLOPS,
                  fp32_equivalent_tflops=tflops, fp32_equivalent_frac_of_fp32_peak=tflops / FP32_PEAK_TFLOPS,
-                 hidden_synapse="exact bf16 split (3 parts)" if split else "fp32",
+                 hidden_synapse={"fp32": "fp32", "bf16x3": "exact bf16 split (3 parts)",
+                                 "int8": "int8 digits (4 products; dW the bf16 split)"}[engine],
                  peak_step_bytes=peak_bytes, dense_hidden_spike_bytes=Tl * Bl * H * 4)
     if not args.no_cpu_baseline and not packed_hidden and checkpoint_size == "memory":
         R = _oracle()

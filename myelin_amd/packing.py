@@ -4,8 +4,9 @@ packing.py:1-273).
 ``PackedSpikes.data`` holds signed int32 words along the last dimension:
 bit ``i`` of word ``w`` is element ``32*w + i`` (LSB first); padding bits
 are zero after packing and ignored by every count.  All compute runs in the
-HIP kernels of ``csrc/packing.hip``: a wave ballot packs 64 elements into two
-words, unpack writes 4 elements per lane, counts use popcount.
+HIP kernels of ``csrc/packing.hip``: a wave ballot packs 64 elements of 4 or
+8 bytes into two words, a lane packs 32 narrower ones, unpack writes 16 bytes
+per lane, counts use popcount.
 """
 
 from __future__ import annotations
