@@ -159,6 +159,14 @@ _DIGITS_MAX_F = 508 * 128
 # packed output F=96 332 and 333, 128 387 and 333, 192 500 and 361
 _DIGITS_MIN_F_FUSED = 192
 _DIGITS_MIN_F_PACKED = 128
+# least multiply-adds of a layer whose input wants its gradient, where the
+# planes are the other choice: the host's way from the flags to the backward's
+# launches, 75 to 110 us, then runs beside the currents' products, and the
+# planes' cover more of it.  Training step, digits and planes, us: 6400 x 1000 x
+# 704 345 and 295-330, 8192 x 1024 x 1024 400 and 361-384, 16384 x 1024 x 1024
+# 655 and 666, 25600 x 1024 x 1024 1012 and 1075; without the input's gradient
+# 8192 x 1024 x 1024 196-247 and 245, 12800 x 1024 x 512 215-243 and 252
+_DIGITS_MIN_MACS_DX = 3 << 32
 
 
 def _cast_spikes(x, flags, stream, bf16=True):
@@ -205,9 +213,9 @@ class _Split:
     A sample of x is checked first: on the int8 products' route the launches
     behind it end at once where it shows real values.  What the check costs
     those (the launches and the host's wait; us without a check and with):
-    784 -> 2048, T=50, B=256 forward 500 and 529, 1024 -> 2048, T=100, B=128
-    packed 520 and 557, 784 -> 2048, T=50, B=64 packed 146 and 170; what it
-    gives spikes: 501 -> 196, 518 -> 161, 146 -> 77.
+    784 -> 2048, T=50, B=256 forward 500 and 523, 1024 -> 2048, T=100, B=128
+    packed 521 and 557, 784 -> 2048, T=50, B=64 packed 146 and 167; what it
+    gives spikes: 501 -> 192, 518 -> 157, 146 -> 77.
 
     ``ints=False`` takes the bf16 products alone, and ``lean`` (the memory
     policy) implies it: no whole copy of x is kept then (``xb`` is a
@@ -697,8 +705,11 @@ class HipLinearLIFFunction(torch.autograd.Function):
         fwd_budget, budget = _budgets(lean, checkpoint, B, N)
         xg = xs
         split = None
-        if not half and bits is None and _split_eligible(prec, T, B, F, N, ints=not lean or checkpoint is None):
-            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None, bf16=need,
+        ints = not lean or checkpoint is None
+        if not _fused(B, N) and ctx.needs_input_grad[0] and T * B * F * N < _DIGITS_MIN_MACS_DX:
+            ints = False
+        if not half and bits is None and _split_eligible(prec, T, B, F, N, ints=ints):
+            split = _split_synapse(x, w, stream, lean=lean and checkpoint is not None, bf16=need, ints=ints,
                                    first=(b, _chunk_steps(T, B, N, fwd_budget), need and checkpoint is not None))
         m_final = torch.empty((B, N), dtype=x.dtype, device=dev)
         out = torch.empty((B, N) if rate else (T, B, N), dtype=x.dtype, device=dev)

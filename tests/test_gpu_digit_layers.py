@@ -28,6 +28,7 @@ def calls(monkeypatch):
     monkeypatch.setattr(_lib, "call", lambda name, *a: names.append(name) or real(name, *a))
     monkeypatch.setattr(L, "_SPLIT_MIN_MACS", 0)
     monkeypatch.setattr(L, "_DIGITS_MIN_F_FUSED", 0)
+    monkeypatch.setattr(L, "_DIGITS_MIN_MACS_DX", 0)
     return names
 
 
@@ -132,6 +133,18 @@ def test_one_value_that_is_no_spike(monkeypatch, calls, value, shape, ck):
             assert float((a - c).abs().max()) <= 1e-5 * float(c.abs().max()), what
         else:
             assert torch.equal(torch.nan_to_num(a, 7.0), torch.nan_to_num(c, 7.0)), what
+
+
+@pytest.mark.parametrize("wants_dx,macs,digits", [(True, 1, True), (True, 1 << 62, False), (False, 1 << 62, True)])
+def test_the_engine_of_a_layer_whose_input_wants_its_gradient(monkeypatch, calls, wants_dx, macs, digits):
+    _print_case(test="digit_dx", wants_dx=wants_dx, macs=macs)
+    monkeypatch.setattr(L, "_DIGITS_MIN_MACS_DX", macs)
+    x, w, b, gs = _case(23, 5, 136, 72, 12)
+    leaves = [x.to(DEV).requires_grad_(wants_dx), *(t.to(DEV).requires_grad_() for t in (w, b))]
+    _, s = myelin.linear_surrogate_lif_forward(*leaves, P, surrogate="atan", checkpoint_size=4)
+    assert (_gemms(calls) > 0) == digits and ("myelin_gemm_parts" in calls) == (not digits)
+    s.backward(gs.to(DEV))
+    assert all((t.grad is not None) == t.requires_grad for t in leaves)
 
 
 @pytest.mark.parametrize("kind", ["spikes", "real", "late", "empty"])
