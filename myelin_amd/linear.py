@@ -120,7 +120,7 @@ def _gemm_parts(A, B, parts, b_part, C, M, N, K, lda, ldb, ldc, trans_a, trans_b
                   dst.numel(), stream)
 
 
-# exact split of an fp32 synapse: tried for products of at least this many
+# split of an fp32 synapse: tried for products of at least this many
 # multiply-adds (the input check costs one host synchronisation)
 _SPLIT_MIN_MACS = 1 << 32
 
@@ -489,11 +489,11 @@ def _lif_fwd(x, w, b, m0, t0, t1, decay, threshold, reset, slope, rule, prec, st
     """Synaptic currents + LIF recurrence over steps [t0, t1).
 
     ``x`` is fp32 with ``w [F, N]`` fp32, or bf16 (bf16 synapse) with ``wt``,
-    the bf16 transposed weight ``[N, F]``; or an exact split's operands: bf16
+    the bf16 transposed weight ``[N, F]``; or a split's operands: bf16
     with ``wt`` its planes ``[3, N, F]``, or words (see _cast_spikes) with
     ``wt`` a _Digits.
     Fused (one launch, currents stay in LDS) when N >= 64 and the fused grid
-    has >= 1024 workgroups, except on the exact split.
+    has >= 1024 workgroups, except on the split.
     Otherwise each workgroup would walk many chunks serially, so the steps
     are processed in chunks of up to ``budget`` currents: an MFMA GEMM (split-K
     when narrow) writes ``x_t @ W + b`` for the chunk, then the recurrence
@@ -749,7 +749,7 @@ class HipLinearLIFFunction(torch.autograd.Function):
             xs = xg = bits  # what the backward's weight GEMM reads
         ctx.set_materialize_grads(False)
         # the bf16 synapse keeps the bf16 copies of x and W^T (what its
-        # GEMMs read), the exact split its copies of x and form of W
+        # GEMMs read), the split its copies of x and form of W
         if checkpoint is None:
             xs, wt = (xg, wt) if not isinstance(wt, _Digits) else (xg, None)  # nothing to recompute
         saved, how = _pack_operands(x, xs, wt, xg) if need else ((), None)
